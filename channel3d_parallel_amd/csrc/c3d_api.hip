@@ -353,6 +353,17 @@ bool build_grid(c3d_ctx* c) {
   return true;
 }
 
+// -(Dyy(j,j) + Dyy(j,j-1) + Dyy(j,j+1)) of the rounded entries: zero but for
+// their rounding, summed in extended precision.
+std::vector<double> dyy_excess(const c3d_ctx* c) {
+  const int n = c->nym;
+  std::vector<double> e(n);
+  for (int j = 0; j < n; j++)
+    e[j] = (double)-((long double)c->dyy_d[j] + (j > 0 ? c->dyy_l[j - 1] : 0.0L) +
+                     (j < n - 1 ? c->dyy_u[j] : 0.0L));
+  return e;
+}
+
 // Fortran-indexed spacing table: t[i] = a(i) - a(i-1) for i = 2..n (t[0], t[1] = 0).
 std::vector<double> face_spacing(const std::vector<double>& a) {
   std::vector<double> t(a.size() + 2, 0.0);
@@ -513,6 +524,7 @@ int c3d_create(const c3d_desc* desc, c3d_ctx** out) {
       (rc = upload(c, &g.dzg, centre_spacing(c->zg))) || (rc = upload(c, &g.kxx, c->kxx)) ||
       (rc = upload(c, &g.kzz, c->kzz)) || (rc = upload(c, &g.dyy_d, c->dyy_d)) ||
       (rc = upload(c, &g.dyy_l, c->dyy_l)) || (rc = upload(c, &g.dyy_u, c->dyy_u)) ||
+      (rc = upload(c, &g.dyy_e, dyy_excess(c))) ||
       (rc = upload(c, &g.twx64, twiddles<double>(c->nxp))) ||
       (rc = upload(c, &g.twz64, twiddles<double>(c->nzp))) ||
       (rc = upload(c, &g.twx32, twiddles<float>(c->nxp))) ||
@@ -533,7 +545,7 @@ int c3d_create(const c3d_desc* desc, c3d_ctx** out) {
       (rc = dalloc(c, &c->part, 2 * (size_t)c3d::massflow_rows(c->g) + 2)) ||
       (rc = dalloc(c, &c->nanflag, 1)) ||
       (rc = dalloc(c, &c->S, c->nspec)) ||
-      (!c3d::tri_part_supported(c->g) && (rc = dalloc(c, &c->CP, c->nspec))) ||
+      (c3d::tri_needs_scratch(c->g) && (rc = dalloc(c, &c->CP, c->nspec))) ||
       (rc = dalloc(c, &c->red, kRedRefine + (size_t)kMaxRef * kResSlots)))
     return cleanup(rc);
   if (d.precision == C3D_PREC_MIXED && (rc = dalloc(c, &c->S32, c->nspec))) return cleanup(rc);

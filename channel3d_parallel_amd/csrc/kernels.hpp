@@ -35,6 +35,7 @@ struct DevGrid {
   const double* dyy_d;  // [nym]   Dyy(j,j)
   const double* dyy_l;  // [nym-1] Dyy(j+1,j)
   const double* dyy_u;  // [nym-1] Dyy(j,j+1)
+  const double* dyy_e;  // [nym]   -(Dyy(j,j) + Dyy(j,j-1) + Dyy(j,j+1)): round-off of the tables
   const cpx<double>* twx64;
   const cpx<double>* twz64;
   const cpx<float>* twx32;
@@ -54,9 +55,11 @@ __host__ __device__ __forceinline__ size_t ridx(int i, int j, int k, int nxg, in
 hipError_t launch_fwd_x(const DevGrid& g, bool from_uvw, const double* U, const double* V,
                         const double* W, const double* rhs, cpx<double>* S, hipStream_t s);
 hipError_t launch_fft_z(const DevGrid& g, int sign, cpx<double>* S, hipStream_t s);
-// Tridiagonal solve along y for every (kx,kz).  nym = 64, 128, 192 use the
-// partitioned register solver; other sizes the plain Thomas sweep with CP,
-// nym*nxh*nzp doubles of scratch (may be null when tri_part_supported).
+// Tridiagonal solve along y for every (kx,kz): the partitioned register
+// solver from 33 to 768 rows, else the plain Thomas sweep with CP, nym*nxh*nzp
+// doubles of scratch (may be null unless tri_needs_scratch).
+bool tri_needs_scratch(const DevGrid& g);
+// The row counts of the FP32 solves (launch_tri32, launch_tri32to64).
 bool tri_part_supported(const DevGrid& g);
 hipError_t launch_tri(const DevGrid& g, cpx<double>* S, double* CP, hipStream_t s);
 // Inverse x transform.  mode 0: out = solution rhs_p (Poisson drop-in).
