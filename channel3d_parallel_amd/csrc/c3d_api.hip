@@ -699,11 +699,11 @@ int c3d_solve_poisson_equation(c3d_ctx* c, double* rhs, int rk_step, double dt) 
   if (!c || !rhs) return C3D_EINVAL;
   if (rk_step == 1 && !(dt != 0.0)) return fail(c, C3D_EINVAL, "dt must be nonzero at rk_step 1");
   HIPCHK(c, hipMemcpyAsync(c->rhs, rhs, c->nr * 8, hipMemcpyHostToDevice, c->stream));
-  HIPCHK(c, c3d::launch_fwd_x(c->g, false, nullptr, nullptr, nullptr, c->rhs, c->S, c->stream));
+  HIPCHK(c, c3d::launch_fwd_x(c->g, false, nullptr, nullptr, nullptr, c->rhs, c->S, false,
+                              c->stream));
   int rc = spectral_core(c);
   if (rc) return rc;
   HIPCHK(c, c3d::launch_inv_x(c->g, 0, c->S, c->rhs, c->P, dt, rk_step == 1, c->stream));
-  if (rk_step == 1) HIPCHK(c, c3d::launch_p_ghosts(c->g, c->P, c->stream));
   HIPCHK(c, hipMemcpyAsync(rhs, c->rhs, c->nr * 8, hipMemcpyDeviceToHost, c->stream));
   return sync(c);
 }
@@ -716,8 +716,11 @@ int c3d_solve_poisson_equation(c3d_ctx* c, double* rhs, int rk_step, double dt) 
 // add the solution to phic; the velocity is corrected by G(phi1) + G(phic).
 // Mixed: the forward half of every pass (x and z transforms) on FP32
 // spectra, the inverse half (tridiagonal solution, inverse z and x
-// transforms) in FP64 (or FP32 with C3D_MIXED_INV64=0).
-static int projection_launch(c3d_ctx* c, double dt, int rk_step, hipEvent_t* ev) {
+// transforms) in FP64 (or FP32 with C3D_MIXED_INV64=0).  bc: the velocity's
+// boundary conditions before and after, without passes of their own: the
+// divergence reads the periodic images in the interior, and the correction
+// stores every value with its boundary images.
+static int projection_launch(c3d_ctx* c, double dt, int rk_step, hipEvent_t* ev, bool bc = false) {
   const bool rk1 = rk_step == 1;
   const bool mixed = c->desc.precision == C3D_PREC_MIXED;
   const int nref = c->nref;
@@ -725,7 +728,7 @@ static int projection_launch(c3d_ctx* c, double dt, int rk_step, hipEvent_t* ev)
   hipStream_t st = c->stream;
   if (ev) HIPCHK(c, hipEventRecord(ev[0], st));
   if (!mixed && nref == 0) {
-    HIPCHK(c, c3d::launch_fwd_x(g, true, c->U, c->V, c->W, nullptr, c->S, st));
+    HIPCHK(c, c3d::launch_fwd_x(g, true, c->U, c->V, c->W, nullptr, c->S, bc, st));
     if (ev) HIPCHK(c, hipEventRecord(ev[1], st));
     HIPCHK(c, c3d::launch_fft_z(g, -1, c->S, st));
     if (ev) HIPCHK(c, hipEventRecord(ev[2], st));
@@ -735,9 +738,8 @@ static int projection_launch(c3d_ctx* c, double dt, int rk_step, hipEvent_t* ev)
     if (ev) HIPCHK(c, hipEventRecord(ev[4], st));
     HIPCHK(c, c3d::launch_inv_x(g, 1, c->S, c->Pint, c->P, dt, rk1, st));
     if (ev) HIPCHK(c, hipEventRecord(ev[5], st));
-    if (rk1) HIPCHK(c, c3d::launch_p_ghosts(g, c->P, st));
     if (ev) HIPCHK(c, hipEventRecord(ev[6], st));
-    HIPCHK(c, c3d::launch_grad_correct(g, c->U, c->V, c->W, c->Pint, dt, st));
+    HIPCHK(c, c3d::launch_grad_correct(g, c->U, c->V, c->W, c->Pint, dt, bc, st));
     if (ev) HIPCHK(c, hipEventRecord(ev[7], st));
     return 0;
   }
@@ -768,9 +770,10 @@ static int projection_launch(c3d_ctx* c, double dt, int rk_step, hipEvent_t* ev)
                              (size_t)kMaxRef * kResSlots * sizeof(unsigned long long), st));
   // first solve; the FP64 divergence b is kept only for the refinement
   if (mixed)
-    HIPCHK(c, c3d::launch_fwd_x32(g, c->U, c->V, c->W, nref > 0 ? c->b64 : nullptr, c->S32, st));
+    HIPCHK(c, c3d::launch_fwd_x32(g, c->U, c->V, c->W, nref > 0 ? c->b64 : nullptr, c->S32, bc,
+                                     st));
   else
-    HIPCHK(c, c3d::launch_fwd_x_b64(g, c->U, c->V, c->W, c->b64, c->S, st));
+    HIPCHK(c, c3d::launch_fwd_x_b64(g, c->U, c->V, c->W, c->b64, c->S, bc, st));
   if (ev) HIPCHK(c, hipEventRecord(ev[1], st));
   HIPCHK(c, fwd_z());
   if (ev) HIPCHK(c, hipEventRecord(ev[2], st));
@@ -796,13 +799,12 @@ static int projection_launch(c3d_ctx* c, double dt, int rk_step, hipEvent_t* ev)
       rc = back(5, c->phi64, s == 1 ? nullptr : c->phic, nullptr, c->phic, rk1, false);
     if (rc) return rc;
   }
-  if (rk1) HIPCHK(c, c3d::launch_p_ghosts(g, c->P, st));
   if (ev) HIPCHK(c, hipEventRecord(ev[6], st));
   if (nref == 0)
-    HIPCHK(c, c3d::launch_grad_correct(g, c->U, c->V, c->W, c->Pint, dt, st));
+    HIPCHK(c, c3d::launch_grad_correct(g, c->U, c->V, c->W, c->Pint, dt, bc, st));
   else
     HIPCHK(c, c3d::launch_grad_correct_split(g, c->U, c->V, c->W, c->phi64, c->phic, c->Pint, dt,
-                                             st));
+                                             bc, st));
   if (ev) HIPCHK(c, hipEventRecord(ev[7], st));
   return 0;
 }
@@ -1215,7 +1217,7 @@ int c3d_wall_shear(c3d_ctx* c, double* utau, double* wtau, double* Umean, double
 
 int c3d_add_to_u(c3d_ctx* c, double d) {
   if (!c) return C3D_EINVAL;
-  HIPCHK(c, c3d::launch_add_u(c->g, c->U, d, c->stream));
+  HIPCHK(c, c3d::launch_add_u(c->g, c->U, d, false, c->stream));
   return sync(c);
 }
 
@@ -1237,18 +1239,13 @@ int c3d_time_step_rk3(c3d_ctx* c, double dt, int x_mass_cte, double q0) {
     }
     c->t = t0 + rk_t[st - 1] * dt;                              // :108
     if (!rc && c->ib && c->ib->moving) rc = ib_move_to(c, c->t);  // :110-115
-    if (!rc && c3d::launch_apply_bc(c->g, c->U, c->V, c->W, c->stream) != hipSuccess)
-      rc = fail(c, C3D_EHIP, "boundary conditions");            // :117
+    // boundary conditions (:117, :123) with the projections' own kernels
     if (!rc) rc = save_interim(c);
-    if (!rc) rc = projection_launch(c, dt, st, nullptr);        // :118
+    if (!rc) rc = projection_launch(c, dt, st, nullptr, true);  // :118
     if (!rc && c->ib) {                                         // :119-122
-      if (c3d::launch_apply_bc(c->g, c->U, c->V, c->W, c->stream) != hipSuccess)
-        rc = fail(c, C3D_EHIP, "boundary conditions");
-      if (!rc) rc = ib_projection_launch(c, dt, st);
+      rc = ib_projection_launch(c, dt, st);
       if (rc == C3D_ENOCONV) rc = 0;  // the reference warns and continues
     }
-    if (!rc && c3d::launch_apply_bc(c->g, c->U, c->V, c->W, c->stream) != hipSuccess)
-      rc = fail(c, C3D_EHIP, "boundary conditions");            // :123
   }
   if (!rc && x_mass_cte == 1) {  // :187-193
     const double prev = c->dPdx;
@@ -1256,8 +1253,7 @@ int c3d_time_step_rk3(c3d_ctx* c, double dt, int x_mass_cte, double q0) {
     rc = mass_flow(c, c->U, &ub);
     if (!rc) {
       const double d = q0 - ub;
-      if (c3d::launch_add_u(c->g, c->U, d, c->stream) != hipSuccess ||
-          c3d::launch_apply_bc(c->g, c->U, c->V, c->W, c->stream) != hipSuccess)
+      if (c3d::launch_add_u(c->g, c->U, d, true, c->stream) != hipSuccess)
         rc = fail(c, C3D_EHIP, "mass-flow correction");
       c->dPdx = 0.5 * (prev + d / dt);
     }
@@ -1363,21 +1359,23 @@ int c3d_time_projection(c3d_ctx* c, int iters, double dt, double* total_ms, doub
 static int ib_poisson_reg(c3d_ctx* c, double dt, int rk_step) {
   IBState* ib = c->ib;
   const bool rk1 = rk_step == 1;
-  HIPCHK(c, c3d::launch_fwd_x(c->g, true, ib->Ureg, ib->Vreg, ib->Wreg, nullptr, c->S, c->stream));
+  HIPCHK(c, c3d::launch_fwd_x(c->g, true, ib->Ureg, ib->Vreg, ib->Wreg, nullptr, c->S, true,
+                              c->stream));
   int rc = spectral_core(c);
   if (rc) return rc;
   HIPCHK(c, c3d::launch_inv_x(c->g, 1, c->S, ib->phi, c->P, dt, rk1, c->stream));
-  if (rk1) HIPCHK(c, c3d::launch_p_ghosts(c->g, c->P, c->stream));
   return 0;
 }
 
-// U_reg = R f (src/projection.f90:66-73): aux, three spreads, boundary conditions.
+// U_reg = R f (src/projection.f90:66-73): aux, three spreads.  The boundary
+// conditions that follow there are not applied: the support lies in the
+// interior, and the users of U_reg (the divergence with its periodic images,
+// the Schur rows and the correction at interior cells) read no boundary cell.
 static int ib_spread_force(c3d_ctx* c, const double* f, double dt) {
   IBState* ib = c->ib;
   const int nb = ib->m.nb;
   HIPCHK(c, c3d::ib::launch_aux(ib->m, f, dt, c->desc.nu, ib->aux, c->stream));
   HIPCHK(c, c3d::ib::launch_spread3(ib->m, ib->sp, ib->aux, ib->Ureg, ib->Vreg, ib->Wreg, c->stream));
-  HIPCHK(c, c3d::launch_apply_bc(c->g, ib->Ureg, ib->Vreg, ib->Wreg, c->stream));
   return 0;
 }
 
@@ -1626,7 +1624,7 @@ static int ib_projection_launch(c3d_ctx* c, double dt, int rk_step) {
   ib->last_dt = dt;
   bool r_ready = false;
   if (ib->guess == 3) {  // learned start: fb = fprev + a d, d from the network
-    int rc0 = mlp_guess(c, dt, rk_step);
+    int rc0 = mlp_guess(c, dt, 0);
     if (rc0) return rc0;
     r_ready = true;
   }
@@ -1635,8 +1633,10 @@ static int ib_projection_launch(c3d_ctx* c, double dt, int rk_step) {
     if (!rc0) rc0 = ib_hist_start(c, dt);
     if (rc0) return rc0;
   }
-  int rc = ib_bicgstab_launch(c, ib->fb, ib->rhs_ib, ib->tol, ib->maxit, dt, rk_step, nullptr,
-                              nullptr, r_ready);                                         // :60
+  // rk_step 1: each Schur product's P (src/poisson.f90:91-99) would be
+  // replaced by that of the solve below, so only that one writes it
+  int rc = ib_bicgstab_launch(c, ib->fb, ib->rhs_ib, ib->tol, ib->maxit, dt, 0, nullptr, nullptr,
+                              r_ready);                                                  // :60
   if (rc && rc != C3D_ENOCONV) return rc;
   const int conv = rc;
   if (!conv && ib->guess == 4 && (rc = ib_hist_push(c, dt))) return rc;
@@ -1649,8 +1649,7 @@ static int ib_projection_launch(c3d_ctx* c, double dt, int rk_step) {
   if ((rc = ib_poisson_reg(c, dt, rk_step))) return rc;                                  // :76-80
   HIPCHK(c, c3d::ib::launch_ib_correct(c->g, ib->Uint, ib->Vint, ib->Wint, ib->Ureg, ib->Vreg,
                                        ib->Wreg, c->Pint, ib->phi, dt, c->U, c->V, c->W,
-                                       c->stream));                                      // :83-92
-  HIPCHK(c, c3d::launch_apply_bc(c->g, c->U, c->V, c->W, c->stream));                  // :94
+                                       c->stream));                                      // :83-94
   return conv;  // C3D_ENOCONV keeps the message set by the solve
 }
 
@@ -1867,7 +1866,7 @@ int ib_heaviside(c3d_ctx* c) {
   ok = ok && c3d::launch_apply_bc(c->g, ib->Ureg, ib->Vreg, ib->Wreg, c->stream) == hipSuccess;
   ok = ok && c3d::launch_divergence(c->g, ib->Ureg, ib->Vreg, ib->Wreg, ib->Hc_ext, c->stream) == hipSuccess;
   ok = ok && B::launch_affine(ib->Hc_ext, -0.0, -1.0, ib->Hc_ext, c->nr, c->stream) == hipSuccess;
-  ok = ok && c3d::launch_fwd_x(c->g, false, nullptr, nullptr, nullptr, ib->Hc_ext, c->S, c->stream) == hipSuccess;
+  ok = ok && c3d::launch_fwd_x(c->g, false, nullptr, nullptr, nullptr, ib->Hc_ext, c->S, false, c->stream) == hipSuccess;
   if (!ok) return fail(c, C3D_EHIP, "Heaviside set-up failed");
   if ((rc = spectral_core(c))) return rc;
   ok = c3d::launch_inv_x(c->g, 0, c->S, ib->Hc_ext, c->P, 1.0, false, c->stream) == hipSuccess;

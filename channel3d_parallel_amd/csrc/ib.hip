@@ -8,6 +8,7 @@
 // order (the order of the reference's serial scatter), with no atomics.
 #include <hip/hip_runtime.h>
 
+#include "bc_images.hpp"
 #include "ib.hpp"
 
 #pragma clang fp contract(off)
@@ -541,7 +542,9 @@ __global__ __launch_bounds__(kBlock) void k_remove_mean(Markers m, double* __res
   f[l] = v;
 }
 
-// U = U_interim - U_reg - G(dt*(P_interim - phi))  (src/projection.f90:83-92)
+// U = U_interim - U_reg - G(dt*(P_interim - phi)) and the boundary conditions
+// of the result (src/projection.f90:83-94): the unique cells, each value
+// stored with its boundary images.
 __global__ __launch_bounds__(kBlock) void k_ib_correct(DevGrid g, const double* __restrict__ Uint,
                                                        const double* __restrict__ Vint,
                                                        const double* __restrict__ Wint,
@@ -553,39 +556,33 @@ __global__ __launch_bounds__(kBlock) void k_ib_correct(DevGrid g, const double* 
                                                        double* __restrict__ U,
                                                        double* __restrict__ V,
                                                        double* __restrict__ W) {
-  const int i = blockIdx.x * 64 + (threadIdx.x & 63) + 1;
-  const int j = blockIdx.y * 4 + (threadIdx.x >> 6) + 1;
-  const int k = blockIdx.z + 1;
-  const int nx = g.nx, ny = g.ny, nz = g.nz, nxg = g.nxg, nyg = g.nyg, nzg = g.nzg;
-  if (i > nxg || j > nyg) return;
+  const int i = blockIdx.x * 64 + (threadIdx.x & 63) + 2;
+  const int j = blockIdx.y * 4 + (threadIdx.x >> 6) + 2;
+  const int k = blockIdx.z + 2;
+  const int nx = g.nx, ny = g.ny, nxg = g.nxg, nyg = g.nyg;
+  if (i > nx - 1 || j > nyg - 1) return;
   auto q = [&](int a, int b, int c) {
     const size_t o = ridx(a, b, c, nxg, nyg);
     return dt * (Pint[o] - phi[o]);
   };
-  const bool core = i >= 2 && i <= nx - 1 && j >= 2 && k >= 2;
+  const double q0 = q(i, j, k);
   bool bad = false;
-  if (i <= nx) {  // U(nx, nyg, nzg)
+  {
     const size_t o = fidx(i, j, k, nx, nyg);
-    double G = 0.0;
-    if (core && j <= nyg - 1 && k <= nzg - 1) G = (q(i + 1, j, k) - q(i, j, k)) / g.dxg[i];
-    const double u = Uint[o] - Ureg[o] - G;
-    U[o] = u;
+    const double u = Uint[o] - Ureg[o] - (q(i + 1, j, k) - q0) / g.dxg[i];
+    put_u(g, U, i, j, k, u);
     bad |= !isfinite(u);
   }
-  if (j <= ny) {  // V(nxg, ny, nzg)
+  if (j <= ny - 1) {
     const size_t o = fidx(i, j, k, nxg, ny);
-    double G = 0.0;
-    if (core && j <= ny - 1 && k <= nzg - 1) G = (q(i, j + 1, k) - q(i, j, k)) / g.dyg[j];
-    const double v = Vint[o] - Vreg[o] - G;
-    V[o] = v;
+    const double v = Vint[o] - Vreg[o] - (q(i, j + 1, k) - q0) / g.dyg[j];
+    put_v(g, V, i, j, k, v);
     bad |= !isfinite(v);
   }
-  if (k <= nz) {  // W(nxg, nyg, nz)
+  {
     const size_t o = fidx(i, j, k, nxg, nyg);
-    double G = 0.0;
-    if (core && j <= nyg - 1 && k <= nz - 1) G = (q(i, j, k + 1) - q(i, j, k)) / g.dzg[k];
-    const double w = Wint[o] - Wreg[o] - G;
-    W[o] = w;
+    const double w = Wint[o] - Wreg[o] - (q(i, j, k + 1) - q0) / g.dzg[k];
+    put_w(g, W, i, j, k, w);
     bad |= !isfinite(w);
   }
   if (bad && g.nonfinite) atomicOr(g.nonfinite, 1u);
@@ -977,8 +974,8 @@ hipError_t launch_ib_correct(const DevGrid& g, const double* Uint, const double*
                              const double* Wint, const double* Ureg, const double* Vreg,
                              const double* Wreg, const double* Pint, const double* phi, double dt,
                              double* U, double* V, double* W, hipStream_t s) {
-  hipLaunchKernelGGL(k_ib_correct, dim3((g.nxg + 63) / 64, (g.nyg + 3) / 4, g.nzg), dim3(kBlock), 0,
-                     s, g, Uint, Vint, Wint, Ureg, Vreg, Wreg, Pint, phi, dt, U, V, W);
+  hipLaunchKernelGGL(k_ib_correct, dim3((g.nx - 2 + 63) / 64, (g.nyg - 2 + 3) / 4, g.nz - 2),
+                     dim3(kBlock), 0, s, g, Uint, Vint, Wint, Ureg, Vreg, Wreg, Pint, phi, dt, U, V, W);
   return hipGetLastError();
 }
 

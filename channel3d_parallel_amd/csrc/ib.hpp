@@ -125,8 +125,8 @@ hipError_t build_spread_map(const Markers& m, int comp, int n1, int n2, size_t n
 // holds 128 doubles of scratch.
 hipError_t launch_remove_mean(const Markers& m, double* f, const double* coef, const double* pj,
                               double* part, hipStream_t s);
-// U = (Uint - Ureg) - G(dt*(Pint - phi)) on the gradient's index ranges,
-// (Uint - Ureg) elsewhere (src/projection.f90:83-92).
+// U = (Uint - Ureg) - G(dt*(Pint - phi)) and the result's boundary conditions
+// (src/projection.f90:83-94); the boundary cells of the inputs are not read.
 hipError_t launch_ib_correct(const DevGrid& g, const double* Uint, const double* Vint,
                              const double* Wint, const double* Ureg, const double* Vreg,
                              const double* Wreg, const double* Pint, const double* phi, double dt,

@@ -10,6 +10,7 @@
 // ghost-inclusive), so host copies need no reshaping.
 #include <cstdlib>
 
+#include "bc_images.hpp"
 #include "fft_lds.hpp"
 #include "kernels.hpp"
 
@@ -63,7 +64,7 @@ __global__ __launch_bounds__(kBlock) void k_fwd_x(DevGrid g, const double* __res
                                                   cpx<real>* __restrict__ S,
                                                   double* __restrict__ bout,
                                                   const double* __restrict__ gauge,
-                                                  unsigned long long* __restrict__ rmax) {
+                                                  unsigned long long* __restrict__ rmax, int per) {
   constexpr bool FROM_UVW = (SRC == kSrcUVW || SRC == kSrcUVWB || SRC == kSrcUVWc);
   constexpr bool RESID = (SRC == kSrcResid);
   constexpr bool NTL = (SRC != kSrcUVWc);  // non-temporal U and W loads
@@ -91,13 +92,17 @@ __global__ __launch_bounds__(kBlock) void k_fwd_x(DevGrid g, const double* __res
   const double ry = g.rdyf[j];
   double wprev[NPL];  // W(k-1) of the next row: the W row of the row before
   if constexpr (FROM_UVW) {
-    const double* W0 = W + fidx(1, j, k0 + 1, nxg, nyg);
+    const double* W0 = W + fidx(1, j, (per && k0 == 0) ? g.nz - 1 : k0 + 1, nxg, nyg);
 #pragma unroll
     for (int p = 0; p < NPL; p++) {
       const int n = tid + p * kBlock;
       wprev[p] = (N % kBlock == 0 || n < N) ? W0[n + 1] : 0.0;
     }
   }
+  // per: the boundary values are taken from the interior (U(1) = U(nx-1),
+  // W(1) = W(nz-1), V = 0 on the walls), so the fields need no boundary
+  // conditions applied; else from the fields as they are
+  const bool vlo = per && j == 2, vhi = per && j == ny;
   // Residual r = b - M phi (D G on the unique cells, periodic in x and z, no
   // gradient on the wall faces, plus the (0,0)-mode gauge row at j = 2), with
   // U = phi and rhs_in = b; each lane walks its x positions down the tile's
@@ -158,6 +163,7 @@ __global__ __launch_bounds__(kBlock) void k_fwd_x(DevGrid g, const double* __res
         for (int p = 0; p < NPL; p++) {
           const int n = tid + p * kBlock;
           if (N % kBlock == 0 || n < N) {
+            const int nm = (per && n == 0) ? N : n;
             // x index i = n + 2 -> offset n + 1 in the row.  U and W rows
             // are read by this workgroup only: non-temporal when the fields
             // are too large to stay in cache between kernels.  V rows are
@@ -165,15 +171,15 @@ __global__ __launch_bounds__(kBlock) void k_fwd_x(DevGrid g, const double* __res
             // workgroup): cached.
             if constexpr (NTL) {
               v[r][p][0] = __builtin_nontemporal_load(&Ur[n + 1]);
-              v[r][p][1] = __builtin_nontemporal_load(&Ur[n]);
+              v[r][p][1] = __builtin_nontemporal_load(&Ur[nm]);
               v[r][p][4] = __builtin_nontemporal_load(&Wr[n + 1]);
             } else {
               v[r][p][0] = Ur[n + 1];
-              v[r][p][1] = Ur[n];
+              v[r][p][1] = Ur[nm];
               v[r][p][4] = Wr[n + 1];
             }
-            v[r][p][2] = Vr[n + 1];
-            v[r][p][3] = Vm[n + 1];
+            v[r][p][2] = vhi ? 0.0 : Vr[n + 1];
+            v[r][p][3] = vlo ? 0.0 : Vm[n + 1];
           }
         }
       } else if constexpr (RESID) {
@@ -452,6 +458,26 @@ __global__ __launch_bounds__(kBlock) void k_inv_x(DevGrid g, const cpx<real>* __
 
   const double norm = (double)((long long)g.nxp * (long long)nzp);
   const double cP = dt * (8.0 / 15.0);
+  // P of this point (i = n + 2) with its copies (src/poisson.f90:91-98): the
+  // periodic ones i = nxg-1 and k = nzp+2, then the ghosts, which repeat
+  // their neighbour in x, y and z: i = 1, nxg, j = 1, nyg, k = 1, nzg.  All
+  // of them repeat an interior value, so they need no pass of their own.
+  auto store_p = [&](int n, int k, double v, bool dupz) {
+    for (int b = 0; b < 2; b++) {
+      if (b == 1 && jj != 0 && j != nyg - 1) break;
+      const int jb = b == 0 ? j : (jj == 0 ? 1 : nyg);
+      for (int c = 0; c < (dupz ? 4 : 1); c++) {
+        const int kc = c == 0 ? k : (c == 1 ? nzp + 2 : (c == 2 ? 1 : g.nzg));
+        double* row = P + fidx(2, jb, kc, nxg, nyg);
+        row[n] = v;
+        if (n == 0) {
+          row[-1] = v;
+          row[N] = v;
+          row[N + 1] = v;
+        }
+      }
+    }
+  };
   const int idup = nxg - 1;     // x duplicate of i = 2
   const int kdup = nzp + 2;     // z duplicate of k = 2
   // rows walked with uniform row bases; lane owns x positions tid + p*kBlock
@@ -461,10 +487,8 @@ __global__ __launch_bounds__(kBlock) void k_inv_x(DevGrid g, const cpx<real>* __
   for (int t = 0; t < TK; t++) {
     const int k = k0 + t + 2;
     double* orow = out + ridx(2, j, k, nxg, nyg);      // x index 2 at offset 0
-    double* prow = P + fidx(2, j, k, nxg, nyg);
     const bool dupz = (k0 == 0 && t == 0);             // row k = 2 also fills k = nzp+2
     double* orow2 = out + ridx(2, j, kdup, nxg, nyg);
-    double* prow2 = P + fidx(2, j, kdup, nxg, nyg);
 #pragma unroll
     for (int p = 0; p < NPL; p++) {
       const int n = tid + p * kBlock;
@@ -485,21 +509,18 @@ __global__ __launch_bounds__(kBlock) void k_inv_x(DevGrid g, const cpx<real>* __
         const double o = (MODE == 1) ? phi / dt : phi;
         if constexpr (OUT) __builtin_nontemporal_store(o, &orow[n]);
         if constexpr (MODE == 5) out2[at] = corr;
-        if (rk1) prow[n] = phi / cP;
+        if (rk1) store_p(n, k, phi / cP, dupz);
         if (n == 0) {  // x duplicate i = nxg-1 (offset nxp)
           if constexpr (OUT) orow[N] = o;
           if constexpr (MODE == 5) out2[at + N] = corr;
-          if (rk1) prow[N] = phi / cP;
         }
         if (dupz) {
           const size_t at2 = ridx(2, j, kdup, nxg, nyg) + n;
           if constexpr (OUT) orow2[n] = o;
           if constexpr (MODE == 5) out2[at2] = corr;
-          if (rk1) prow2[n] = phi / cP;
           if (n == 0) {
             if constexpr (OUT) orow2[N] = o;
             if constexpr (MODE == 5) out2[at2 + N] = corr;
-            if (rk1) prow2[N] = phi / cP;
           }
         }
       }
@@ -549,28 +570,6 @@ __global__ __launch_bounds__(kBlock) void k_gauge_final(DevGrid g, const double*
 }
 
 // ---------------------------------------------------------------------------
-// P ghost copies (src/poisson.f90:93-98): x, then y, then z.
-// ---------------------------------------------------------------------------
-__global__ void k_pghost_x(DevGrid g, double* __restrict__ P) {
-  const int j = blockIdx.x * blockDim.x + threadIdx.x + 1, k = blockIdx.y + 1;
-  if (j > g.nyg) return;
-  P[fidx(1, j, k, g.nxg, g.nyg)] = P[fidx(2, j, k, g.nxg, g.nyg)];
-  P[fidx(g.nxg, j, k, g.nxg, g.nyg)] = P[fidx(g.nxg - 1, j, k, g.nxg, g.nyg)];
-}
-__global__ void k_pghost_y(DevGrid g, double* __restrict__ P) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x + 1, k = blockIdx.y + 1;
-  if (i > g.nxg) return;
-  P[fidx(i, 1, k, g.nxg, g.nyg)] = P[fidx(i, 2, k, g.nxg, g.nyg)];
-  P[fidx(i, g.nyg, k, g.nxg, g.nyg)] = P[fidx(i, g.nyg - 1, k, g.nxg, g.nyg)];
-}
-__global__ void k_pghost_z(DevGrid g, double* __restrict__ P) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x + 1, j = blockIdx.y + 1;
-  if (i > g.nxg) return;
-  P[fidx(i, j, 1, g.nxg, g.nyg)] = P[fidx(i, j, 2, g.nxg, g.nyg)];
-  P[fidx(i, j, g.nzg, g.nxg, g.nyg)] = P[fidx(i, j, g.nzg - 1, g.nxg, g.nyg)];
-}
-
-// ---------------------------------------------------------------------------
 // Gradient correction: U = U - G(dt*Pint) on the index ranges of
 // src/differential_operators.f90:28-50 (faces outside them keep U).
 // SPLIT: U = U - (G(phi1) + G(phic)) for a potential kept as two parts (the
@@ -579,7 +578,9 @@ __global__ void k_pghost_z(DevGrid g, double* __restrict__ P) {
 // split kernel also writes P_interim = (phi1 + phic)/dt to pout on the whole
 // rhs_p shape (the duplicates i = nxg-1 from i = 2, the zero plane nzg).
 // ---------------------------------------------------------------------------
-template <int KC, bool SPLIT>
+// BC: the corrected velocity's boundary conditions too (bc_images.hpp): the
+// unique planes only, each value stored with its images.
+template <int KC, bool SPLIT, bool BC>
 __global__ __launch_bounds__(kBlock) void k_grad_correct(DevGrid g, double* __restrict__ U,
                                                          double* __restrict__ V,
                                                          double* __restrict__ W,
@@ -626,12 +627,18 @@ __global__ __launch_bounds__(kBlock) void k_grad_correct(DevGrid g, double* __re
 #pragma unroll
   for (int kk = 0; kk < KC; kk++) {
     const int k = kb + kk;
-    if (k > nzg - 1) break;
+    if (k > (BC ? nz - 1 : nzg - 1)) break;
     if constexpr (SPLIT) {
       const double o = (p + pc) / dt;
       pout[ridx(i, j, k, nxg, nyg)] = o;
       if (i == 2) pout[ridx(nxg - 1, j, k, nxg, nyg)] = o;
-      if (k == nzg - 1) {
+      if constexpr (BC) {
+        if (k == 2) {  // the duplicate plane nzg-1
+          pout[ridx(i, j, nzg - 1, nxg, nyg)] = o;
+          if (i == 2) pout[ridx(nxg - 1, j, nzg - 1, nxg, nyg)] = o;
+        }
+      }
+      if (k == (BC ? 2 : nzg - 1)) {
         pout[ridx(i, j, nzg, nxg, nyg)] = 0.0;
         if (i == 2) pout[ridx(nxg - 1, j, nzg, nxg, nyg)] = 0.0;
       }
@@ -644,14 +651,16 @@ __global__ __launch_bounds__(kBlock) void k_grad_correct(DevGrid g, double* __re
     const double pxc = (i == ie) ? pxce : pxcn;
     const size_t iu = fidx(i, j, k, nx, nyg);
     const double u = U[iu] - dif(px, pxc, p, pc) / hx;
-    U[iu] = u;
+    if constexpr (BC) put_u(g, U, i, j, k, u);
+    else U[iu] = u;
     bad |= !isfinite(u);
     if (j <= ny - 1) {
       double pyc;
       const double py = pot(ridx(i, j + 1, k, nxg, nyg), pyc);
       const size_t iv = fidx(i, j, k, nxg, ny);
       const double v = V[iv] - dif(py, pyc, p, pc) / hy;
-      V[iv] = v;
+      if constexpr (BC) put_v(g, V, i, j, k, v);
+      else V[iv] = v;
       bad |= !isfinite(v);
     }
     if (k <= nz - 1) {
@@ -659,7 +668,8 @@ __global__ __launch_bounds__(kBlock) void k_grad_correct(DevGrid g, double* __re
       const double pz = pot(ridx(i, j, k + 1, nxg, nyg), pzc);
       const size_t iw = fidx(i, j, k, nxg, nyg);
       const double w = W[iw] - dif(pz, pzc, p, pc) / g.dzg[k];
-      W[iw] = w;
+      if constexpr (BC) put_w(g, W, i, j, k, w);
+      else W[iw] = w;
       bad |= !isfinite(w);
       p = pz;
       pc = pzc;
@@ -872,7 +882,7 @@ inline dim3 grid_pts(const DevGrid& g, int ni, int nj, int nk) {
 }  // namespace
 
 hipError_t launch_fwd_x(const DevGrid& g, bool from_uvw, const double* U, const double* V,
-                        const double* W, const double* rhs, cpx<double>* S, hipStream_t s) {
+                        const double* W, const double* rhs, cpx<double>* S, bool per, hipStream_t s) {
   const int tk = tile_rows(g.nxp, g.nzp);
   dim3 grid(g.nzp / tk, g.nym);
   // U, V, W together below 128 MB stay in the 256 MB last-level cache
@@ -882,29 +892,29 @@ hipError_t launch_fwd_x(const DevGrid& g, bool from_uvw, const double* U, const 
   C3D_DISPATCH_N(g.nxp, C3D_DISPATCH_TK(tk, {
     if (from_uvw && small)
       hipLaunchKernelGGL((k_fwd_x<double, NN, TK, kSrcUVWc>), grid, dim3(kBlock), 0, s, g, U, V, W,
-                         (const void*)rhs, g.twx64, S, nullptr, nullptr, nullptr);
+                         (const void*)rhs, g.twx64, S, nullptr, nullptr, nullptr, per ? 1 : 0);
     else if (from_uvw)
       hipLaunchKernelGGL((k_fwd_x<double, NN, TK, kSrcUVW>), grid, dim3(kBlock), 0, s, g, U, V, W,
-                         (const void*)rhs, g.twx64, S, nullptr, nullptr, nullptr);
+                         (const void*)rhs, g.twx64, S, nullptr, nullptr, nullptr, per ? 1 : 0);
     else
       hipLaunchKernelGGL((k_fwd_x<double, NN, TK, kSrcRhs>), grid, dim3(kBlock), 0, s, g, U, V, W,
-                         (const void*)rhs, g.twx64, S, nullptr, nullptr, nullptr);
+                         (const void*)rhs, g.twx64, S, nullptr, nullptr, nullptr, per ? 1 : 0);
   }));
   return hipGetLastError();
 }
 
 hipError_t launch_fwd_x32(const DevGrid& g, const double* U, const double* V, const double* W,
-                          double* b, cpx<float>* S, hipStream_t s) {
+                          double* b, cpx<float>* S, bool per, hipStream_t s) {
   if (!U || !V || !W) return hipErrorInvalidValue;
   const int tk = tile_rows(g.nxp, g.nzp);
   dim3 grid(g.nzp / tk, g.nym);
   C3D_DISPATCH_N(g.nxp, C3D_DISPATCH_TK(tk, {
     if (b)
       hipLaunchKernelGGL((k_fwd_x<float, NN, TK, kSrcUVWB>), grid, dim3(kBlock), 0, s, g, U, V, W,
-                         (const void*)nullptr, g.twx32, S, b, nullptr, nullptr);
+                         (const void*)nullptr, g.twx32, S, b, nullptr, nullptr, per ? 1 : 0);
     else
       hipLaunchKernelGGL((k_fwd_x<float, NN, TK, kSrcUVW>), grid, dim3(kBlock), 0, s, g, U, V, W,
-                         (const void*)nullptr, g.twx32, S, nullptr, nullptr, nullptr);
+                         (const void*)nullptr, g.twx32, S, nullptr, nullptr, nullptr, per ? 1 : 0);
   }));
   return hipGetLastError();
 }
@@ -921,7 +931,7 @@ hipError_t fwd_x_resid(const DevGrid& g, const double* b, const double* phi, dou
   hipLaunchKernelGGL(k_gauge_final, dim3(1), dim3(kBlock), 0, s, g, (const double*)(gauge + 1), gauge);
   C3D_DISPATCH_N(g.nxp, C3D_DISPATCH_TK(tk, {
     hipLaunchKernelGGL((k_fwd_x<real, NN, TK, kSrcResid>), grid, dim3(kBlock), 0, s, g, phi,
-                       nullptr, nullptr, (const void*)b, tw, S, rout, (const double*)gauge, rmax);
+                       nullptr, nullptr, (const void*)b, tw, S, rout, (const double*)gauge, rmax, 0);
   }));
   return hipGetLastError();
 }
@@ -939,12 +949,12 @@ hipError_t launch_fwd_x_resid64(const DevGrid& g, const double* b, const double*
 }
 
 hipError_t launch_fwd_x_b64(const DevGrid& g, const double* U, const double* V, const double* W,
-                            double* b, cpx<double>* S, hipStream_t s) {
+                            double* b, cpx<double>* S, bool per, hipStream_t s) {
   const int tk = tile_rows(g.nxp, g.nzp);
   dim3 grid(g.nzp / tk, g.nym);
   C3D_DISPATCH_N(g.nxp, C3D_DISPATCH_TK(tk, {
     hipLaunchKernelGGL((k_fwd_x<double, NN, TK, kSrcUVWB>), grid, dim3(kBlock), 0, s, g, U, V, W,
-                       (const void*)nullptr, g.twx64, S, b, nullptr, nullptr);
+                       (const void*)nullptr, g.twx64, S, b, nullptr, nullptr, per ? 1 : 0);
   }));
   return hipGetLastError();
 }
@@ -1034,13 +1044,6 @@ hipError_t launch_inv_x32(const DevGrid& g, int mode, const cpx<float>* S, const
   return inv_x_modes<float>(g, mode, S, g.twx32, phi_in, phi_in2, out, out2, P, dt, rk1, s);
 }
 
-hipError_t launch_p_ghosts(const DevGrid& g, double* P, hipStream_t s) {
-  hipLaunchKernelGGL(k_pghost_x, dim3((g.nyg + 63) / 64, g.nzg), dim3(64), 0, s, g, P);
-  hipLaunchKernelGGL(k_pghost_y, dim3((g.nxg + 63) / 64, g.nzg), dim3(64), 0, s, g, P);
-  hipLaunchKernelGGL(k_pghost_z, dim3((g.nxg + 63) / 64, g.nyg), dim3(64), 0, s, g, P);
-  return hipGetLastError();
-}
-
 // z planes per lane of the gradient correction (at 384x193x384, 2 measured
 // fastest for the single potential: 0.303 against 0.305 ms for 1, more
 // workgroups in flight; 4 for the two-part potential: 0.457 against
@@ -1055,15 +1058,15 @@ static int grad_kc(bool split) {
 }
 
 namespace {
-template <bool SPLIT>
+template <bool SPLIT, bool BC>
 hipError_t grad_correct_any(const DevGrid& g, double* U, double* V, double* W, const double* Pint,
                             const double* phic, double* pout, double dt, hipStream_t s) {
   const int kc = grad_kc(SPLIT);
-  const dim3 grid = grid_pts(g, g.nx - 2, g.nyg - 2, (g.nzg - 2 + kc - 1) / kc);
+  const dim3 grid = grid_pts(g, g.nx - 2, g.nyg - 2, ((BC ? g.nz : g.nzg) - 2 + kc - 1) / kc);
   switch (kc) {
 #define C3D_GC_CASE(KC)                                                                         \
   case KC:                                                                                      \
-    hipLaunchKernelGGL((k_grad_correct<KC, SPLIT>), grid, dim3(kBlock), 0, s, g, U, V, W, Pint,     \
+    hipLaunchKernelGGL((k_grad_correct<KC, SPLIT, BC>), grid, dim3(kBlock), 0, s, g, U, V, W, Pint, \
                        phic, pout, dt);                                                         \
     break;
     C3D_GC_CASE(1)
@@ -1081,14 +1084,16 @@ hipError_t grad_correct_any(const DevGrid& g, double* U, double* V, double* W, c
 }  // namespace
 
 hipError_t launch_grad_correct(const DevGrid& g, double* U, double* V, double* W, const double* Pint,
-                               double dt, hipStream_t s) {
-  return grad_correct_any<false>(g, U, V, W, Pint, nullptr, nullptr, dt, s);
+                               double dt, bool bc, hipStream_t s) {
+  return bc ? grad_correct_any<false, true>(g, U, V, W, Pint, nullptr, nullptr, dt, s)
+            : grad_correct_any<false, false>(g, U, V, W, Pint, nullptr, nullptr, dt, s);
 }
 
 hipError_t launch_grad_correct_split(const DevGrid& g, double* U, double* V, double* W,
                                      const double* phi1, const double* phic, double* Pint, double dt,
-                                     hipStream_t s) {
-  return grad_correct_any<true>(g, U, V, W, phi1, phic, Pint, dt, s);
+                                     bool bc, hipStream_t s) {
+  return bc ? grad_correct_any<true, true>(g, U, V, W, phi1, phic, Pint, dt, s)
+            : grad_correct_any<true, false>(g, U, V, W, phi1, phic, Pint, dt, s);
 }
 
 hipError_t launch_apply_bc(const DevGrid& g, double* U, double* V, double* W, hipStream_t s) {

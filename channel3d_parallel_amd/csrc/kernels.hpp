@@ -51,9 +51,11 @@ __host__ __device__ __forceinline__ size_t ridx(int i, int j, int k, int nxg, in
 }
 
 // Forward x transform.  from_uvw: input is div(U,V,W) computed on the fly,
-// else the rhs_p array.  Writes the half spectrum S[j][kx][kz].
+// else the rhs_p array.  Writes the half spectrum S[j][kx][kz].  per: the
+// divergence takes the boundary values from the interior (the periodic
+// images and V = 0 on the walls) instead of the fields' boundary cells.
 hipError_t launch_fwd_x(const DevGrid& g, bool from_uvw, const double* U, const double* V,
-                        const double* W, const double* rhs, cpx<double>* S, hipStream_t s);
+                        const double* W, const double* rhs, cpx<double>* S, bool per, hipStream_t s);
 hipError_t launch_fft_z(const DevGrid& g, int sign, cpx<double>* S, hipStream_t s);
 // Tridiagonal solve along y for every (kx,kz): the partitioned register
 // solver from 33 to 768 rows, else the plain Thomas sweep with CP, nym*nxh*nzp
@@ -63,17 +65,18 @@ bool tri_needs_scratch(const DevGrid& g);
 bool tri_part_supported(const DevGrid& g);
 hipError_t launch_tri(const DevGrid& g, cpx<double>* S, double* CP, hipStream_t s);
 // Inverse x transform.  mode 0: out = solution rhs_p (Poisson drop-in).
-// mode 1: out = P_interim = solution/dt (projection).  rk1: also write P.
+// mode 1: out = P_interim = solution/dt (projection).  rk1: also write P,
+// ghosts included.
 hipError_t launch_inv_x(const DevGrid& g, int mode, const cpx<double>* S, double* out, double* P,
                         double dt, bool rk1, hipStream_t s);
 // Refinement pieces (mixed precision: FP32 forward spectra; FP64: the same
 // sweeps on FP64 spectra).  launch_fwd_x32: divergence of U, V, W (FP64,
 // also stored to b when b != null) -> FP32 spectrum.
 hipError_t launch_fwd_x32(const DevGrid& g, const double* U, const double* V, const double* W,
-                          double* b, cpx<float>* S, hipStream_t s);
+                          double* b, cpx<float>* S, bool per, hipStream_t s);
 // FP64 spectrum of div(U, V, W), the FP64 divergence also stored to b.
 hipError_t launch_fwd_x_b64(const DevGrid& g, const double* U, const double* V, const double* W,
-                            double* b, cpx<double>* S, hipStream_t s);
+                            double* b, cpx<double>* S, bool per, hipStream_t s);
 // The refinement residual r = b - M phi formed on the fly as the forward
 // transform's input, M = D G on the unique cells plus the spectral solver's
 // (0,0)-mode gauge row (gauge: nzp + 1 doubles of scratch).  The FP32 variant
@@ -108,16 +111,15 @@ hipError_t launch_inv_x64_ref(const DevGrid& g, int mode, const cpx<double>* S, 
 hipError_t launch_inv_x32(const DevGrid& g, int mode, const cpx<float>* S, const double* phi_in,
                           const double* phi_in2, double* out, double* out2, double* P, double dt,
                           bool rk1, hipStream_t s);
-// Ghost copies of P (src/poisson.f90:93-98), in the reference order.
-hipError_t launch_p_ghosts(const DevGrid& g, double* P, hipStream_t s);
-// U -= G(dt * Pint) on the gradient's index ranges.
+// U -= G(dt * Pint) on the gradient's index ranges; bc: and the boundary
+// conditions of the result (the whole fields as launch_apply_bc leaves them).
 hipError_t launch_grad_correct(const DevGrid& g, double* U, double* V, double* W, const double* Pint,
-                               double dt, hipStream_t s);
+                               double dt, bool bc, hipStream_t s);
 // U -= G(phi1) + G(phic), each part differenced on its own; Pint =
 // (phi1 + phic)/dt on the whole rhs_p shape.
 hipError_t launch_grad_correct_split(const DevGrid& g, double* U, double* V, double* W,
                                      const double* phi1, const double* phic, double* Pint, double dt,
-                                     hipStream_t s);
+                                     bool bc, hipStream_t s);
 // apply_boundary_conditions on device-resident staggered fields.
 hipError_t launch_apply_bc(const DevGrid& g, double* U, double* V, double* W, hipStream_t s);
 // Divergence into an rhs_p-shaped array (plane nzg zero).
@@ -139,7 +141,9 @@ hipError_t launch_rhs(const DevGrid& g, const double* U, const double* V, const 
 hipError_t launch_rk_update(const DevGrid& g, int which, int stage, double dt, const double* F1,
                             const double* F2, const double* F3, const double* Xo, double* X,
                             hipStream_t s);
-hipError_t launch_add_u(const DevGrid& g, double* U, double d, hipStream_t s);
+// U(2:nx-1, 2:nyg-1, 2:nzg-1) += d; bc: and U's boundary conditions (a U
+// whose boundary cells hold the images of its interior keeps them).
+hipError_t launch_add_u(const DevGrid& g, double* U, double d, bool bc, hipStream_t s);
 // Fused right-hand side and stage update (rk3_fast.hip), to round-off of the
 // reference's operations: reads the stage input U, V, W, writes the updated
 // interiors Un, Vn, Wn (a different set of fields) and, for stages 1 and 2,

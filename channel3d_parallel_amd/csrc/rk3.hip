@@ -8,6 +8,7 @@
 // contraction is disabled so the results round exactly as written.
 #include <cstdlib>
 
+#include "bc_images.hpp"
 #include "kernels.hpp"
 
 #pragma clang fp contract(off)
@@ -107,7 +108,9 @@ __global__ __launch_bounds__(kB) void k_rk_update(int n1, int n2, int i1, int j1
   (void)k1;
 }
 
-// U(2:nx-1, 2:nyg-1, 2:nzg-1) += d  (src/time_integration.f90:190)
+// U(2:nx-1, 2:nyg-1, 2:nzg-1) += d  (src/time_integration.f90:190); BC: the
+// unique cells, each with its boundary images.
+template <bool BC>
 __global__ __launch_bounds__(kB) void k_add_u(DevGrid g, double* __restrict__ U, double d) {
   unsigned bx, by, bz;
   xcd_tile(bx, by, bz);  // neighbouring tiles on one XCD (shared halo rows)
@@ -116,7 +119,9 @@ __global__ __launch_bounds__(kB) void k_add_u(DevGrid g, double* __restrict__ U,
   const int k = bz + 2;
   if (i > g.nx - 1 || j > g.nyg - 1) return;
   const size_t o = fidx(i, j, k, g.nx, g.nyg);
-  U[o] = U[o] + d;
+  const double u = U[o] + d;
+  if constexpr (BC) put_u(g, U, i, j, k, u);
+  else U[o] = u;
 }
 
 // compute_dt maxima (src/time_integration.f90:228-239): max over the
@@ -349,8 +354,10 @@ hipError_t launch_rk_update(const DevGrid& g, int which, int stage, double dt, c
   return hipGetLastError();
 }
 
-hipError_t launch_add_u(const DevGrid& g, double* U, double d, hipStream_t s) {
-  hipLaunchKernelGGL(k_add_u, gpts(g.nx - 2, g.nyg - 2, g.nzg - 2), dim3(kB), 0, s, g, U, d);
+hipError_t launch_add_u(const DevGrid& g, double* U, double d, bool bc, hipStream_t s) {
+  const dim3 grid = gpts(g.nx - 2, g.nyg - 2, (bc ? g.nz : g.nzg) - 2);
+  if (bc) hipLaunchKernelGGL(k_add_u<true>, grid, dim3(kB), 0, s, g, U, d);
+  else hipLaunchKernelGGL(k_add_u<false>, grid, dim3(kB), 0, s, g, U, d);
   return hipGetLastError();
 }
 
