@@ -129,7 +129,13 @@ struct c3d_ctx {
   cpx<double>* S = nullptr;
   double* CP = nullptr;
   unsigned long long* red = nullptr;
-  unsigned* nanflag = nullptr;  // g.nonfinite: set by the velocity corrections
+  // Results that kernels store straight into (coherent) host memory, read
+  // after a synchronisation: no copy and no staging per result.
+  struct HostWords {
+    double v[8];         // flow integral and its norm
+    unsigned nonfinite;  // g.nonfinite: set by the velocity corrections
+  };
+  HostWords* host = nullptr;
   double* psum = nullptr;  // 7*nyg plane sums of compute_statistics
   double* mon = nullptr;   // output_monitor partials and results
   size_t nu = 0, nv = 0, nw = 0, np = 0, nr = 0, nspec = 0;
@@ -542,14 +548,19 @@ int c3d_create(const c3d_desc* desc, c3d_ctx** out) {
       (rc = dalloc(c, &c->Pint, c->nr)) || (rc = dalloc(c, &c->rhs, c->nr)) ||
       (rc = dalloc(c, &c->xU, c->nu)) || (rc = dalloc(c, &c->xV, c->nv)) ||
       (rc = dalloc(c, &c->xW, c->nw)) || (rc = dalloc(c, &c->xF, interior_total(c))) ||
-      (rc = dalloc(c, &c->part, 2 * (size_t)c3d::massflow_rows(c->g) + 2)) ||
-      (rc = dalloc(c, &c->nanflag, 1)) ||
+      (rc = dalloc(c, &c->part, 2 * (size_t)c3d::massflow_parts(c->g) + 2)) ||
       (rc = dalloc(c, &c->S, c->nspec)) ||
       (c3d::tri_needs_scratch(c->g) && (rc = dalloc(c, &c->CP, c->nspec))) ||
       (rc = dalloc(c, &c->red, kRedRefine + (size_t)kMaxRef * kResSlots)))
     return cleanup(rc);
   if (d.precision == C3D_PREC_MIXED && (rc = dalloc(c, &c->S32, c->nspec))) return cleanup(rc);
-  c->g.nonfinite = c->nanflag;
+  if (hipHostMalloc((void**)&c->host, sizeof(*c->host), hipHostMallocCoherent) != hipSuccess) {
+    c->host = nullptr;
+    (void)hipGetLastError();
+    return cleanup(C3D_ENOMEM);
+  }
+  std::memset((void*)c->host, 0, sizeof(*c->host));
+  c->g.nonfinite = &c->host->nonfinite;
   {
     const char* e = getenv("C3D_RHS_EXACT");
     c->rhs_exact = e && atoi(e) != 0;
@@ -563,8 +574,7 @@ int c3d_create(const c3d_desc* desc, c3d_ctx** out) {
     c->nref = c->mixed_inv64 ? 1 : 2;
     if ((rc = refine_buffers(c, c->nref))) return cleanup(rc);
   }
-  if (hipMemsetAsync(c->nanflag, 0, sizeof(unsigned), c->stream) != hipSuccess ||
-      hipMemsetAsync(c->U, 0, c->nu * 8, c->stream) != hipSuccess ||
+  if (hipMemsetAsync(c->U, 0, c->nu * 8, c->stream) != hipSuccess ||
       hipMemsetAsync(c->V, 0, c->nv * 8, c->stream) != hipSuccess ||
       hipMemsetAsync(c->W, 0, c->nw * 8, c->stream) != hipSuccess ||
       hipMemsetAsync(c->P, 0, c->np * 8, c->stream) != hipSuccess ||
@@ -579,6 +589,7 @@ int c3d_destroy(c3d_ctx* c) {
   if (!c) return C3D_OK;
   if (c->stream) (void)hipStreamSynchronize(c->stream);
   for (void* p : c->allocs) (void)hipFree(p);
+  if (c->host) (void)hipHostFree(c->host);
   if (c->stream) (void)hipStreamDestroy(c->stream);
   if (c->mlp)
     for (void* p : c->mlp->bufs) (void)hipFree(p);
@@ -962,14 +973,20 @@ static int rk_stage_fast(c3d_ctx* c, int st, double dt) {
   return 0;
 }
 
+// The flow integral and its norm of U, on the device in *sums and, once the
+// stream is synchronised, in c->host->v[0..1].
+static int mass_flow_launch(c3d_ctx* c, const double* U, double** sums) {
+  *sums = c->part + 2 * (size_t)c3d::massflow_parts(c->g);
+  HIPCHK(c, c3d::launch_massflow(c->g, U, c->Hm, c->part, *sums, c->host->v, c->stream));
+  return 0;
+}
+
 static int mass_flow(c3d_ctx* c, const double* U, double* q) {
-  double* out = c->part + 2 * (size_t)c3d::massflow_rows(c->g);
-  HIPCHK(c, c3d::launch_massflow(c->g, U, c->Hm, c->part, out, c->stream));
-  double h[2];
-  HIPCHK(c, hipMemcpyAsync(h, out, sizeof(h), hipMemcpyDeviceToHost, c->stream));
-  int rc = sync(c);
+  double* sums = nullptr;
+  int rc = mass_flow_launch(c, U, &sums);
+  if (!rc) rc = sync(c);
   if (rc) return rc;
-  *q = h[0] / h[1];
+  *q = c->host->v[0] / c->host->v[1];
   return 0;
 }
 
@@ -1217,15 +1234,14 @@ int c3d_wall_shear(c3d_ctx* c, double* utau, double* wtau, double* Umean, double
 
 int c3d_add_to_u(c3d_ctx* c, double d) {
   if (!c) return C3D_EINVAL;
-  HIPCHK(c, c3d::launch_add_u(c->g, c->U, d, false, c->stream));
+  HIPCHK(c, c3d::launch_add_u(c->g, c->U, d, c->stream));
   return sync(c);
 }
 
 int c3d_time_step_rk3(c3d_ctx* c, double dt, int x_mass_cte, double q0) {
   if (!c || !(dt > 0.0)) return C3D_EINVAL;
   int rc = ensure_rk(c);
-  if (!rc && hipMemsetAsync(c->nanflag, 0, sizeof(unsigned), c->stream) != hipSuccess)
-    rc = fail(c, C3D_EHIP, "non-finite flag reset");
+  if (!rc) c->host->nonfinite = 0;  // no velocity correction of this context is running
   const bool exact = c->rhs_exact;
   if (!rc && exact) rc = save_state(c);  // src/time_integration.f90:91-94 (fused: kept in place)
   const double t0 = c->t;
@@ -1248,23 +1264,18 @@ int c3d_time_step_rk3(c3d_ctx* c, double dt, int x_mass_cte, double q0) {
     }
   }
   if (!rc && x_mass_cte == 1) {  // :187-193
-    const double prev = c->dPdx;
-    double ub = 0.0;
-    rc = mass_flow(c, c->U, &ub);
-    if (!rc) {
-      const double d = q0 - ub;
-      if (c3d::launch_add_u(c->g, c->U, d, true, c->stream) != hipSuccess)
-        rc = fail(c, C3D_EHIP, "mass-flow correction");
-      c->dPdx = 0.5 * (prev + d / dt);
-    }
+    double* sums = nullptr;
+    rc = mass_flow_launch(c, c->U, &sums);
+    if (!rc && c3d::launch_hold_flow(c->g, c->U, sums, q0, c->stream) != hipSuccess)
+      rc = fail(c, C3D_EHIP, "mass-flow correction");
   }
+  if (!rc) rc = sync(c);
+  if (!rc && x_mass_cte == 1)
+    c->dPdx = 0.5 * (c->dPdx + (q0 - c->host->v[0] / c->host->v[1]) / dt);
   // NaN stop of compute_statistics (src/statistics.f90:142-144), checked at
   // every step: the velocity corrections flag any non-finite value they write
-  unsigned bad = 0;
-  if (!rc && hipMemcpyAsync(&bad, c->nanflag, sizeof(bad), hipMemcpyDeviceToHost, c->stream) != hipSuccess)
-    rc = fail(c, C3D_EHIP, "non-finite flag read");
-  if (!rc) rc = sync(c);
-  if (!rc && bad) rc = fail(c, C3D_ENAN, "non-finite velocity after the time step at t = %.6e", c->t);
+  if (!rc && c->host->nonfinite)
+    rc = fail(c, C3D_ENAN, "non-finite velocity after the time step at t = %.6e", c->t);
   return rc;
 }
 

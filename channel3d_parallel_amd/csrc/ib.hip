@@ -585,7 +585,7 @@ __global__ __launch_bounds__(kBlock) void k_ib_correct(DevGrid g, const double* 
     put_w(g, W, i, j, k, w);
     bad |= !isfinite(w);
   }
-  if (bad && g.nonfinite) atomicOr(g.nonfinite, 1u);
+  if (bad && g.nonfinite) *g.nonfinite = 1u;  // every writer writes the same
 }
 
 __global__ void k_affine(const double* __restrict__ x, double a, double b, double* __restrict__ y,

@@ -675,7 +675,7 @@ __global__ __launch_bounds__(kBlock) void k_grad_correct(DevGrid g, double* __re
       pc = pzc;
     }
   }
-  if (bad && g.nonfinite) atomicOr(g.nonfinite, 1u);
+  if (bad && g.nonfinite) *g.nonfinite = 1u;  // every writer writes the same
 }
 
 // ---------------------------------------------------------------------------

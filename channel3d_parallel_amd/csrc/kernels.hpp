@@ -40,8 +40,9 @@ struct DevGrid {
   const cpx<double>* twz64;
   const cpx<float>* twx32;
   const cpx<float>* twz32;
-  // flag word: the velocity-correction kernels (k_grad_correct,
-  // k_ib_correct) set it to 1 when a corrected velocity is not finite
+  // flag word in host memory: the velocity-correction kernels
+  // (k_grad_correct, k_ib_correct) set it to 1 when a corrected velocity is
+  // not finite, and write it only then
   unsigned* nonfinite;
 };
 
@@ -141,9 +142,10 @@ hipError_t launch_rhs(const DevGrid& g, const double* U, const double* V, const 
 hipError_t launch_rk_update(const DevGrid& g, int which, int stage, double dt, const double* F1,
                             const double* F2, const double* F3, const double* Xo, double* X,
                             hipStream_t s);
-// U(2:nx-1, 2:nyg-1, 2:nzg-1) += d; bc: and U's boundary conditions (a U
-// whose boundary cells hold the images of its interior keeps them).
-hipError_t launch_add_u(const DevGrid& g, double* U, double d, bool bc, hipStream_t s);
+hipError_t launch_add_u(const DevGrid& g, double* U, double d, hipStream_t s);
+// U(interior) += q0 - sums[0]/sums[1] (launch_massflow's sums) and U's
+// boundary conditions.
+hipError_t launch_hold_flow(const DevGrid& g, double* U, const double* sums, double q0, hipStream_t s);
 // Fused right-hand side and stage update (rk3_fast.hip), to round-off of the
 // reference's operations: reads the stage input U, V, W, writes the updated
 // interiors Un, Vn, Wn (a different set of fields) and, for stages 1 and 2,
@@ -163,11 +165,11 @@ hipError_t launch_rhs_stage(const DevGrid& g, int stage, const RkStage& a, hipSt
 // (red3 zeroed by the caller).
 hipError_t launch_dt_max(const DevGrid& g, const double* U, const double* V, const double* W,
                          unsigned long long* red3, hipStream_t s);
-// Bulk-flow integral and norm of U into out2[0..1]; part holds
-// 2*massflow_rows(g) doubles.
-int massflow_rows(const DevGrid& g);
+// Bulk-flow integral and norm of U into out2[0..1] and host2[0..1] (host
+// memory that the device writes); part holds 2*massflow_parts(g) doubles.
+int massflow_parts(const DevGrid& g);
 hipError_t launch_massflow(const DevGrid& g, const double* U, const double* H, double* part,
-                           double* out2, hipStream_t s);
+                           double* out2, double* host2, hipStream_t s);
 // output_monitor field summaries: out7 = sums of U, V, W over their
 // interiors, maxima of the same, and the count of non-finite entries; part
 // holds monitor_part_size() doubles of scratch.

@@ -108,9 +108,7 @@ __global__ __launch_bounds__(kB) void k_rk_update(int n1, int n2, int i1, int j1
   (void)k1;
 }
 
-// U(2:nx-1, 2:nyg-1, 2:nzg-1) += d  (src/time_integration.f90:190); BC: the
-// unique cells, each with its boundary images.
-template <bool BC>
+// U(2:nx-1, 2:nyg-1, 2:nzg-1) += d  (src/time_integration.f90:190).
 __global__ __launch_bounds__(kB) void k_add_u(DevGrid g, double* __restrict__ U, double d) {
   unsigned bx, by, bz;
   xcd_tile(bx, by, bz);  // neighbouring tiles on one XCD (shared halo rows)
@@ -119,9 +117,23 @@ __global__ __launch_bounds__(kB) void k_add_u(DevGrid g, double* __restrict__ U,
   const int k = bz + 2;
   if (i > g.nx - 1 || j > g.nyg - 1) return;
   const size_t o = fidx(i, j, k, g.nx, g.nyg);
-  const double u = U[o] + d;
-  if constexpr (BC) put_u(g, U, i, j, k, u);
-  else U[o] = u;
+  U[o] = U[o] + d;
+}
+
+// The constant-flow correction (src/time_integration.f90:187-190) with U's
+// boundary conditions: d = q0 - sums[0]/sums[1] from the flow integral on the
+// device (no wait for the host in the middle of a step), added to the unique
+// cells, each stored with its boundary images.
+__global__ __launch_bounds__(kB) void k_hold_flow(DevGrid g, double* __restrict__ U,
+                                                  const double* __restrict__ sums, double q0) {
+  unsigned bx, by, bz;
+  xcd_tile(bx, by, bz);
+  const int i = bx * 64 + (threadIdx.x & 63) + 2;
+  const int j = __builtin_amdgcn_readfirstlane((int)(by * 4 + (threadIdx.x >> 6) + 2));
+  const int k = bz + 2;
+  if (i > g.nx - 1 || j > g.nyg - 1) return;
+  const double d = q0 - sums[0] / sums[1];
+  put_u(g, U, i, j, k, U[fidx(i, j, k, g.nx, g.nyg)] + d);
 }
 
 // compute_dt maxima (src/time_integration.f90:228-239): max over the
@@ -154,40 +166,80 @@ __global__ __launch_bounds__(kB) void k_dt_max(DevGrid g, const double* __restri
   }
 }
 
-// Bulk-flow partial sums (src/mass_flow.f90:36-44) per (j,k) row, summed
-// over i in order: part[2*r] = sum of (H U + H U)*dy/2, part[2*r+1] = norm.
-__global__ __launch_bounds__(kB) void k_massflow_rows(DevGrid g, const double* __restrict__ U,
-                                                      const double* __restrict__ H,
-                                                      double* __restrict__ part) {
+// Bulk-flow integral (src/mass_flow.f90:36-44): sums of (H U + H U(j-1))*dy/2
+// and of its norm over i = 2..nx-1, j = 3..nyg-1, k = 2..nzg-1.  One wavefront
+// per 64 x positions, z plane and chunk of kFlowJ rows, each row's loads in
+// flight together and row j-1 reused: U is read once, in whole rows.  The
+// chunks keep short channels from running on a few wavefronts.  Per
+// workgroup one pair of partials, added in a fixed order.
+constexpr int kFlowJ = 16;
+template <bool MASK>
+__global__ __launch_bounds__(kB) void k_massflow(DevGrid g, const double* __restrict__ U,
+                                                 const double* __restrict__ H, int ni, int nj,
+                                                 double* __restrict__ part) {
 #pragma clang fp contract(off)
-  const int r = blockIdx.x * kB + threadIdx.x;  // row index over (j = 3..nyg-1, k = 2..nzg-1)
-  const int nj = g.nyg - 3, nk = g.nzg - 2;
-  if (r >= nj * nk) return;
-  const int j = r % nj + 3, k = r / nj + 2;
+  __shared__ double ss[kB / 64], sn[kB / 64];
+  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+  const int w = __builtin_amdgcn_readfirstlane((int)(blockIdx.x * (kB / 64)) + wv);
+  const int i = (w % ni) * 64 + lane + 2;
+  const int jc = (w / ni) % nj, k = w / (ni * nj) + 2;
   double s = 0.0, n = 0.0;
-  for (int i = 2; i <= g.nx - 1; i++) {
-    const double h1 = H ? H[fidx(i, j, k, g.nx, g.nyg)] : 1.0;
-    const double h0 = H ? H[fidx(i, j - 1, k, g.nx, g.nyg)] : 1.0;
-    s = s + (h1 * U_(i, j, k) + h0 * U_(i, j - 1, k)) * 0.5 * g.dyg[j - 1];
-    n = n + (h1 + h0) * 0.5 * g.dyg[j - 1];
+  if (k <= g.nzg - 1 && i <= g.nx - 1) {
+    const int j0 = 3 + jc * kFlowJ;
+    const size_t row = g.nx;
+    const double* u = U + fidx(i, j0 - 1, k, g.nx, g.nyg);
+    const double* h = MASK ? H + fidx(i, j0 - 1, k, g.nx, g.nyg) : nullptr;
+    double um[kFlowJ + 1], hm[kFlowJ + 1];
+#pragma unroll
+    for (int r = 0; r <= kFlowJ; r++) {
+      const int rr = min(r, g.nyg - j0);  // rows j0-1 .. nyg-1
+      um[r] = u[rr * row];
+      hm[r] = MASK ? h[rr * row] : 1.0;
+    }
+#pragma unroll
+    for (int r = 1; r <= kFlowJ; r++) {
+      const int j = j0 + r - 1;
+      if (j <= g.nyg - 1) {
+        s = s + (hm[r] * um[r] + hm[r - 1] * um[r - 1]) * 0.5 * g.dyg[j - 1];
+        n = n + (hm[r] + hm[r - 1]) * 0.5 * g.dyg[j - 1];
+      }
+    }
   }
-  part[2 * (size_t)r] = s;
-  part[2 * (size_t)r + 1] = n;
+  for (int off = 32; off > 0; off >>= 1) {
+    s += __shfl_xor(s, off, 64);
+    n += __shfl_xor(n, off, 64);
+  }
+  if (lane == 0) {
+    ss[wv] = s;
+    sn[wv] = n;
+  }
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    for (int q = 1; q < kB / 64; q++) {
+      s += ss[q];
+      n += sn[q];
+    }
+    part[2 * (size_t)blockIdx.x] = s;
+    part[2 * (size_t)blockIdx.x + 1] = n;
+  }
 }
 
-// Ordered sum of the row partials (single workgroup, fixed order).
-__global__ __launch_bounds__(kB) void k_sum_pairs(const double* __restrict__ part, int nrow,
-                                                  double* __restrict__ out) {
-  __shared__ double ss[kB], sn[kB];
+// Ordered sum of the partials (single workgroup, fixed order) into out and
+// host (host memory that the device writes).
+constexpr int kSumB = 1024;
+__global__ __launch_bounds__(kSumB) void k_sum_pairs(const double* __restrict__ part, int nrow,
+                                                     double* __restrict__ out, double* host) {
+  __shared__ double ss[kSumB], sn[kSumB];
   double s = 0.0, n = 0.0;
-  for (int r = threadIdx.x; r < nrow; r += kB) {
+#pragma unroll 4
+  for (int r = threadIdx.x; r < nrow; r += kSumB) {
     s += part[2 * (size_t)r];
     n += part[2 * (size_t)r + 1];
   }
   ss[threadIdx.x] = s;
   sn[threadIdx.x] = n;
   __syncthreads();
-  for (int w = kB / 2; w > 0; w >>= 1) {
+  for (int w = kSumB / 2; w > 0; w >>= 1) {
     if ((int)threadIdx.x < w) {
       ss[threadIdx.x] += ss[threadIdx.x + w];
       sn[threadIdx.x] += sn[threadIdx.x + w];
@@ -195,8 +247,8 @@ __global__ __launch_bounds__(kB) void k_sum_pairs(const double* __restrict__ par
     __syncthreads();
   }
   if (threadIdx.x == 0) {
-    out[0] = ss[0];
-    out[1] = sn[0];
+    out[0] = host[0] = ss[0];
+    out[1] = host[1] = sn[0];
   }
 }
 
@@ -354,10 +406,13 @@ hipError_t launch_rk_update(const DevGrid& g, int which, int stage, double dt, c
   return hipGetLastError();
 }
 
-hipError_t launch_add_u(const DevGrid& g, double* U, double d, bool bc, hipStream_t s) {
-  const dim3 grid = gpts(g.nx - 2, g.nyg - 2, (bc ? g.nz : g.nzg) - 2);
-  if (bc) hipLaunchKernelGGL(k_add_u<true>, grid, dim3(kB), 0, s, g, U, d);
-  else hipLaunchKernelGGL(k_add_u<false>, grid, dim3(kB), 0, s, g, U, d);
+hipError_t launch_add_u(const DevGrid& g, double* U, double d, hipStream_t s) {
+  hipLaunchKernelGGL(k_add_u, gpts(g.nx - 2, g.nyg - 2, g.nzg - 2), dim3(kB), 0, s, g, U, d);
+  return hipGetLastError();
+}
+
+hipError_t launch_hold_flow(const DevGrid& g, double* U, const double* sums, double q0, hipStream_t s) {
+  hipLaunchKernelGGL(k_hold_flow, gpts(g.nx - 2, g.nyg - 2, g.nz - 2), dim3(kB), 0, s, g, U, sums, q0);
   return hipGetLastError();
 }
 
@@ -368,7 +423,12 @@ hipError_t launch_dt_max(const DevGrid& g, const double* U, const double* V, con
   return hipGetLastError();
 }
 
-int massflow_rows(const DevGrid& g) { return (g.nyg - 3) * (g.nzg - 2); }
+// Wavefronts of the flow integral: x tiles, row chunks, z planes.
+static int flow_ni(const DevGrid& g) { return (g.nx - 2 + 63) / 64; }
+static int flow_nj(const DevGrid& g) { return (g.nyg - 3 + kFlowJ - 1) / kFlowJ; }
+int massflow_parts(const DevGrid& g) {
+  return (flow_ni(g) * flow_nj(g) * (g.nzg - 2) + kB / 64 - 1) / (kB / 64);
+}
 
 int monitor_part_size() { return kMonBlocks * kMon; }
 static_assert(kMonBlocks * kMon == kMonitorPartDoubles, "partials of the monitor kernels");
@@ -408,10 +468,11 @@ hipError_t launch_plane_sums(const DevGrid& g, const double* U, const double* V,
 }
 
 hipError_t launch_massflow(const DevGrid& g, const double* U, const double* H, double* part,
-                           double* out2, hipStream_t s) {
-  const int nrow = massflow_rows(g);
-  hipLaunchKernelGGL(k_massflow_rows, dim3((nrow + kB - 1) / kB), dim3(kB), 0, s, g, U, H, part);
-  hipLaunchKernelGGL(k_sum_pairs, dim3(1), dim3(kB), 0, s, part, nrow, out2);
+                           double* out2, double* host2, hipStream_t s) {
+  const int n = massflow_parts(g), ni = flow_ni(g), nj = flow_nj(g);
+  if (H) hipLaunchKernelGGL(k_massflow<true>, dim3(n), dim3(kB), 0, s, g, U, H, ni, nj, part);
+  else hipLaunchKernelGGL(k_massflow<false>, dim3(n), dim3(kB), 0, s, g, U, H, ni, nj, part);
+  hipLaunchKernelGGL(k_sum_pairs, dim3(1), dim3(kSumB), 0, s, part, n, out2, host2);
   return hipGetLastError();
 }
 
