@@ -135,6 +135,17 @@ __global__ void k_setup(DevGrid g, SetupGrid sg, Markers m, int* bad) {
   }
 }
 
+__global__ void k_mark_planes(Markers m, int* live) {
+  const int tid = blockIdx.x * blockDim.x + threadIdx.x;
+  const int nb = m.nb;
+  if (tid >= 20 * nb) return;
+  const int s = tid / (5 * nb), e = tid - s * 5 * nb;  // e = t*nb + l
+  const int jj = m.st[s].idx[5 * nb + e] - 2;
+  // every writer stores the same value; a set plane is not stored again
+  if (!live[jj]) live[jj] = 1;
+  if (s == 1 && !live[jj + 1]) live[jj + 1] = 1;
+}
+
 // Wall height of marker i (1-based, x-periodic) of one wall at the time wt
 // (src/immersed_boundary_geometry.f90:186-191 standing, :295-299 traveling),
 // and x itself.  The standing wave's top wall returns the bottom wall's
@@ -888,6 +899,11 @@ inline dim3 wave_blocks(int nb) { return dim3((unsigned)((nb + kBlock / 64 - 1) 
 hipError_t launch_setup(const DevGrid& g, const SetupGrid& sg, const Markers& m, int* bad,
                         hipStream_t s) {
   hipLaunchKernelGGL(k_setup, blocks_for((size_t)4 * m.nb), dim3(kBlock), 0, s, g, sg, m, bad);
+  return hipGetLastError();
+}
+
+hipError_t launch_mark_planes(const Markers& m, int* live, hipStream_t s) {
+  hipLaunchKernelGGL(k_mark_planes, blocks_for((size_t)20 * m.nb), dim3(kBlock), 0, s, m, live);
   return hipGetLastError();
 }
 

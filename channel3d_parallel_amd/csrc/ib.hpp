@@ -61,6 +61,13 @@ struct SetupGrid {
 hipError_t launch_setup(const DevGrid& g, const SetupGrid& sg, const Markers& m, int* bad,
                         hipStream_t s);
 
+// live[jj] = 1 for the planes jj = j - 2 that a Schur product's Poisson solve
+// needs: those where the divergence of the spread forces can be non-zero,
+// which are also those whose potential the Schur rows read (cells Y of the u,
+// w and centre nodes, Y and Y + 1 of the v nodes).  live[nym]: zeroed by the
+// caller.
+hipError_t launch_mark_planes(const Markers& m, int* live, hipStream_t s);
+
 // Moving wall bodies of setup_IB_geometry (src/immersed_boundary_geometry.f90:
 // 176-390).  Markers k = i + 2 nxb (j-1) (bottom wall) and k + nxb (top wall),
 // i = 1..nxb, j = 1..nzb.  Scalars that depend on t alone are evaluated on the

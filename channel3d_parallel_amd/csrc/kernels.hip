@@ -64,7 +64,8 @@ __global__ __launch_bounds__(kBlock) void k_fwd_x(DevGrid g, const double* __res
                                                   cpx<real>* __restrict__ S,
                                                   double* __restrict__ bout,
                                                   const double* __restrict__ gauge,
-                                                  unsigned long long* __restrict__ rmax, int per) {
+                                                  unsigned long long* __restrict__ rmax, int per,
+                                                  const int* __restrict__ planes) {
   constexpr bool FROM_UVW = (SRC == kSrcUVW || SRC == kSrcUVWB || SRC == kSrcUVWc);
   constexpr bool RESID = (SRC == kSrcResid);
   constexpr bool NTL = (SRC != kSrcUVWc);  // non-temporal U and W loads
@@ -79,8 +80,8 @@ __global__ __launch_bounds__(kBlock) void k_fwd_x(DevGrid g, const double* __res
 
   const int tid = threadIdx.x;
   const int k0 = blockIdx.x * TK;
-  const int jj = blockIdx.y;
-  const int j = jj + 2;
+  const int js = blockIdx.y;  // the plane's place in the spectrum
+  const int j = (planes ? planes[js] : js) + 2;
   const int nx = g.nx, ny = g.ny, nxg = g.nxg, nyg = g.nyg;
 
   // 1) rows -> LDS.  Rows are walked with uniform (scalar) row bases; each
@@ -297,7 +298,7 @@ __global__ __launch_bounds__(kBlock) void k_fwd_x(DevGrid g, const double* __res
     const int kx = e / TK, t = e % TK;
     // streaming store: the spectrum is next read by another kernel
     const cpx<real> v = buf[kx * TKP + t];
-    cpx<real>* d = &S[((size_t)jj * NH + kx) * nzp + k0 + t];
+    cpx<real>* d = &S[((size_t)js * NH + kx) * nzp + k0 + t];
     __builtin_nontemporal_store(v.x, &d->x);
     __builtin_nontemporal_store(v.y, &d->y);
   }
@@ -379,7 +380,8 @@ __global__ __launch_bounds__(kBlock) void k_inv_x(DevGrid g, const cpx<real>* __
                                                   const cpx<real>* __restrict__ tw,
                                                   double* out, double* __restrict__ P,
                                                   double dt, int rk1, const double* phi_in,
-                                                  const double* phi_in2, double* out2) {
+                                                  const double* phi_in2, double* out2,
+                                                  const int* __restrict__ planes) {
   constexpr int NP = TK / 2;
   constexpr int NT = kBlock / NP;
   constexpr int NH = N / 2 + 1;
@@ -390,8 +392,8 @@ __global__ __launch_bounds__(kBlock) void k_inv_x(DevGrid g, const cpx<real>* __
 
   const int tid = threadIdx.x;
   const int k0 = blockIdx.x * TK;
-  const int jj = blockIdx.y;
-  const int j = jj + 2;
+  const int js = blockIdx.y;  // the plane's place in the spectrum
+  const int j = (planes ? planes[js] : js) + 2;
   const int nzp = g.nzp, nxg = g.nxg, nyg = g.nyg;
 
   {
@@ -404,7 +406,7 @@ __global__ __launch_bounds__(kBlock) void k_inv_x(DevGrid g, const cpx<real>* __
       vy[q] = (real)0;
       if (e < NH * TK) {
         const int kx = e / TK, t = e % TK;
-        const cpx<real>* sp = &S[((size_t)jj * NH + kx) * nzp + k0 + t];
+        const cpx<real>* sp = &S[((size_t)js * NH + kx) * nzp + k0 + t];
         cpx<real> v;
         v.x = __builtin_nontemporal_load(&sp->x);  // read once
         v.y = __builtin_nontemporal_load(&sp->y);
@@ -464,8 +466,8 @@ __global__ __launch_bounds__(kBlock) void k_inv_x(DevGrid g, const cpx<real>* __
   // of them repeat an interior value, so they need no pass of their own.
   auto store_p = [&](int n, int k, double v, bool dupz) {
     for (int b = 0; b < 2; b++) {
-      if (b == 1 && jj != 0 && j != nyg - 1) break;
-      const int jb = b == 0 ? j : (jj == 0 ? 1 : nyg);
+      if (b == 1 && j != 2 && j != nyg - 1) break;
+      const int jb = b == 0 ? j : (j == 2 ? 1 : nyg);
       for (int c = 0; c < (dupz ? 4 : 1); c++) {
         const int kc = c == 0 ? k : (c == 1 ? nzp + 2 : (c == 2 ? 1 : g.nzg));
         double* row = P + fidx(2, jb, kc, nxg, nyg);
@@ -882,9 +884,11 @@ inline dim3 grid_pts(const DevGrid& g, int ni, int nj, int nk) {
 }  // namespace
 
 hipError_t launch_fwd_x(const DevGrid& g, bool from_uvw, const double* U, const double* V,
-                        const double* W, const double* rhs, cpx<double>* S, bool per, hipStream_t s) {
+                        const double* W, const double* rhs, cpx<double>* S, bool per, hipStream_t s,
+                        const Planes* pl) {
   const int tk = tile_rows(g.nxp, g.nzp);
-  dim3 grid(g.nzp / tk, g.nym);
+  dim3 grid(g.nzp / tk, pl ? pl->n : g.nym);
+  const int* list = pl ? pl->list : nullptr;
   // U, V, W together below 128 MB stay in the 256 MB last-level cache
   // between the kernel that wrote them and this one: cached loads there
   // (measured 13.2 against 15.6 us at 128^3), non-temporal loads above.
@@ -892,13 +896,13 @@ hipError_t launch_fwd_x(const DevGrid& g, bool from_uvw, const double* U, const 
   C3D_DISPATCH_N(g.nxp, C3D_DISPATCH_TK(tk, {
     if (from_uvw && small)
       hipLaunchKernelGGL((k_fwd_x<double, NN, TK, kSrcUVWc>), grid, dim3(kBlock), 0, s, g, U, V, W,
-                         (const void*)rhs, g.twx64, S, nullptr, nullptr, nullptr, per ? 1 : 0);
+                         (const void*)rhs, g.twx64, S, nullptr, nullptr, nullptr, per ? 1 : 0, list);
     else if (from_uvw)
       hipLaunchKernelGGL((k_fwd_x<double, NN, TK, kSrcUVW>), grid, dim3(kBlock), 0, s, g, U, V, W,
-                         (const void*)rhs, g.twx64, S, nullptr, nullptr, nullptr, per ? 1 : 0);
+                         (const void*)rhs, g.twx64, S, nullptr, nullptr, nullptr, per ? 1 : 0, list);
     else
       hipLaunchKernelGGL((k_fwd_x<double, NN, TK, kSrcRhs>), grid, dim3(kBlock), 0, s, g, U, V, W,
-                         (const void*)rhs, g.twx64, S, nullptr, nullptr, nullptr, per ? 1 : 0);
+                         (const void*)rhs, g.twx64, S, nullptr, nullptr, nullptr, per ? 1 : 0, list);
   }));
   return hipGetLastError();
 }
@@ -911,10 +915,12 @@ hipError_t launch_fwd_x32(const DevGrid& g, const double* U, const double* V, co
   C3D_DISPATCH_N(g.nxp, C3D_DISPATCH_TK(tk, {
     if (b)
       hipLaunchKernelGGL((k_fwd_x<float, NN, TK, kSrcUVWB>), grid, dim3(kBlock), 0, s, g, U, V, W,
-                         (const void*)nullptr, g.twx32, S, b, nullptr, nullptr, per ? 1 : 0);
+                         (const void*)nullptr, g.twx32, S, b, nullptr, nullptr, per ? 1 : 0,
+                         nullptr);
     else
       hipLaunchKernelGGL((k_fwd_x<float, NN, TK, kSrcUVW>), grid, dim3(kBlock), 0, s, g, U, V, W,
-                         (const void*)nullptr, g.twx32, S, nullptr, nullptr, nullptr, per ? 1 : 0);
+                         (const void*)nullptr, g.twx32, S, nullptr, nullptr, nullptr, per ? 1 : 0,
+                         nullptr);
   }));
   return hipGetLastError();
 }
@@ -931,7 +937,8 @@ hipError_t fwd_x_resid(const DevGrid& g, const double* b, const double* phi, dou
   hipLaunchKernelGGL(k_gauge_final, dim3(1), dim3(kBlock), 0, s, g, (const double*)(gauge + 1), gauge);
   C3D_DISPATCH_N(g.nxp, C3D_DISPATCH_TK(tk, {
     hipLaunchKernelGGL((k_fwd_x<real, NN, TK, kSrcResid>), grid, dim3(kBlock), 0, s, g, phi,
-                       nullptr, nullptr, (const void*)b, tw, S, rout, (const double*)gauge, rmax, 0);
+                       nullptr, nullptr, (const void*)b, tw, S, rout, (const double*)gauge, rmax, 0,
+                       nullptr);
   }));
   return hipGetLastError();
 }
@@ -954,7 +961,8 @@ hipError_t launch_fwd_x_b64(const DevGrid& g, const double* U, const double* V, 
   dim3 grid(g.nzp / tk, g.nym);
   C3D_DISPATCH_N(g.nxp, C3D_DISPATCH_TK(tk, {
     hipLaunchKernelGGL((k_fwd_x<double, NN, TK, kSrcUVWB>), grid, dim3(kBlock), 0, s, g, U, V, W,
-                       (const void*)nullptr, g.twx64, S, b, nullptr, nullptr, per ? 1 : 0);
+                       (const void*)nullptr, g.twx64, S, b, nullptr, nullptr, per ? 1 : 0,
+                       nullptr);
   }));
   return hipGetLastError();
 }
@@ -973,8 +981,8 @@ static int fft_z_nt32() {
 
 template <typename real>
 static hipError_t fft_z_any(const DevGrid& g, int sign, cpx<real>* S, const cpx<real>* tw,
-                            hipStream_t s) {
-  const int ncol = g.nym * g.nxh;
+                            hipStream_t s, const Planes* pl) {
+  const int ncol = (pl ? pl->n : g.nym) * g.nxh;
   const int nt = (sizeof(real) == 4) ? fft_z_nt32() : 64;
   const int nc = kBlock / nt;
   dim3 grid((ncol + nc - 1) / nc);
@@ -991,33 +999,27 @@ static hipError_t fft_z_any(const DevGrid& g, int sign, cpx<real>* S, const cpx<
   return hipGetLastError();
 }
 
-hipError_t launch_fft_z(const DevGrid& g, int sign, cpx<double>* S, hipStream_t s) {
-  return fft_z_any<double>(g, sign, S, g.twz64, s);
+hipError_t launch_fft_z(const DevGrid& g, int sign, cpx<double>* S, hipStream_t s, const Planes* pl) {
+  return fft_z_any<double>(g, sign, S, g.twz64, s, pl);
 }
 hipError_t launch_fft_z32(const DevGrid& g, int sign, cpx<float>* S, hipStream_t s) {
-  return fft_z_any<float>(g, sign, S, g.twz32, s);
-}
-
-hipError_t launch_inv_x(const DevGrid& g, int mode, const cpx<double>* S, double* out, double* P,
-                        double dt, bool rk1, hipStream_t s) {
-  if (mode != 0 && mode != 1) return hipErrorInvalidValue;
-  return launch_inv_x64_ref(g, mode, S, nullptr, nullptr, out, nullptr, P, dt, rk1, s);
+  return fft_z_any<float>(g, sign, S, g.twz32, s, nullptr);
 }
 
 namespace {
 #define C3D_INV_CASE(MD)                                                                          \
   case MD:                                                                                        \
     hipLaunchKernelGGL((k_inv_x<real, NN, TK, MD>), grid, dim3(kBlock), 0, s, g, S, tw, out, P, dt, \
-                       rk1 ? 1 : 0, phi_in, phi_in2, out2);                                       \
+                       rk1 ? 1 : 0, phi_in, phi_in2, out2, pl ? pl->list : nullptr);              \
     break;
 template <typename real>
 hipError_t inv_x_modes(const DevGrid& g, int mode, const cpx<real>* S, const cpx<real>* tw,
                        const double* phi_in, const double* phi_in2, double* out, double* out2,
-                       double* P, double dt, bool rk1, hipStream_t s) {
+                       double* P, double dt, bool rk1, hipStream_t s, const Planes* pl = nullptr) {
   if ((mode == 3 && !phi_in) || (mode == 5 && (!out2 || (rk1 && !phi_in))))
     return hipErrorInvalidValue;
   const int tk = tile_rows(g.nxp, g.nzp);
-  dim3 grid(g.nzp / tk, g.nym);
+  dim3 grid(g.nzp / tk, pl ? pl->n : g.nym);
   C3D_DISPATCH_N(g.nxp, C3D_DISPATCH_TK(tk, {
     switch (mode) {
       C3D_INV_CASE(0)
@@ -1031,6 +1033,12 @@ hipError_t inv_x_modes(const DevGrid& g, int mode, const cpx<real>* S, const cpx
 }
 #undef C3D_INV_CASE
 }  // namespace
+
+hipError_t launch_inv_x(const DevGrid& g, int mode, const cpx<double>* S, double* out, double* P,
+                        double dt, bool rk1, hipStream_t s, const Planes* pl) {
+  if (mode != 0 && mode != 1) return hipErrorInvalidValue;
+  return inv_x_modes<double>(g, mode, S, g.twx64, nullptr, nullptr, out, nullptr, P, dt, rk1, s, pl);
+}
 
 hipError_t launch_inv_x64_ref(const DevGrid& g, int mode, const cpx<double>* S, const double* phi_in,
                               const double* phi_in2, double* out, double* out2, double* P, double dt,

@@ -51,25 +51,42 @@ __host__ __device__ __forceinline__ size_t ridx(int i, int j, int k, int nxg, in
   return (size_t)(i - 2) + (size_t)(nxg - 2) * ((size_t)(j - 2) + (size_t)(nyg - 2) * (size_t)(k - 2));
 }
 
+// The y planes (jj = j - 2, ascending) that a Poisson solve transforms when the
+// right-hand side is zero on all others and its solution is read on these
+// alone: the spectrum then holds just these planes, one after the other.
+// list[n] the planes, slot[nym] a plane's position among them or -1 (device).
+struct Planes {
+  const int* list;
+  const int* slot;
+  int n;
+};
+// Whether the tridiagonal solve takes such a spectrum (the partitioned one does).
+bool planes_supported(const DevGrid& g);
+
 // Forward x transform.  from_uvw: input is div(U,V,W) computed on the fly,
 // else the rhs_p array.  Writes the half spectrum S[j][kx][kz].  per: the
 // divergence takes the boundary values from the interior (the periodic
 // images and V = 0 on the walls) instead of the fields' boundary cells.
 hipError_t launch_fwd_x(const DevGrid& g, bool from_uvw, const double* U, const double* V,
-                        const double* W, const double* rhs, cpx<double>* S, bool per, hipStream_t s);
-hipError_t launch_fft_z(const DevGrid& g, int sign, cpx<double>* S, hipStream_t s);
+                        const double* W, const double* rhs, cpx<double>* S, bool per, hipStream_t s,
+                        const Planes* pl = nullptr);
+hipError_t launch_fft_z(const DevGrid& g, int sign, cpx<double>* S, hipStream_t s,
+                        const Planes* pl = nullptr);
 // Tridiagonal solve along y for every (kx,kz): the partitioned register
 // solver from 33 to 768 rows, else the plain Thomas sweep with CP, nym*nxh*nzp
 // doubles of scratch (may be null unless tri_needs_scratch).
 bool tri_needs_scratch(const DevGrid& g);
 // The row counts of the FP32 solves (launch_tri32, launch_tri32to64).
 bool tri_part_supported(const DevGrid& g);
-hipError_t launch_tri(const DevGrid& g, cpx<double>* S, double* CP, hipStream_t s);
+// pl (planes_supported): S holds the planes of pl, the other right-hand sides
+// are zero and their solutions are not stored.
+hipError_t launch_tri(const DevGrid& g, cpx<double>* S, double* CP, hipStream_t s,
+                      const Planes* pl = nullptr);
 // Inverse x transform.  mode 0: out = solution rhs_p (Poisson drop-in).
 // mode 1: out = P_interim = solution/dt (projection).  rk1: also write P,
 // ghosts included.
 hipError_t launch_inv_x(const DevGrid& g, int mode, const cpx<double>* S, double* out, double* P,
-                        double dt, bool rk1, hipStream_t s);
+                        double dt, bool rk1, hipStream_t s, const Planes* pl = nullptr);
 // Refinement pieces (mixed precision: FP32 forward spectra; FP64: the same
 // sweeps on FP64 spectra).  launch_fwd_x32: divergence of U, V, W (FP64,
 // also stored to b when b != null) -> FP32 spectrum.

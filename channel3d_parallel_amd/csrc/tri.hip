@@ -103,11 +103,14 @@ constexpr int kTriList = 2;  // the modes list[0 .. nlist)
 // P*M rows hold g.nym <= P*M of the system and identity rows after them
 // (x = 0, no coupling), which leave the other rows as they are: the last
 // part may be short and parts after it empty.
+// PLANES: S holds the planes of `Planes` only (slot[row], or -1: the row's
+// right-hand side is zero and its solution is not stored).
 template <typename real, typename acc, int M, int SEL, typename rout = real, int P = 8, int MWX = 0,
-          bool PAD = false>
+          bool PAD = false, bool PLANES = false>
 __global__ __launch_bounds__(kBlock) void k_tri_part(DevGrid g, cpx<real>* S,
                                                      const int* __restrict__ list, int nlist,
-                                                     double lam_thr, cpx<rout>* Sout) {
+                                                     double lam_thr, cpx<rout>* Sout,
+                                                     const int* __restrict__ slot) {
   constexpr int N = P * M;        // rows
   // modes per wave: a row access of a wave is MW consecutive modes, 256
   // contiguous bytes of the input spectrum (16 FP64 or 32 FP32 complex)
@@ -155,8 +158,16 @@ __global__ __launch_bounds__(kBlock) void k_tri_part(DevGrid g, cpx<real>* S,
   const acc lam = (acc)(g.kxx[kx] + g.kzz[kz]);
   const bool zero_first = (kx == 0 && kz == 0 && p == 0);
   const int row0 = p * M;
-  cpx<real>* s = S + mv + (PAD ? 0 : (size_t)row0 * stride);
-  cpx<rout>* so = Sout + mv + (size_t)row0 * stride;
+  cpx<real>* s = S + mv + (PAD || PLANES ? 0 : (size_t)row0 * stride);
+  cpx<rout>* so = Sout + mv + (PLANES ? 0 : (size_t)row0 * stride);
+  int sl[PLANES ? M : 1];
+  if constexpr (PLANES) {
+#pragma unroll
+    for (int r = 0; r < M; r++) {
+      const int v = slot[PAD ? min(row0 + r, nrow - 1) : row0 + r];
+      sl[r] = (PAD && row0 + r >= nrow) ? -1 : v;
+    }
+  }
 
   // All M rows are loaded unconditionally and converted afterwards: mv is a
   // valid mode for every lane, so the addresses stay in bounds, and without
@@ -166,10 +177,15 @@ __global__ __launch_bounds__(kBlock) void k_tri_part(DevGrid g, cpx<real>* S,
   {
     cpx<real> t[M];
 #pragma unroll
-    for (int r = 0; r < M; r++) t[r] = s[(size_t)(PAD ? min(row0 + r, nrow - 1) : r) * stride];
+    for (int r = 0; r < M; r++) {
+      // a row without a plane reads the first plane and does not use it
+      if constexpr (PLANES) t[r] = s[(size_t)max(sl[r], 0) * stride];
+      else t[r] = s[(size_t)(PAD ? min(row0 + r, nrow - 1) : r) * stride];
+    }
 #pragma unroll
     for (int r = 0; r < M; r++) {
-      const bool in = valid && (!PAD || row0 + r < nrow);
+      bool in = valid && (!PAD || row0 + r < nrow);
+      if constexpr (PLANES) in = valid && sl[r] >= 0;
       yr[r] = in ? -(acc)t[r].x : (acc)0;
       yi[r] = in ? -(acc)t[r].y : (acc)0;
     }
@@ -273,7 +289,11 @@ __global__ __launch_bounds__(kBlock) void k_tri_part(DevGrid g, cpx<real>* S,
   for (int r = M - 1; r >= 0; r--) {
     const acc xr = (yr[r] + sp[r] * xar) + cp[r] * xnr;
     const acc xi = (yi[r] + sp[r] * xai) + cp[r] * xni;
-    if (valid && (!PAD || row0 + r < nrow)) so[(size_t)r * stride] = cmk((rout)xr, (rout)xi);
+    if constexpr (PLANES) {
+      if (valid && sl[r] >= 0) so[(size_t)sl[r] * stride] = cmk((rout)xr, (rout)xi);
+    } else if (valid && (!PAD || row0 + r < nrow)) {
+      so[(size_t)r * stride] = cmk((rout)xr, (rout)xi);
+    }
     xnr = xr;
     xni = xi;
   }
@@ -294,11 +314,16 @@ __global__ __launch_bounds__(kBlock) void k_tri_part(DevGrid g, cpx<real>* S,
 namespace {
 // FP64 solve of every mode in P parts of MM rows, MW modes per wave.
 template <int P, int MM, int MW, bool PAD>
-void tri64_parts(const DevGrid& g, cpx<double>* S, hipStream_t s) {
+void tri64_parts(const DevGrid& g, cpx<double>* S, hipStream_t s, const Planes* pl) {
   constexpr int MB = kBlock / P;
   const size_t nm = (size_t)g.nxh * g.nzp;
-  hipLaunchKernelGGL((k_tri_part<double, double, MM, kTriAll, double, P, MW, PAD>),
-                     dim3((unsigned)((nm + MB - 1) / MB)), dim3(kBlock), 0, s, g, S, nullptr, 0, 0.0, S);
+  const dim3 grid((unsigned)((nm + MB - 1) / MB));
+  if (pl)
+    hipLaunchKernelGGL((k_tri_part<double, double, MM, kTriAll, double, P, MW, PAD, true>), grid,
+                       dim3(kBlock), 0, s, g, S, nullptr, 0, 0.0, S, pl->slot);
+  else
+    hipLaunchKernelGGL((k_tri_part<double, double, MM, kTriAll, double, P, MW, PAD>), grid,
+                       dim3(kBlock), 0, s, g, S, nullptr, 0, 0.0, S, nullptr);
 }
 // Row counts of the plain elimination, one lane per mode: above what the
 // lanes of a workgroup hold in registers, and up to 32 rows, where the number
@@ -310,14 +335,17 @@ constexpr int kTriMinRows = 33, kTriMaxRows = 32 * 24;
 
 bool tri_needs_scratch(const DevGrid& g) { return g.nym < kTriMinRows || g.nym > kTriMaxRows; }
 
-hipError_t launch_tri(const DevGrid& g, cpx<double>* S, double* CP, hipStream_t s) {
+bool planes_supported(const DevGrid& g) { return !tri_needs_scratch(g); }
+
+hipError_t launch_tri(const DevGrid& g, cpx<double>* S, double* CP, hipStream_t s, const Planes* pl) {
+  if (pl && (pl->n < 1 || !planes_supported(g))) return hipErrorInvalidValue;
   const size_t nm = (size_t)g.nxh * g.nzp;
   // 64, 128 and 192 rows fill 8 parts exactly.
   if (g.nym % 64 == 0 && g.nym <= 192) {
     switch (g.nym) {
-      case 64: tri64_parts<8, 8, 16, false>(g, S, s); break;
-      case 128: tri64_parts<8, 16, 16, false>(g, S, s); break;
-      default: tri64_parts<8, 24, 16, false>(g, S, s); break;
+      case 64: tri64_parts<8, 8, 16, false>(g, S, s, pl); break;
+      case 128: tri64_parts<8, 16, 16, false>(g, S, s, pl); break;
+      default: tri64_parts<8, 24, 16, false>(g, S, s, pl); break;
     }
     return hipGetLastError();
   }
@@ -330,18 +358,18 @@ hipError_t launch_tri(const DevGrid& g, cpx<double>* S, double* CP, hipStream_t 
   // modes: 6.6 us, one lane per mode 72 us; 96 rows of 65 x 128 modes: 10.3
   // against 68 us.
   const int per = (g.nym + 15) / 16;
-  if (per <= 4) tri64_parts<16, 4, 16, true>(g, S, s);
-  else if (per <= 5) tri64_parts<16, 5, 16, true>(g, S, s);
-  else if (per <= 6) tri64_parts<16, 6, 16, true>(g, S, s);
-  else if (per <= 7) tri64_parts<16, 7, 16, true>(g, S, s);
-  else if (per <= 8) tri64_parts<16, 8, 16, true>(g, S, s);
-  else if (per <= 10) tri64_parts<16, 10, 16, true>(g, S, s);
-  else if (per <= 12) tri64_parts<16, 12, 16, true>(g, S, s);
-  else if (per <= 16) tri64_parts<16, 16, 16, true>(g, S, s);
-  else if (per <= 20) tri64_parts<16, 20, 16, true>(g, S, s);
-  else if (per <= 24) tri64_parts<16, 24, 16, true>(g, S, s);
-  else if (per <= 32) tri64_parts<32, 16, 8, true>(g, S, s);
-  else tri64_parts<32, 24, 8, true>(g, S, s);
+  if (per <= 4) tri64_parts<16, 4, 16, true>(g, S, s, pl);
+  else if (per <= 5) tri64_parts<16, 5, 16, true>(g, S, s, pl);
+  else if (per <= 6) tri64_parts<16, 6, 16, true>(g, S, s, pl);
+  else if (per <= 7) tri64_parts<16, 7, 16, true>(g, S, s, pl);
+  else if (per <= 8) tri64_parts<16, 8, 16, true>(g, S, s, pl);
+  else if (per <= 10) tri64_parts<16, 10, 16, true>(g, S, s, pl);
+  else if (per <= 12) tri64_parts<16, 12, 16, true>(g, S, s, pl);
+  else if (per <= 16) tri64_parts<16, 16, 16, true>(g, S, s, pl);
+  else if (per <= 20) tri64_parts<16, 20, 16, true>(g, S, s, pl);
+  else if (per <= 24) tri64_parts<16, 24, 16, true>(g, S, s, pl);
+  else if (per <= 32) tri64_parts<32, 16, 8, true>(g, S, s, pl);
+  else tri64_parts<32, 24, 8, true>(g, S, s, pl);
   return hipGetLastError();
 }
 
@@ -359,15 +387,15 @@ hipError_t tri32_parts(const DevGrid& g, cpx<float>* S, const int* low, int nlow
   const dim3 grid((unsigned)((nm + MB - 1) / MB));
   if (!low) {  // FP64 arithmetic on every mode
     hipLaunchKernelGGL((k_tri_part<float, double, MM, kTriAll, float, P, MWX>), grid, dim3(kBlock),
-                       0, s, g, S, nullptr, 0, 0.0, S);
+                       0, s, g, S, nullptr, 0, 0.0, S, nullptr);
     return hipGetLastError();
   }
   if (nlow <= 0) return hipErrorInvalidValue;  // the (0,0) mode is always a low mode
   const dim3 gridl((unsigned)((nlow + MB - 1) / MB));
   hipLaunchKernelGGL((k_tri_part<float, float, MM, kTriHigh, float, P, MWX>), grid, dim3(kBlock), 0,
-                     s, g, S, nullptr, 0, lam_thr, S);
+                     s, g, S, nullptr, 0, lam_thr, S, nullptr);
   hipLaunchKernelGGL((k_tri_part<float, double, MM, kTriList, float, P, MWX>), gridl, dim3(kBlock),
-                     0, s, g, S, low, nlow, 0.0, S);
+                     0, s, g, S, low, nlow, 0.0, S, nullptr);
   return hipGetLastError();
 }
 }  // namespace
@@ -392,7 +420,7 @@ hipError_t launch_tri32to64(const DevGrid& g, cpx<float>* S32, cpx<double>* S64,
   constexpr int MB = kBlock / 16;
   const dim3 grid((unsigned)((nm + MB - 1) / MB));
   C3D_DISPATCH_M16(g.nym, hipLaunchKernelGGL((k_tri_part<float, double, MM, kTriAll, double, 16, 16>),
-                                             grid, dim3(kBlock), 0, s, g, S32, nullptr, 0, 0.0, S64));
+                                             grid, dim3(kBlock), 0, s, g, S32, nullptr, 0, 0.0, S64, nullptr));
   return hipGetLastError();
 }
 
