@@ -1408,7 +1408,7 @@ static int ib_schur_launch(c3d_ctx* c, const double* f, double* Sf, double dt, i
   int rc = ib_spread_force(c, f, dt);
   if (!rc) rc = ib_poisson_reg(c, dt, rk_step, true);
   if (rc) return rc;
-  HIPCHK(c, c3d::ib::launch_schur_rows(c->g, ib->m, ib->phi, dt, ib->Ureg, ib->Vreg, ib->Wreg,
+  HIPCHK(c, c3d::ib::launch_schur_rows(c->g, ib->m, ib->sp, ib->phi, dt, ib->Ureg, ib->Vreg, ib->Wreg,
                                        ib->E1nH, f, Sf, c->stream));
   HIPCHK(c, c3d::ib::launch_remove_mean(ib->m, Sf + 3 * nb, ib->E1nHc, f + 3 * nb, ib->mpart, c->stream));
   return 0;
@@ -1708,10 +1708,14 @@ int ib_create(c3d_ctx* c, int nb, int nzb, int nxb, int nxb1) {
     return rc;
   m.xb = ib->xb; m.yb = ib->yb; m.zb = ib->zb; m.normals = ib->normals; m.sb = ib->sb;
   m.ub = ib->ub; m.yref = ib->yref;
-  for (int s = 0; s < 4; s++)
-    if ((rc = dalloc(c, &m.st[s].idx, 15 * (size_t)nb)) || (rc = dalloc(c, &m.st[s].phi, 15 * (size_t)nb)) ||
-        (rc = dalloc(c, &m.st[s].dd, 15 * (size_t)nb)))
-      return rc;
+  const size_t ns = B::kStencils * (size_t)nb;
+  if ((rc = dalloc(c, &m.st[0].idx, ns)) || (rc = dalloc(c, &m.st[0].phi, ns)) ||
+      (rc = dalloc(c, &m.st[0].dd, ns)))
+    return rc;
+  for (int s = 1; s < 4; s++) {
+    const size_t o = s * (size_t)B::kStencil;
+    m.st[s] = {m.st[0].idx + o, m.st[0].phi + o, m.st[0].dd + o};
+  }
   B::SetupGrid& sg = ib->sg;
   if ((rc = upload(c, &sg.x, c->x)) || (rc = upload(c, &sg.y, c->y)) || (rc = upload(c, &sg.z, c->z)))
     return rc;
@@ -1782,13 +1786,10 @@ int ib_operators_host_map(c3d_ctx* c) {
   int rc = 0;
   if (B::launch_setup(c->g, ib->sg, m, nullptr, c->stream) != hipSuccess)
     return fail(c, C3D_EHIP, "IB stencil set-up launch failed");
-  std::vector<int> idx[4];
-  for (int s = 0; s < 4; s++) {
-    idx[s].resize(15 * (size_t)nb);
-    if (hipMemcpyAsync(idx[s].data(), m.st[s].idx, idx[s].size() * 4, hipMemcpyDeviceToHost,
-                       c->stream) != hipSuccess)
-      return fail(c, C3D_EHIP, "stencil copy-back failed");
-  }
+  std::vector<int> idx(B::kStencils * (size_t)nb);
+  if (hipMemcpyAsync(idx.data(), m.st[0].idx, idx.size() * 4, hipMemcpyDeviceToHost, c->stream) !=
+      hipSuccess)
+    return fail(c, C3D_EHIP, "stencil copy-back failed");
   if ((rc = sync(c))) return rc;
   // every node must be a canonical interior node inside the gradient's
   // ranges (the Schur kernels evaluate G at the nodes and skip the boundary
@@ -1798,8 +1799,8 @@ int ib_operators_host_map(c3d_ctx* c) {
   for (int s = 0; s < 4; s++)
     for (int t = 0; t < 5; t++)
       for (int l = 0; l < nb; l++) {
-        const int X = idx[s][(0 * 5 + t) * (size_t)nb + l], Y = idx[s][(1 * 5 + t) * (size_t)nb + l],
-                  Z = idx[s][(2 * 5 + t) * (size_t)nb + l];
+        const int* I = idx.data() + s * B::kStencil;
+        const int X = I[B::sidx(0, t, l)], Y = I[B::sidx(1, t, l)], Z = I[B::sidx(2, t, l)];
         if (X < 2 || X > c->nx - 1 || Z < 2 || Z > c->nz - 1)
           return fail(c, C3D_EINVAL, "stencil %d of marker %d: x/z index out of range", s, l);
         if (Y < 2 || Y > ylim[s])
@@ -1810,13 +1811,13 @@ int ib_operators_host_map(c3d_ctx* c) {
   const int n1[3] = {c->nx, c->nxg, c->nxg}, n2[3] = {c->nyg, c->ny, c->nyg};
   const size_t nf[3] = {c->nu, c->nv, c->nw};
   for (int q = 0; q < 3; q++) {
-    const std::vector<int>& I = idx[q];
+    const int* I = idx.data() + q * B::kStencil;
     std::vector<int> cnt(nf[q] + 1, 0), off((size_t)nb * 125);
     for (int l = 0; l < nb; l++)
       for (int p = 0; p < 125; p++) {
         const int i = p % 5, j = (p / 5) % 5, k = p / 25;
-        const size_t o = c3d::fidx(I[(0 * 5 + i) * (size_t)nb + l], I[(1 * 5 + j) * (size_t)nb + l],
-                                   I[(2 * 5 + k) * (size_t)nb + l], n1[q], n2[q]);
+        const size_t o = c3d::fidx(I[B::sidx(0, i, l)], I[B::sidx(1, j, l)], I[B::sidx(2, k, l)],
+                                   n1[q], n2[q]);
         off[(size_t)l * 125 + p] = (int)o;
         cnt[o + 1]++;
       }
@@ -2124,18 +2125,20 @@ int c3d_ib_get_stencil(c3d_ctx* c, int s, int* xi, int* yi, int* zi, double* w, 
   if (rc) return rc;
   if (s < 0 || s > 3) return fail(c, C3D_EINVAL, "stencil must be 0..3");
   IBState* ib = c->ib;
-  const size_t nb = ib->m.nb, n = 15 * nb;
+  namespace B = c3d::ib;
+  const size_t nb = ib->m.nb, n = B::kStencils * nb;
   std::vector<int> I(n);
   std::vector<double> ph(n), dd(n), nrm(3 * nb);
-  HIPCHK(c, hipMemcpyAsync(I.data(), ib->m.st[s].idx, n * 4, hipMemcpyDeviceToHost, c->stream));
-  HIPCHK(c, hipMemcpyAsync(ph.data(), ib->m.st[s].phi, n * 8, hipMemcpyDeviceToHost, c->stream));
-  HIPCHK(c, hipMemcpyAsync(dd.data(), ib->m.st[s].dd, n * 8, hipMemcpyDeviceToHost, c->stream));
+  HIPCHK(c, hipMemcpyAsync(I.data(), ib->m.st[0].idx, n * 4, hipMemcpyDeviceToHost, c->stream));
+  HIPCHK(c, hipMemcpyAsync(ph.data(), ib->m.st[0].phi, n * 8, hipMemcpyDeviceToHost, c->stream));
+  HIPCHK(c, hipMemcpyAsync(dd.data(), ib->m.st[0].dd, n * 8, hipMemcpyDeviceToHost, c->stream));
   HIPCHK(c, hipMemcpyAsync(nrm.data(), ib->m.normals, 3 * nb * 8, hipMemcpyDeviceToHost, c->stream));
   if ((rc = sync(c))) return rc;
   for (size_t l = 0; l < nb; l++)
     for (int p = 0; p < 125; p++) {
-      const size_t a = (size_t)(p % 5) * nb + l, b = (size_t)(5 + (p / 5) % 5) * nb + l,
-                   d = (size_t)(10 + p / 25) * nb + l, o = l * 125 + p;
+      const size_t q = s * (size_t)B::kStencil, a = q + B::sidx(0, p % 5, (int)l),
+                   b = q + B::sidx(1, (p / 5) % 5, (int)l), d = q + B::sidx(2, p / 25, (int)l),
+                   o = l * 125 + p;
       if (xi) xi[o] = I[a];
       if (yi) yi[o] = I[b];
       if (zi) zi[o] = I[d];

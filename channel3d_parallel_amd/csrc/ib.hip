@@ -53,7 +53,7 @@ __global__ void k_setup(DevGrid g, SetupGrid sg, Markers m, int* bad) {
   const int tid = blockIdx.x * blockDim.x + threadIdx.x;
   const int nb = m.nb;
   if (tid >= 4 * nb) return;
-  const int s = tid / nb, l = tid - s * nb;
+  const int l = tid / 4, s = tid - 4 * l;
   const int nx = g.nx, nz = g.nz, nzg = g.nzg;
   const double dx = sg.dx, dz = sg.dz, dymin = sg.dymin;
   const double xb = m.xb[l], yb = m.yb[l], zb = m.zb[l];
@@ -123,15 +123,15 @@ __global__ void k_setup(DevGrid g, SetupGrid sg, Markers m, int* bad) {
     const double ddx = xgd - xb, ddy = ygd - yb, ddz = zgd - zb;
     if (bad && (X < 2 || X > nx - 1 || Z < 2 || Z > nz - 1 || Y < 2 || Y > ylim))
       atomicMax(bad, l + 1);
-    st.idx[(0 * 5 + t) * nb + l] = X;
-    st.idx[(1 * 5 + t) * nb + l] = Y;
-    st.idx[(2 * 5 + t) * nb + l] = Z;
-    st.dd[(0 * 5 + t) * nb + l] = ddx;
-    st.dd[(1 * 5 + t) * nb + l] = ddy;
-    st.dd[(2 * 5 + t) * nb + l] = ddz;
-    st.phi[(0 * 5 + t) * nb + l] = deltafnc(ddx, dx);
-    st.phi[(1 * 5 + t) * nb + l] = deltafnc(ddy, dymin);
-    st.phi[(2 * 5 + t) * nb + l] = deltafnc(ddz, dz);
+    st.idx[sidx(0, t, l)] = X;
+    st.idx[sidx(1, t, l)] = Y;
+    st.idx[sidx(2, t, l)] = Z;
+    st.dd[sidx(0, t, l)] = ddx;
+    st.dd[sidx(1, t, l)] = ddy;
+    st.dd[sidx(2, t, l)] = ddz;
+    st.phi[sidx(0, t, l)] = deltafnc(ddx, dx);
+    st.phi[sidx(1, t, l)] = deltafnc(ddy, dymin);
+    st.phi[sidx(2, t, l)] = deltafnc(ddz, dz);
   }
 }
 
@@ -139,8 +139,8 @@ __global__ void k_mark_planes(Markers m, int* live) {
   const int tid = blockIdx.x * blockDim.x + threadIdx.x;
   const int nb = m.nb;
   if (tid >= 20 * nb) return;
-  const int s = tid / (5 * nb), e = tid - s * 5 * nb;  // e = t*nb + l
-  const int jj = m.st[s].idx[5 * nb + e] - 2;
+  const int l = tid / 20, e = tid - 20 * l, s = e / 5;
+  const int jj = m.st[s].idx[sidx(1, e - 5 * s, l)] - 2;
   // every writer stores the same value; a set plane is not stored again
   if (!live[jj]) live[jj] = 1;
   if (s == 1 && !live[jj + 1]) live[jj + 1] = 1;
@@ -226,220 +226,207 @@ __device__ __forceinline__ double wave_sum(double v) {
   return v;
 }
 
-// Point p = i + 5*(j + 5*k) of marker l in stencil st: node indices, weight
-// and (optionally) the normal distance n . (x_node - xb).
-struct Pt {
-  int X, Y, Z;
-  double w, dxn;
-};
-
-template <bool DXN>
-__device__ __forceinline__ Pt stencil_point(const Markers& m, const Stencil& st, int l, int p) {
-  const int nb = m.nb;
-  const int i = p % 5, j = (p / 5) % 5, k = p / 25;
-  Pt r;
-  r.X = st.idx[(0 * 5 + i) * nb + l];
-  r.Y = st.idx[(1 * 5 + j) * nb + l];
-  r.Z = st.idx[(2 * 5 + k) * nb + l];
-  r.w = ((m.A * st.phi[(0 * 5 + i) * nb + l]) * st.phi[(1 * 5 + j) * nb + l]) *
-        st.phi[(2 * 5 + k) * nb + l];
-  r.dxn = 0.0;
-  if (DXN)
-    r.dxn = (m.normals[l] * st.dd[(0 * 5 + i) * nb + l] +
-             m.normals[nb + l] * st.dd[(1 * 5 + j) * nb + l]) +
-            m.normals[2 * nb + l] * st.dd[(2 * 5 + k) * nb + l];
-  return r;
+// Sum over the 32 lanes of each half of the wavefront: lane pairs, quads and
+// rows of 16 through DPP, the two rows by a cross-lane read.
+template <int CTRL>
+__device__ __forceinline__ double dpp_add(double v) {
+  const unsigned long long b = __builtin_bit_cast(unsigned long long, v);
+  const unsigned lo = (unsigned)__builtin_amdgcn_update_dpp(0, (int)(unsigned)b, CTRL, 0xf, 0xf, false);
+  const unsigned hi =
+      (unsigned)__builtin_amdgcn_update_dpp(0, (int)(unsigned)(b >> 32), CTRL, 0xf, 0xf, false);
+  return v + __builtin_bit_cast(double, ((unsigned long long)hi << 32) | lo);
 }
+__device__ __forceinline__ double half_sum(double v) {
+  v = dpp_add<0xB1>(v);   // quad_perm 1,0,3,2
+  v = dpp_add<0x4E>(v);   // quad_perm 2,3,0,1
+  v = dpp_add<0x141>(v);  // mirrored within 8 (the quads' sums are equal there)
+  v = dpp_add<0x140>(v);  // mirrored within 16
+  return v + __shfl_xor(v, 16, 64);
+}
+
+// The stencil tables and normals as arguments of their own: read-only for the
+// whole kernel, so that wave-uniform reads become scalar loads.
+#define C3D_STENCIL_ARGS                                                           \
+  const int *__restrict__ idx, const double *__restrict__ phi, const double *__restrict__ dd, \
+      const double *__restrict__ normals
+#define C3D_STENCIL(m) m.st[0].idx, m.st[0].phi, m.st[0].dd, m.normals
 
 // Marker handled by this wavefront (XCD-aware: neighbouring markers, whose
 // stencils share nodes, run on the same XCD and L2).
 __device__ __forceinline__ int wave_marker(int nb) {
   unsigned bx, by, bz;
   xcd_tile(bx, by, bz);
-  return (int)bx * (kBlock / 64) + (int)(threadIdx.x >> 6);
+  return __builtin_amdgcn_readfirstlane((int)bx * (kBlock / 64) + (int)(threadIdx.x >> 6));
 }
 
-// Sums over the u, v and w stencils of marker l at once: the 375 points are
-// spread over the 64 lanes (up to 6 per lane, all loads in flight together)
-// and term(c, point) is accumulated per component; the three sums are then
-// reduced across the wavefront.
-// Per-axis stencil values of marker l held one per lane: lane 15c + 5a + t
-// (c < ncomp) holds entry (axis a, position t) of stencil st[c0 + c]; the
-// 125 points then fetch theirs by cross-lane reads instead of 6 loads each.
-struct LaneStencil {
-  int idx;
-  double phi, dd;
-};
-
-template <bool DXN>
-__device__ __forceinline__ LaneStencil load_lane_stencil(const Markers& m, int l, int lane, int c0,
-                                                         int ncomp) {
-  LaneStencil r{0, 0.0, 0.0};
-  if (lane < 15 * ncomp) {
-    const int c = c0 + lane / 15, e = lane % 15;  // e = 5a + t
-    const Stencil st = c == 0 ? m.st[0] : (c == 1 ? m.st[1] : (c == 2 ? m.st[2] : m.st[3]));
-    const size_t o = (size_t)e * m.nb + l;
-    r.idx = st.idx[o];
-    r.phi = st.phi[o];
-    if (DXN) r.dd = st.dd[o];
-  }
-  return r;
-}
-
-// Point p = i + 5*(j + 5*k) of the c-th loaded stencil, from the lanes.
-template <bool DXN>
-__device__ __forceinline__ Pt lane_point(const Markers& m, const LaneStencil& ls, int l, int c, int p) {
-  const int i = p % 5, j = (p / 5) % 5, k = p / 25;
-  const int b = 15 * c;
-  Pt r;
-  r.X = __shfl(ls.idx, b + i, 64);
-  r.Y = __shfl(ls.idx, b + 5 + j, 64);
-  r.Z = __shfl(ls.idx, b + 10 + k, 64);
-  r.w = ((m.A * __shfl(ls.phi, b + i, 64)) * __shfl(ls.phi, b + 5 + j, 64)) *
-        __shfl(ls.phi, b + 10 + k, 64);
-  r.dxn = 0.0;
-  if (DXN) {
-    r.dxn = (m.normals[l] * __shfl(ls.dd, b + i, 64) + m.normals[m.nb + l] * __shfl(ls.dd, b + 5 + j, 64)) +
-            m.normals[2 * m.nb + l] * __shfl(ls.dd, b + 10 + k, 64);
-  }
-  return r;
-}
-
-template <bool DXN, typename Term>
-__device__ __forceinline__ void gather3(const Markers& m, int l, int lane, Term term, double out[3]) {
-  const LaneStencil ls = load_lane_stencil<DXN>(m, l, lane, 0, 3);
-  double acc[3] = {0.0, 0.0, 0.0};
+// Stencil sums of marker l over field FA with stencil CA on lanes 0..31 and FB
+// with CB on lanes 32..63 (CB < 0: those lanes idle); every lane of a half
+// returns its half's sum.  Lane 5j + i of a half holds window position (i, j)
+// and walks the five z positions, whose values are wave-uniform (scalar
+// loads): five gathers per lane, each of 5-node runs, and no cross-lane reads
+// before the sum.  Spreading the 125 points over the lanes took 70 LDS
+// permutations a marker to hand out the per-axis values, which bound it.
+// DA, DB: terms times the normal distance n . (x_node - xb).
+template <int CA, int CB, bool DA, bool DB>
+__device__ __forceinline__ double gather_pair(const DevGrid& g, const Markers& m,
+                                              const int* __restrict__ idx,
+                                              const double* __restrict__ phi,
+                                              const double* __restrict__ dd,
+                                              const double* __restrict__ normals, int l, int lane,
+                                              const double* __restrict__ FA,
+                                              const double* __restrict__ FB) {
+  constexpr int C1 = CB < 0 ? CA : CB;
+  constexpr int DS = C1 - CA;
+  const bool hi = lane >= 32;
+  const int p = lane & 31;
+  const bool on = p < 25 && (CB >= 0 || !hi);
+  const int i = on ? p % 5 : 0, j = on ? p / 5 : 0;
+  const size_t b = (size_t)l * kStencils;           // wave-uniform
+  const int ba = CA * kStencil;
+  const int bl = ba + (hi ? DS * kStencil : 0);     // this half's stencil
+  // strides of the field (the centre field is rhs_p-shaped, first index 2)
+  auto n1 = [&](int c) { return c == 0 ? g.nx : (c == 3 ? g.nxg - 2 : g.nxg); };
+  auto n2 = [&](int c) { return c == 1 ? g.ny : (c == 3 ? g.nyg - 2 : g.nyg); };
+  const int s1 = hi ? n1(C1) : n1(CA);
+  const int s2 = hi ? n1(C1) * n2(C1) : n1(CA) * n2(CA);
+  const int first = (hi ? C1 : CA) == 3 ? 2 : 1;
+  const double* F = hi && CB >= 0 ? FB : FA;
+  const int X = idx[b + bl + i], Y = idx[b + bl + 5 + j];
+  const double px = phi[b + bl + i], py = phi[b + bl + 5 + j];
+  int Z[5];
+  double pz[5];
 #pragma unroll
-  for (int q = 0; q < 6; q++) {
-    const int p = lane + 64 * q;
-    const int c = p >= 250 ? 2 : (p >= 125 ? 1 : 0);
-    // all lanes take part in the cross-lane reads; out-of-range points add 0
-    const Pt pt = lane_point<DXN>(m, ls, l, c, (p < 375) ? p - 125 * c : 0);
-    if (p < 375) {
-      const double v = term(c, pt);
-      acc[0] += c == 0 ? v : 0.0;
-      acc[1] += c == 1 ? v : 0.0;
-      acc[2] += c == 2 ? v : 0.0;
+  for (int k = 0; k < 5; k++) {
+    const int za = idx[b + ba + 10 + k], zb = idx[b + ba + DS * kStencil + 10 + k];
+    const double pa = phi[b + ba + 10 + k], pb = phi[b + ba + DS * kStencil + 10 + k];
+    Z[k] = hi ? zb : za;
+    pz[k] = hi ? pb : pa;
+  }
+  const int o0 = (X - first) + s1 * (Y - first);
+  double f[5];
+#pragma unroll
+  for (int k = 0; k < 5; k++) f[k] = F[o0 + s2 * (Z[k] - first)];
+  const double wxy = (m.A * px) * py;
+  double acc = 0.0;
+  if (DA || DB) {
+    const double dx = dd[b + bl + i], dy = dd[b + bl + 5 + j];
+    const double nx = normals[l], ny = normals[m.nb + l], nz = normals[2 * (size_t)m.nb + l];
+    const double dxy = nx * dx + ny * dy;
+#pragma unroll
+    for (int k = 0; k < 5; k++) {
+      const double da = dd[b + ba + 10 + k], db = dd[b + ba + DS * kStencil + 10 + k];
+      const double v = (wxy * pz[k]) * f[k];
+      const double vd = v * (dxy + nz * (hi ? db : da));
+      acc += (hi ? DB : DA) ? vd : v;
     }
-  }
+  } else {
 #pragma unroll
-  for (int c = 0; c < 3; c++) out[c] = wave_sum(acc[c]);
+    for (int k = 0; k < 5; k++) acc += (wxy * pz[k]) * f[k];
+  }
+  return half_sum(on ? acc : 0.0);
 }
 
-// E / E1n of U, V, W (src/immersed_boundary_operators.f90:409-501).
+// E / E1n of U, V, W (src/immersed_boundary_operators.f90:409-501): the sums
+// of the three components of marker l, component c < 2 on half c, 2 on half 0.
 template <bool DXN>
-__global__ __launch_bounds__(kBlock) void k_interp_uvw(DevGrid g, Markers m, const double* __restrict__ U,
+__device__ __forceinline__ void gather_uvw(const DevGrid& g, const Markers& m, int l, int lane,
+                                           const int* __restrict__ idx, const double* __restrict__ phi,
+                                           const double* __restrict__ dd,
+                                           const double* __restrict__ normals,
+                                           const double* __restrict__ U, const double* __restrict__ V,
+                                           const double* __restrict__ W, double r[2]) {
+  r[0] = gather_pair<0, 1, DXN, DXN>(g, m, idx, phi, dd, normals, l, lane, U, V);
+  r[1] = gather_pair<2, -1, DXN, DXN>(g, m, idx, phi, dd, normals, l, lane, W, W);
+}
+
+template <bool DXN>
+__global__ __launch_bounds__(kBlock) void k_interp_uvw(DevGrid g, Markers m, C3D_STENCIL_ARGS,
+                                                       const double* __restrict__ U,
                                                        const double* __restrict__ V,
                                                        const double* __restrict__ W,
                                                        double* __restrict__ out) {
   const int l = wave_marker(m.nb);
   const int lane = threadIdx.x & 63;
   if (l >= m.nb) return;
-  const int nx = g.nx, ny = g.ny, nxg = g.nxg, nyg = g.nyg;
-  double r[3];
-  gather3<DXN>(m, l, lane, [&](int c, const Pt& q) {
-    const double f = c == 0 ? U[fidx(q.X, q.Y, q.Z, nx, nyg)]
-                            : (c == 1 ? V[fidx(q.X, q.Y, q.Z, nxg, ny)] : W[fidx(q.X, q.Y, q.Z, nxg, nyg)]);
-    double v = q.w * f;
-    if (DXN) v = v * q.dxn;
-    return v;
-  }, r);
-  if (lane == 0)
-    for (int c = 0; c < 3; c++) out[c * m.nb + l] = r[c];
+  double r[2];
+  gather_uvw<DXN>(g, m, l, lane, idx, phi, dd, normals, U, V, W, r);
+  if ((lane & 31) == 0) out[(lane >> 5) * m.nb + l] = r[0];
+  if (lane == 0) out[2 * m.nb + l] = r[1];
 }
 
-// E1n of a centre field in rhs_p layout (:503-526), marker l on one wave.
-__device__ __forceinline__ void interp_c_marker(const DevGrid& g, const Markers& m, int l, int lane,
-                                                const double* __restrict__ P, double sign,
-                                                double* __restrict__ out) {
-  const LaneStencil ls = load_lane_stencil<true>(m, l, lane, 3, 1);
-  double acc = 0.0;
-#pragma unroll
-  for (int q = 0; q < 2; q++) {
-    const int p = lane + 64 * q;
-    const Pt pt = lane_point<true>(m, ls, l, 0, p < 125 ? p : 0);
-    if (p < 125) acc += (pt.w * P[ridx(pt.X, pt.Y, pt.Z, g.nxg, g.nyg)]) * pt.dxn;
-  }
-  acc = wave_sum(acc);
-  if (lane == 0) out[l] = sign * acc;
-}
-
-__global__ __launch_bounds__(kBlock) void k_interp_c(DevGrid g, Markers m, const double* __restrict__ P,
-                                                     double sign, double* __restrict__ out) {
+// E1n of a centre field in rhs_p layout (:503-526).
+__global__ __launch_bounds__(kBlock) void k_interp_c(DevGrid g, Markers m, C3D_STENCIL_ARGS,
+                                                     const double* __restrict__ P, double sign,
+                                                     double* __restrict__ out) {
   const int l = wave_marker(m.nb);
+  const int lane = threadIdx.x & 63;
   if (l >= m.nb) return;
-  interp_c_marker(g, m, l, threadIdx.x & 63, P, sign, out);
+  const double r = gather_pair<3, -1, true, true>(g, m, idx, phi, dd, normals, l, lane, P, P);
+  if (lane == 0) out[l] = sign * r;
 }
 
-// Schur velocity rows (src/projection.f90:131-142) with the gradient of
-// dt*phi evaluated at the stencil nodes; every node lies in the gradient's
-// index ranges (checked at set-up), where apply_boundary_conditions does not
-// write.
-__device__ __forceinline__ void schur_u_marker(const DevGrid& g, const Markers& m, int l, int lane,
-                                               const double* __restrict__ phi, double dt,
-                                               const double* __restrict__ Ureg,
-                                               const double* __restrict__ Vreg,
-                                               const double* __restrict__ Wreg,
-                                               const double* __restrict__ E1nH,
-                                               const double* __restrict__ dudn,
-                                               double* __restrict__ Sf) {
-  const int nx = g.nx, ny = g.ny, nxg = g.nxg, nyg = g.nyg;
-  double r[3];
-  gather3<false>(m, l, lane, [&](int c, const Pt& q) {
-    const double p0 = dt * phi[ridx(q.X, q.Y, q.Z, nxg, nyg)];
-    double G, R;
-    if (c == 0) {
-      G = (dt * phi[ridx(q.X + 1, q.Y, q.Z, nxg, nyg)] - p0) / g.dxg[q.X];
-      R = Ureg[fidx(q.X, q.Y, q.Z, nx, nyg)];
-    } else if (c == 1) {
-      G = (dt * phi[ridx(q.X, q.Y + 1, q.Z, nxg, nyg)] - p0) / g.dyg[q.Y];
-      R = Vreg[fidx(q.X, q.Y, q.Z, nxg, ny)];
-    } else {
-      G = (dt * phi[ridx(q.X, q.Y, q.Z + 1, nxg, nyg)] - p0) / g.dzg[q.Z];
-      R = Wreg[fidx(q.X, q.Y, q.Z, nxg, nyg)];
-    }
-    return q.w * (G - R);
-  }, r);
-  if (lane == 0)
-    for (int c = 0; c < 3; c++)
-      Sf[c * m.nb + l] = r[c] - E1nH[c * m.nb + l] * dudn[c * m.nb + l];
+// G(dt*phi) - Reg_c of the Schur velocity rows (src/projection.f90:131-142) in
+// place of Reg_c, at the support nodes of each component (block row c): each
+// node once, where the markers' stencils would evaluate it for every one of
+// the (36 on average, two cylinders) entries that share it.  Every node lies
+// in the gradient's index ranges (checked at set-up), where
+// apply_boundary_conditions does not write.
+__global__ __launch_bounds__(kBlock) void k_node_grad(DevGrid g, Spread s0, Spread s1, Spread s2,
+                                                      const double* __restrict__ phi, double dt,
+                                                      double* __restrict__ F0, double* __restrict__ F1,
+                                                      double* __restrict__ F2) {
+  const int c = blockIdx.y;
+  const int nn = c == 0 ? s0.nnodes : (c == 1 ? s1.nnodes : s2.nnodes);
+  const int t = blockIdx.x * blockDim.x + threadIdx.x;
+  if (t >= nn) return;
+  const int* node = c == 0 ? s0.node : (c == 1 ? s1.node : s2.node);
+  double* F = c == 0 ? F0 : (c == 1 ? F1 : F2);
+  const unsigned n1 = c == 0 ? g.nx : g.nxg, n2 = c == 1 ? g.ny : g.nyg;
+  const unsigned o = (unsigned)node[t], r = o / n1;
+  const int i = (int)(o - r * n1) + 1, k = (int)(r / n2) + 1, j = (int)(r - (unsigned)(k - 1) * n2) + 1;
+  const double p0 = dt * phi[ridx(i, j, k, g.nxg, g.nyg)];
+  const double p1 = dt * phi[ridx(i + (c == 0), j + (c == 1), k + (c == 2), g.nxg, g.nyg)];
+  const double h = c == 0 ? g.dxg[i] : (c == 1 ? g.dyg[j] : g.dzg[k]);
+  F[o] = (p1 - p0) / h - F[o];
 }
 
-// Both row groups of the Schur product in one launch, one wave per marker:
-// the velocity rows (schur_u_marker), then the pressure row -E1n(phi) into
-// Sf[3nb..4nb) (as k_interp_c with sign -1), whose nodes the velocity rows
-// have just read.
-__global__ __launch_bounds__(kBlock) void k_schur_rows(DevGrid g, Markers m, const double* __restrict__ phi,
-                                                       double dt, const double* __restrict__ Ureg,
-                                                       const double* __restrict__ Vreg,
-                                                       const double* __restrict__ Wreg,
+// The four Schur rows of a marker (src/projection.f90:131-142) on one
+// wavefront: u with v, then w with the pressure row -E1n(phi).
+__global__ __launch_bounds__(kBlock) void k_schur_rows(DevGrid g, Markers m, C3D_STENCIL_ARGS,
+                                                       const double* __restrict__ P,
+                                                       const double* __restrict__ Du,
+                                                       const double* __restrict__ Dv,
+                                                       const double* __restrict__ Dw,
                                                        const double* __restrict__ E1nH,
                                                        const double* __restrict__ dudn,
                                                        double* __restrict__ Sf) {
   const int l = wave_marker(m.nb);
-  if (l >= m.nb) return;
   const int lane = threadIdx.x & 63;
-  schur_u_marker(g, m, l, lane, phi, dt, Ureg, Vreg, Wreg, E1nH, dudn, Sf);
-  interp_c_marker(g, m, l, lane, phi, -1.0, Sf + 3 * (size_t)m.nb);
+  if (l >= m.nb) return;
+  const double r0 = gather_pair<0, 1, false, false>(g, m, idx, phi, dd, normals, l, lane, Du, Dv);
+  const double r1 = gather_pair<2, 3, false, true>(g, m, idx, phi, dd, normals, l, lane, Dw, P);
+  if ((lane & 31) == 0) {
+    const int h = lane >> 5, o0 = h * m.nb + l;
+    Sf[o0] = r0 - E1nH[o0] * dudn[o0];
+    const int o1 = o0 + 2 * m.nb;
+    Sf[o1] = h ? -r1 : r1 - E1nH[o1] * dudn[o1];
+  }
 }
 
 // -E u + ub (src/projection.f90:51-52).
-__global__ __launch_bounds__(kBlock) void k_rhs_u(DevGrid g, Markers m, const double* __restrict__ U,
+__global__ __launch_bounds__(kBlock) void k_rhs_u(DevGrid g, Markers m, C3D_STENCIL_ARGS,
+                                                  const double* __restrict__ U,
                                                   const double* __restrict__ V,
                                                   const double* __restrict__ W,
                                                   double* __restrict__ out) {
   const int l = wave_marker(m.nb);
   const int lane = threadIdx.x & 63;
   if (l >= m.nb) return;
-  const int nx = g.nx, ny = g.ny, nxg = g.nxg, nyg = g.nyg;
-  double r[3];
-  gather3<false>(m, l, lane, [&](int c, const Pt& q) {
-    const double f = c == 0 ? U[fidx(q.X, q.Y, q.Z, nx, nyg)]
-                            : (c == 1 ? V[fidx(q.X, q.Y, q.Z, nxg, ny)] : W[fidx(q.X, q.Y, q.Z, nxg, nyg)]);
-    return q.w * f;
-  }, r);
-  if (lane == 0)
-    for (int c = 0; c < 3; c++) out[c * m.nb + l] = -r[c] + m.ub[c * m.nb + l];
+  double r[2];
+  gather_uvw<false>(g, m, l, lane, idx, phi, dd, normals, U, V, W, r);
+  const int o = (lane >> 5) * m.nb + l;
+  if ((lane & 31) == 0) out[o] = -r[0] + m.ub[o];
+  if (lane == 0) out[2 * m.nb + l] = -r[1] + m.ub[2 * m.nb + l];
 }
 
 __global__ void k_aux(Markers m, const double* __restrict__ f, double dt, double nu,
@@ -459,8 +446,8 @@ __global__ void k_spread_coeffs(int nb, double A, double factor, const double* _
   const int q = sp.q[e];
   const int l = q / 125, p = q - 125 * l;
   const int i = p % 5, j = (p / 5) % 5, k = p / 25;
-  const double w = ((A * phi[(0 * 5 + i) * nb + l]) * phi[(1 * 5 + j) * nb + l]) *
-                   phi[(2 * 5 + k) * nb + l];
+  const double w = ((A * phi[sidx(0, i, l)]) * phi[sidx(1, j, l)]) *
+                   phi[sidx(2, k, l)];
   sp.ml[e] = l;
   sp.wfs[e] = w * factor * sb[l];
 }
@@ -867,7 +854,8 @@ __global__ void k_hscale(double* __restrict__ q, double* __restrict__ x,
 }
 
 // check_slip, src/monitor.f90:223-231
-__global__ __launch_bounds__(kBlock) void k_max_slip(DevGrid g, Markers m, const double* __restrict__ U,
+__global__ __launch_bounds__(kBlock) void k_max_slip(DevGrid g, Markers m, C3D_STENCIL_ARGS,
+                                                     const double* __restrict__ U,
                                                      const double* __restrict__ V,
                                                      const double* __restrict__ W,
                                                      const double* __restrict__ E1nH,
@@ -876,22 +864,24 @@ __global__ __launch_bounds__(kBlock) void k_max_slip(DevGrid g, Markers m, const
   const int l = wave_marker(m.nb);
   const int lane = threadIdx.x & 63;
   if (l >= m.nb) return;
-  const int nx = g.nx, ny = g.ny, nxg = g.nxg, nyg = g.nyg;
-  double r[3];
-  gather3<false>(m, l, lane, [&](int c, const Pt& q) {
-    const double f = c == 0 ? U[fidx(q.X, q.Y, q.Z, nx, nyg)]
-                            : (c == 1 ? V[fidx(q.X, q.Y, q.Z, nxg, ny)] : W[fidx(q.X, q.Y, q.Z, nxg, nyg)]);
-    return q.w * f;
-  }, r);
-  double mx = 0.0;
-  for (int c = 0; c < 3; c++) {
-    const int o = c * m.nb + l;
-    mx = fmax(mx, fabs(r[c] - E1nH[o] * fb[o] - m.ub[o]));
-  }
+  double r[2];
+  gather_uvw<false>(g, m, l, lane, idx, phi, dd, normals, U, V, W, r);
+  auto slip = [&](double v, int o) { return fabs(v - E1nH[o] * fb[o] - m.ub[o]); };
+  double mx = slip(r[0], (lane >> 5) * m.nb + l);
+  if (lane < 32) mx = fmax(mx, slip(r[1], 2 * m.nb + l));
+  mx = fmax(mx, __shfl_xor(mx, 32, 64));
   if (lane == 0) atomicMax(red, (unsigned long long)__double_as_longlong(mx));
 }
 
 inline dim3 blocks_for(size_t n, int b = kBlock) { return dim3((unsigned)((n + b - 1) / b)); }
+// one lane per support node, a block row per component
+inline dim3 node_blocks(const Spread sp[3]) {
+  int mx = 1;
+  for (int c = 0; c < 3; c++) mx = sp[c].nnodes > mx ? sp[c].nnodes : mx;
+  dim3 grid = blocks_for((size_t)mx);
+  grid.y = 3;
+  return grid;
+}
 inline dim3 wave_blocks(int nb) { return dim3((unsigned)((nb + kBlock / 64 - 1) / (kBlock / 64))); }
 
 }  // namespace
@@ -919,29 +909,32 @@ hipError_t launch_wave_geometry(const WaveBody& w, const WaveTime& wt, double* x
 hipError_t launch_interp_uvw(const DevGrid& g, const Markers& m, const double* U, const double* V,
                              const double* W, bool with_dxn, double* out, hipStream_t s) {
   if (with_dxn)
-    hipLaunchKernelGGL(k_interp_uvw<true>, wave_blocks(m.nb), dim3(kBlock), 0, s, g, m, U, V, W, out);
+    hipLaunchKernelGGL(k_interp_uvw<true>, wave_blocks(m.nb), dim3(kBlock), 0, s, g, m, C3D_STENCIL(m), U, V, W, out);
   else
-    hipLaunchKernelGGL(k_interp_uvw<false>, wave_blocks(m.nb), dim3(kBlock), 0, s, g, m, U, V, W, out);
+    hipLaunchKernelGGL(k_interp_uvw<false>, wave_blocks(m.nb), dim3(kBlock), 0, s, g, m, C3D_STENCIL(m), U, V, W, out);
   return hipGetLastError();
 }
 
 hipError_t launch_interp_c(const DevGrid& g, const Markers& m, const double* P, double sign,
                            double* out, hipStream_t s) {
-  hipLaunchKernelGGL(k_interp_c, wave_blocks(m.nb), dim3(kBlock), 0, s, g, m, P, sign, out);
+  hipLaunchKernelGGL(k_interp_c, wave_blocks(m.nb), dim3(kBlock), 0, s, g, m, C3D_STENCIL(m), P, sign, out);
   return hipGetLastError();
 }
 
-hipError_t launch_schur_rows(const DevGrid& g, const Markers& m, const double* phi, double dt,
-                             const double* Ureg, const double* Vreg, const double* Wreg,
-                             const double* E1nH, const double* dudn, double* Sf, hipStream_t s) {
-  hipLaunchKernelGGL(k_schur_rows, wave_blocks(m.nb), dim3(kBlock), 0, s, g, m, phi, dt, Ureg, Vreg,
-                     Wreg, E1nH, dudn, Sf);
+hipError_t launch_schur_rows(const DevGrid& g, const Markers& m, const Spread sp[3],
+                             const double* phi, double dt, double* Ureg, double* Vreg,
+                             double* Wreg, const double* E1nH, const double* dudn, double* Sf,
+                             hipStream_t s) {
+  hipLaunchKernelGGL(k_node_grad, node_blocks(sp), dim3(kBlock), 0, s, g, sp[0], sp[1], sp[2], phi, dt,
+                     Ureg, Vreg, Wreg);
+  hipLaunchKernelGGL(k_schur_rows, wave_blocks(m.nb), dim3(kBlock), 0, s, g, m, C3D_STENCIL(m), phi,
+                     (const double*)Ureg, (const double*)Vreg, (const double*)Wreg, E1nH, dudn, Sf);
   return hipGetLastError();
 }
 
 hipError_t launch_rhs_u(const DevGrid& g, const Markers& m, const double* U, const double* V,
                         const double* W, double* out, hipStream_t s) {
-  hipLaunchKernelGGL(k_rhs_u, wave_blocks(m.nb), dim3(kBlock), 0, s, g, m, U, V, W, out);
+  hipLaunchKernelGGL(k_rhs_u, wave_blocks(m.nb), dim3(kBlock), 0, s, g, m, C3D_STENCIL(m), U, V, W, out);
   return hipGetLastError();
 }
 
@@ -953,11 +946,7 @@ hipError_t launch_aux(const Markers& m, const double* f, double dt, double nu, d
 
 hipError_t launch_spread3(const Markers& m, const Spread sp[3], const double* f, double* F0,
                           double* F1, double* F2, hipStream_t s) {
-  int mx = 0;
-  for (int c = 0; c < 3; c++) mx = sp[c].nnodes > mx ? sp[c].nnodes : mx;
-  if (mx == 0) return hipSuccess;
-  dim3 grid = blocks_for((size_t)mx);
-  grid.y = 3;
+  const dim3 grid = node_blocks(sp);
   hipLaunchKernelGGL(k_spread3, grid, dim3(kBlock), 0, s, sp[0], sp[1], sp[2], f, m.nb, F0, F1, F2);
   return hipGetLastError();
 }
@@ -1087,7 +1076,7 @@ hipError_t launch_hscale(double* q, double* x, const double* nrm2, const double*
 hipError_t launch_max_slip(const DevGrid& g, const Markers& m, const double* U, const double* V,
                            const double* W, const double* E1nH, const double* fb,
                            unsigned long long* red, hipStream_t s) {
-  hipLaunchKernelGGL(k_max_slip, wave_blocks(m.nb), dim3(kBlock), 0, s, g, m, U, V, W, E1nH, fb, red);
+  hipLaunchKernelGGL(k_max_slip, wave_blocks(m.nb), dim3(kBlock), 0, s, g, m, C3D_STENCIL(m), U, V, W, E1nH, fb, red);
   return hipGetLastError();
 }
 

@@ -9,12 +9,18 @@ namespace c3d {
 namespace ib {
 
 // Stencil of one staggered location (u, v, w or cell centre) for all
-// markers, separable per axis: entry (a, t, l) at [(a*5 + t)*nb + l] for axis
-// a = 0 x, 1 y, 2 z and window position t = 0..4.  idx holds the canonical
+// markers, separable per axis: entry (a, t, l) at sidx(a, t, l) for axis a = 0
+// x, 1 y, 2 z and window position t = 0..4.  The four stencils of a marker lie
+// side by side (st[s] points 15*s entries into the common arrays), so a
+// wavefront reads its marker's entries as a few whole lines.  idx holds the canonical
 // Fortran index of the node, phi the 1-D kernel value deltafnc(grid, xb, d),
 // dd the signed distance grid - xb.  The 125-point weight of (i, j, k) is
 // ((dx*dymin*dz * phi_x[i]) * phi_y[j]) * phi_z[k], the reference's product
 // order (src/immersed_boundary_operators.f90:86-91).
+constexpr int kStencil = 15, kStencils = 4 * kStencil;
+__host__ __device__ __forceinline__ size_t sidx(int a, int t, int l) {
+  return (size_t)l * kStencils + a * 5 + t;
+}
 struct Stencil {
   int* idx;
   double* phi;
@@ -96,12 +102,13 @@ hipError_t launch_interp_uvw(const DevGrid& g, const Markers& m, const double* U
 hipError_t launch_interp_c(const DevGrid& g, const Markers& m, const double* P, double sign,
                            double* out, hipStream_t s);
 // Schur rows: velocity rows Sf[c*nb+l] = E_c(G(dt*phi) - Reg_c)[l] -
-// E1nH[c*nb+l]*dudn[c*nb+l], G the gradient of the rhs_p-shaped phi evaluated
-// at the stencil nodes, and the pressure row Sf[3nb+l] = -E1n(phi)[l], in
-// one launch.
-hipError_t launch_schur_rows(const DevGrid& g, const Markers& m, const double* phi, double dt,
-                             const double* Ureg, const double* Vreg, const double* Wreg,
-                             const double* E1nH, const double* dudn, double* Sf, hipStream_t s);
+// E1nH[c*nb+l]*dudn[c*nb+l], G the gradient of the rhs_p-shaped phi, and the
+// pressure row Sf[3nb+l] = -E1n(phi)[l].  Leaves G(dt*phi) - Reg_c in place of
+// Reg_c at the support nodes.
+hipError_t launch_schur_rows(const DevGrid& g, const Markers& m, const Spread sp[3],
+                             const double* phi, double dt, double* Ureg, double* Vreg,
+                             double* Wreg, const double* E1nH, const double* dudn, double* Sf,
+                             hipStream_t s);
 // Velocity-rhs rows: out[c*nb+l] = -E_c(U)[l] + ub[c*nb+l].
 hipError_t launch_rhs_u(const DevGrid& g, const Markers& m, const double* U, const double* V,
                         const double* W, double* out, hipStream_t s);

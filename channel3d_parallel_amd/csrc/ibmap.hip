@@ -40,8 +40,8 @@ __global__ void k_map_keys(Stencil st, int nb, int n1, int n2, int* __restrict__
   if (e >= nb * 125) return;
   const int l = e / 125, p = e - 125 * l;
   const int i = p % 5, j = (p / 5) % 5, k = p / 25;
-  const int X = st.idx[(0 * 5 + i) * nb + l], Y = st.idx[(1 * 5 + j) * nb + l],
-            Z = st.idx[(2 * 5 + k) * nb + l];
+  const int X = st.idx[sidx(0, i, l)], Y = st.idx[sidx(1, j, l)],
+            Z = st.idx[sidx(2, k, l)];
   key[e] = (int)fidx(X, Y, Z, n1, n2);
   val[e] = e;
 }
