@@ -137,11 +137,11 @@ struct c3d_ctx {
   // Results that kernels store straight into (coherent) host memory, read
   // after a synchronisation: no copy and no staging per result.
   struct HostWords {
-    double v[8];         // flow integral and its norm
+    double v[8];         // flow integral and its norm; [2..4] compute_dt maxima
     unsigned nonfinite;  // g.nonfinite: set by the velocity corrections
   };
   HostWords* host = nullptr;
-  double* psum = nullptr;  // 7*nyg plane sums of compute_statistics
+  double* psum = nullptr;  // 7*nyg plane sums of compute_statistics, then their partials
   double* mon = nullptr;   // output_monitor partials and results
   size_t nu = 0, nv = 0, nw = 0, np = 0, nr = 0, nspec = 0;
   // RK3 state (allocated on first use): step-start copies, stage
@@ -553,7 +553,8 @@ int c3d_create(const c3d_desc* desc, c3d_ctx** out) {
       (rc = dalloc(c, &c->Pint, c->nr)) || (rc = dalloc(c, &c->rhs, c->nr)) ||
       (rc = dalloc(c, &c->xU, c->nu)) || (rc = dalloc(c, &c->xV, c->nv)) ||
       (rc = dalloc(c, &c->xW, c->nw)) || (rc = dalloc(c, &c->xF, interior_total(c))) ||
-      (rc = dalloc(c, &c->part, 2 * (size_t)c3d::massflow_parts(c->g) + 2)) ||
+      (rc = dalloc(c, &c->part, std::max(2 * (size_t)c3d::massflow_parts(c->g) + 2,
+                                           3 * (size_t)c3d::dt_parts(c->g)))) ||
       (rc = dalloc(c, &c->S, c->nspec)) ||
       (c3d::tri_needs_scratch(c->g) && (rc = dalloc(c, &c->CP, c->nspec))) ||
       (rc = dalloc(c, &c->red, kRedRefine + (size_t)kMaxRef * kResSlots)))
@@ -1051,15 +1052,10 @@ int c3d_rk3_update(c3d_ctx* c, int rk_step, double dt) {
 
 int c3d_compute_dt(c3d_ctx* c, double cfl, double* dt_out) {
   if (!c || !dt_out) return C3D_EINVAL;
-  unsigned long long h[3] = {0, 0, 0};
-  unsigned long long* red3 = c->red + 1;  // slots 1..3 of the reduction buffer
-  HIPCHK(c, hipMemsetAsync(red3, 0, sizeof(h), c->stream));
-  HIPCHK(c, c3d::launch_dt_max(c->g, c->U, c->V, c->W, red3, c->stream));
-  HIPCHK(c, hipMemcpyAsync(h, red3, sizeof(h), hipMemcpyDeviceToHost, c->stream));
+  double* lmax = c->host->v + 2;
+  HIPCHK(c, c3d::launch_dt_max(c->g, c->U, c->V, c->W, c->part, lmax, c->stream));
   int rc = sync(c);
   if (rc) return rc;
-  double lmax[3];
-  std::memcpy(lmax, h, sizeof(lmax));
   // src/time_integration.f90:241-265
   const double dtc = std::fmin(std::fmin(cfl * lmax[0], cfl * lmax[1]), cfl * lmax[2]);
   const double nu = c->desc.nu;
@@ -1107,10 +1103,11 @@ int c3d_compute_rhs_arrays(c3d_ctx* c, const double* U, const double* V, const d
 static int plane_means(c3d_ctx* c, std::vector<double>& m) {
   const int n = c->nyg;
   if (!c->psum) {
-    int rc = dalloc(c, &c->psum, 7 * (size_t)n);
+    int rc = dalloc(c, &c->psum, 7 * (size_t)n + c3d::plane_sums_part_size(c->g));
     if (rc) return rc;
   }
-  HIPCHK(c, c3d::launch_plane_sums(c->g, c->U, c->V, c->W, c->psum, c->stream));
+  HIPCHK(c, c3d::launch_plane_sums(c->g, c->U, c->V, c->W, c->psum + 7 * (size_t)n, c->psum,
+                                   c->stream));
   m.assign(7 * (size_t)n, 0.0);
   HIPCHK(c, hipMemcpyAsync(m.data(), c->psum, m.size() * sizeof(double), hipMemcpyDeviceToHost,
                            c->stream));
@@ -1148,12 +1145,12 @@ int c3d_monitor(c3d_ctx* c, double* out) {
 }
 
 // ---- allocation-free field summaries ----------------------------------------
-// Device scratch of c3d_monitor_noalloc: the 256 x 7 per-workgroup partials
+// Device scratch of c3d_monitor_noalloc: the 1024 x 7 per-workgroup partials
 // and the 7 reduced sums of the monitor kernels (the same count whatever the
 // grid).  Each device holds its own copy for the life of the process; its
 // address is looked up once per device and kept in kScratchPtr.
 namespace {
-constexpr size_t kScratchDoubles = 2048;
+constexpr size_t kScratchDoubles = 8192;
 static_assert((size_t)c3d::kMonitorPartDoubles + 8 <= kScratchDoubles, "monitor scratch");
 static __device__ __align__(256) double scratch[kScratchDoubles];
 constexpr int kMaxDevices = 64;
@@ -1185,7 +1182,7 @@ int c3d_monitor_noalloc(int nx, int ny, int nz, const double* U, const double* V
                         double* out, void* stream) {
   if (nx < 3 || ny < 3 || nz < 3 || nx > 1000000 || ny > 1000000 || nz > 1000000) return C3D_EINVAL;
   if (!U || !V || !W || !out) return C3D_EINVAL;
-  // the partials are a fixed 256 x 7 for every grid; this holds for the
+  // the partials are a fixed 1024 x 7 for every grid; this holds for the
   // kernels as built (the static_assert above), checked here as a limit
   if ((size_t)c3d::monitor_part_size() + 8 > kScratchDoubles) return C3D_EINVAL;
   hipError_t e = hipSuccess;

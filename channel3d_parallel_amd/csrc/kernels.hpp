@@ -177,11 +177,14 @@ struct RkStage {
   double *Fu, *Fv, *Fw;
   double *Un, *Vn, *Wn;
 };
+// z planes per workgroup of the right-hand-side kernels (2, 4 or 8).
+int rhs_planes(const DevGrid& g);
 hipError_t launch_rhs_stage(const DevGrid& g, int stage, const RkStage& a, hipStream_t s);
-// compute_dt maxima of dx/|u|, dy/|v|, dz/|w| as double bits into red3[0..2]
-// (red3 zeroed by the caller).
+// compute_dt maxima of dx/|u|, dy/|v|, dz/|w| into host3[0..2] (host memory
+// that the device writes); part holds 3*dt_parts(g) doubles.
+int dt_parts(const DevGrid& g);
 hipError_t launch_dt_max(const DevGrid& g, const double* U, const double* V, const double* W,
-                         unsigned long long* red3, hipStream_t s);
+                         double* part, double* host3, hipStream_t s);
 // Bulk-flow integral and norm of U into out2[0..1] and host2[0..1] (host
 // memory that the device writes); part holds 2*massflow_parts(g) doubles.
 int massflow_parts(const DevGrid& g);
@@ -191,7 +194,7 @@ hipError_t launch_massflow(const DevGrid& g, const double* U, const double* H, d
 // interiors, maxima of the same, and the count of non-finite entries; part
 // holds monitor_part_size() doubles of scratch.
 int monitor_part_size();
-constexpr int kMonitorPartDoubles = 256 * 7;  // monitor_part_size()
+constexpr int kMonitorPartDoubles = 1024 * 7;  // monitor_part_size()
 // out[0..6] = the results of c3d_monitor (maxima, sums / vol, non-finite
 // count) from the reduced sums r7 of launch_monitor, on the device.
 hipError_t launch_monitor_finish(const double* r7, double vol, double* out, hipStream_t s);
@@ -200,8 +203,10 @@ hipError_t launch_monitor(const DevGrid& g, const double* U, const double* V, co
 // Plane sums of compute_statistics over the unique cells of every row
 // j = 1..nyg: sums[q*nyg + j-1] for q = 0 x-centred U, 1 y-centred V (wall
 // rows mirrored), 2 W, 3 U^2, 4 V^2, 5 W^2, 6 UV (7*nyg doubles).
+// part holds plane_sums_part_size(g) doubles of scratch.
+size_t plane_sums_part_size(const DevGrid& g);
 hipError_t launch_plane_sums(const DevGrid& g, const double* U, const double* V, const double* W,
-                             double* sums, hipStream_t s);
+                             double* part, double* sums, hipStream_t s);
 
 // Streaming copy of nbytes (multiple of 16) for bandwidth calibration.
 hipError_t launch_copy(const void* src, void* dst, size_t nbytes, hipStream_t s);

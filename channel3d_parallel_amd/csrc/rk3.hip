@@ -6,6 +6,7 @@
 // expressions below (same operands, same operation order, same order of
 // accumulation: convective x, y, z, viscous, pressure gradient).  FMA
 // contraction is disabled so the results round exactly as written.
+#include <algorithm>
 #include <cstdlib>
 
 #include "bc_images.hpp"
@@ -137,22 +138,39 @@ __global__ __launch_bounds__(kB) void k_hold_flow(DevGrid g, double* __restrict_
 }
 
 // compute_dt maxima (src/time_integration.f90:228-239): max over the
-// centre range of dx/|u| per component, as bit patterns of non-negative
-// doubles (+Inf where u = 0).
+// centre range of dx/|u| per component (+Inf where u = 0).  A workgroup takes
+// 64 x positions, 4 rows and a run of planes, four planes' loads in flight at
+// a time, and leaves one partial per component: an atomic per workgroup onto
+// three words took most of the time of a small grid.
+constexpr int kDtPlanes = 4;
 __global__ __launch_bounds__(kB) void k_dt_max(DevGrid g, const double* __restrict__ U,
                                                const double* __restrict__ V,
-                                               const double* __restrict__ W,
-                                               unsigned long long* __restrict__ red) {
+                                               const double* __restrict__ W, int run,
+                                               double* __restrict__ part) {
   __shared__ double sm[3][kB / 64];
   const int i = blockIdx.x * 64 + (threadIdx.x & 63) + 2;
   const int j = blockIdx.y * 4 + (threadIdx.x >> 6) + 2;
   double m[3] = {0.0, 0.0, 0.0};
-  if (i <= g.nxg - 1 && j <= g.nyg - 1)
-    for (int k = blockIdx.z + 2; k <= g.nzg - 1; k += gridDim.z) {
-      m[0] = fmax(m[0], g.dxg[i] / fabs(U_(i, j, k)));
-      m[1] = fmax(m[1], g.dyg[j] / fabs(V_(i, j, k)));
-      m[2] = fmax(m[2], g.dzg[k] / fabs(W_(i, j, k)));
+  if (i <= g.nxg - 1 && j <= g.nyg - 1) {
+    const int ka = blockIdx.z * run + 2, ke = min(ka + run - 1, g.nzg - 1);
+    const double dx = g.dxg[i], dy = g.dyg[j];
+    for (int k0 = ka; k0 <= ke; k0 += kDtPlanes) {
+      double u[kDtPlanes], v[kDtPlanes], w[kDtPlanes];
+#pragma unroll
+      for (int r = 0; r < kDtPlanes; r++) {
+        const int k = min(k0 + r, ke);  // past the run: its last plane again
+        u[r] = U_(i, j, k);
+        v[r] = V_(i, j, k);
+        w[r] = W_(i, j, k);
+      }
+#pragma unroll
+      for (int r = 0; r < kDtPlanes; r++) {
+        m[0] = fmax(m[0], dx / fabs(u[r]));
+        m[1] = fmax(m[1], dy / fabs(v[r]));
+        m[2] = fmax(m[2], g.dzg[min(k0 + r, ke)] / fabs(w[r]));
+      }
     }
+  }
   for (int c = 0; c < 3; c++) {
     double v = m[c];
     for (int off = 32; off > 0; off >>= 1) v = fmax(v, __shfl_xor(v, off, 64));
@@ -162,7 +180,28 @@ __global__ __launch_bounds__(kB) void k_dt_max(DevGrid g, const double* __restri
   if (threadIdx.x < 3) {
     double v = sm[threadIdx.x][0];
     for (int w = 1; w < kB / 64; w++) v = fmax(v, sm[threadIdx.x][w]);
-    atomicMax(red + threadIdx.x, (unsigned long long)__double_as_longlong(v));
+    const size_t b = blockIdx.x + (size_t)gridDim.x * (blockIdx.y + (size_t)gridDim.y * blockIdx.z);
+    part[3 * b + threadIdx.x] = v;
+  }
+}
+
+constexpr int kDtFinal = 1024;
+__global__ __launch_bounds__(kDtFinal) void k_dt_final(const double* __restrict__ part, int n,
+                                                       double* host3) {
+  __shared__ double sm[3][kDtFinal / 64];
+  double m[3] = {0.0, 0.0, 0.0};
+#pragma unroll 2
+  for (int b = threadIdx.x; b < n; b += kDtFinal)
+    for (int c = 0; c < 3; c++) m[c] = fmax(m[c], part[3 * (size_t)b + c]);
+  for (int c = 0; c < 3; c++) {
+    for (int off = 32; off > 0; off >>= 1) m[c] = fmax(m[c], __shfl_xor(m[c], off, 64));
+    if ((threadIdx.x & 63) == 0) sm[c][threadIdx.x >> 6] = m[c];
+  }
+  __syncthreads();
+  if (threadIdx.x < 3) {
+    double v = sm[threadIdx.x][0];
+    for (int w = 1; w < kDtFinal / 64; w++) v = fmax(v, sm[threadIdx.x][w]);
+    host3[threadIdx.x] = v;
   }
 }
 
@@ -261,45 +300,62 @@ __global__ __launch_bounds__(kSumB) void k_sum_pairs(const double* __restrict__ 
 // i = 2..nxg-2 and k = 2..nzg-2 (W, W^2: k = 2..nz-1); fixed-order sums.
 constexpr int kStats = 7;
 
+// The planes are split into chunks so that 1024 workgroups share them (one
+// workgroup per row was 193 of them, 597 us on 384x192x384 cells); the chunks
+// are added in order by k_plane_final.
 __global__ __launch_bounds__(kB) void k_plane_sums(DevGrid g, const double* __restrict__ U,
                                                    const double* __restrict__ V,
-                                                   const double* __restrict__ W,
-                                                   double* __restrict__ sums) {
-  __shared__ double sh[kStats][kB];
+                                                   const double* __restrict__ W, int run,
+                                                   double* __restrict__ part) {
+  __shared__ double sh[kStats][kB / 64];
   const int j = blockIdx.x + 1;
   const int nx = g.nx, ny = g.ny, nxg = g.nxg, nyg = g.nyg;
-  const int ni = nxg - 3;
-  const int nku = g.nzg - 3, nkw = g.nz - 2;
+  const int lane = threadIdx.x & 63;
+  const int wv = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
   // term_2 at row j from V rows jv - 1, jv with sign sg (the wall rows mirror)
   const int jv = (j == 1) ? 2 : ((j == nyg) ? nyg - 1 : j);
   const double sg = (j == 1 || j == nyg) ? -1.0 : 1.0;
   double a[kStats] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
-  for (int t = threadIdx.x; t < ni * nku; t += kB) {
-    const int i = t % ni + 2, k = t / ni + 2;
-    const double t1 = 0.5 * (U[fidx(i - 1, j, k, nx, nyg)] + U[fidx(i, j, k, nx, nyg)]);
-    const double t2 = sg * (0.5 * (V[fidx(i, jv - 1, k, nxg, ny)] + V[fidx(i, jv, k, nxg, ny)]));
-    a[0] += t1;
-    a[1] += t2;
-    a[3] += t1 * t1;
-    a[4] += t2 * t2;
-    a[6] += t1 * t2;
-  }
-  for (int t = threadIdx.x; t < ni * nkw; t += kB) {
-    const int i = t % ni + 2, k = t / ni + 2;
-    const double w = W[fidx(i, j, k, nxg, nyg)];
-    a[2] += w;
-    a[5] += w * w;
+  // U, V: k = 2..nzg-2; W: k = 2..nz-1, the same range (nzg = nz + 1)
+  const int ka = blockIdx.y * run + 2, ke = min(ka + run - 1, g.nzg - 2);
+  for (int k = ka + wv; k <= ke; k += kB / 64) {
+    const double* u = U + fidx(1, j, k, nx, nyg);
+    const double* v = V + fidx(1, jv, k, nxg, ny);
+    const double* w = W + fidx(1, j, k, nxg, nyg);
+#pragma unroll 2
+    for (int i = 1 + lane; i <= nxg - 3; i += 64) {  // offset of x index i + 1
+      const double t1 = 0.5 * (u[i - 1] + u[i]);
+      const double t2 = sg * (0.5 * (v[i - nxg] + v[i]));
+      const double t3 = w[i];
+      a[0] += t1;
+      a[1] += t2;
+      a[2] += t3;
+      a[3] += t1 * t1;
+      a[4] += t2 * t2;
+      a[5] += t3 * t3;
+      a[6] += t1 * t2;
+    }
   }
 #pragma unroll
-  for (int q = 0; q < kStats; q++) sh[q][threadIdx.x] = a[q];
+  for (int q = 0; q < kStats; q++) {
+    for (int off = 32; off > 0; off >>= 1) a[q] += __shfl_xor(a[q], off, 64);
+    if (lane == 0) sh[q][wv] = a[q];
+  }
   __syncthreads();
-  for (int w = kB / 2; w > 0; w >>= 1) {
-    if ((int)threadIdx.x < w)
-#pragma unroll
-      for (int q = 0; q < kStats; q++) sh[q][threadIdx.x] += sh[q][threadIdx.x + w];
-    __syncthreads();
+  if (threadIdx.x < kStats) {
+    const double* t = sh[threadIdx.x];
+    part[((size_t)blockIdx.y * kStats + threadIdx.x) * nyg + j - 1] = (t[0] + t[1]) + (t[2] + t[3]);
   }
-  if (threadIdx.x < kStats) sums[threadIdx.x * (size_t)nyg + j - 1] = sh[threadIdx.x][0];
+}
+
+__global__ __launch_bounds__(kB) void k_plane_final(const double* __restrict__ part, int n, int chunks,
+                                                    double* __restrict__ sums) {
+  const int e = blockIdx.x * kB + threadIdx.x;
+  if (e >= n) return;
+  double s = 0.0;
+#pragma unroll 4
+  for (int c = 0; c < chunks; c++) s += part[(size_t)c * n + e];
+  sums[e] = s;
 }
 
 // output_monitor's field summaries (src/monitor.f90:27-47): per workgroup
@@ -308,18 +364,32 @@ __global__ __launch_bounds__(kB) void k_plane_sums(DevGrid g, const double* __re
 // three (a NaN guard), into part[b*kMon + q]; k_monitor_final reduces the
 // kMonBlocks partials in a fixed order.
 constexpr int kMon = 7;  // sum U, V, W; max U, V, W; non-finite count
-constexpr int kMonBlocks = 256;
+constexpr int kMonBlocks = 1024;
 
 __device__ __forceinline__ void mon_field(const double* __restrict__ F, int n1, int n2, int i1, int j1,
                                           int k1, double& sum, double& mx, double& bad) {
-  // interior (2..i1, 2..j1, 2..k1) of an (n1, n2, *) array, i fastest
-  const size_t ni = i1 - 1, nj = j1 - 1, n = ni * nj * (size_t)(k1 - 1);
-  for (size_t t = (size_t)blockIdx.x * kB + threadIdx.x; t < n; t += (size_t)kMonBlocks * kB) {
-    const int i = (int)(t % ni) + 2, j = (int)((t / ni) % nj) + 2, k = (int)(t / (ni * nj)) + 2;
-    const double v = F[fidx(i, j, k, n1, n2)];
-    sum += v;
-    mx = fmax(mx, v);
-    bad += isfinite(v) ? 0.0 : 1.0;
+  // interior (2..i1, 2..j1, 2..k1) of an (n1, n2, *) array: a wavefront takes
+  // 256 x positions of a row at a time, so the index arithmetic is scalar (a
+  // division per element made this 838 us on 384x192x384 cells)
+  const int lane = threadIdx.x & 63;
+  const long long ni = i1 - 1, nj = j1 - 1, nseg = (ni + 255) / 256;
+  const long long n = nseg * nj * (k1 - 1);
+  const int wv = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+  for (long long t = (long long)blockIdx.x * (kB / 64) + wv; t < n; t += kMonBlocks * (kB / 64)) {
+    const long long r = t / nseg, i0 = (t - r * nseg) * 256;
+    const long long k = r / nj, j = r - k * nj;
+    const double* row = F + 1 + (size_t)n1 * ((size_t)(j + 1) + (size_t)n2 * (size_t)(k + 1)) + i0;
+    double v[4];
+#pragma unroll
+    for (int q = 0; q < 4; q++)
+      if (i0 + q * 64 + lane < ni) v[q] = row[q * 64 + lane];
+#pragma unroll
+    for (int q = 0; q < 4; q++)
+      if (i0 + q * 64 + lane < ni) {
+        sum += v[q];
+        mx = fmax(mx, v[q]);
+        bad += isfinite(v[q]) ? 0.0 : 1.0;
+      }
   }
 }
 
@@ -351,7 +421,14 @@ __global__ __launch_bounds__(kB) void k_monitor_final(const double* __restrict__
                                                       double* __restrict__ out) {
   __shared__ double sh[kMon][kB];
 #pragma unroll
-  for (int q = 0; q < kMon; q++) sh[q][threadIdx.x] = part[(size_t)threadIdx.x * kMon + q];
+  for (int q = 0; q < kMon; q++) {
+    double a = part[(size_t)threadIdx.x * kMon + q];
+    for (int b = threadIdx.x + kB; b < kMonBlocks; b += kB) {
+      const double v = part[(size_t)b * kMon + q];
+      a = (q >= 3 && q < 6) ? fmax(a, v) : a + v;
+    }
+    sh[q][threadIdx.x] = a;
+  }
   __syncthreads();
   for (int w = kB / 2; w > 0; w >>= 1) {
     if ((int)threadIdx.x < w) {
@@ -369,26 +446,30 @@ inline dim3 gpts(int ni, int nj, int nk) { return dim3((ni + 63) / 64, (nj + 3) 
 
 }  // namespace
 
-// z planes per workgroup of the right-hand sides; C3D_RHS_KC (2, 4, 8, 16)
-// overrides the default 8 (tuning knob).
-static int rhs_kc() {
-  static const int kc = [] {
+// Eight planes (1.25 loaded per plane) where that leaves 4 workgroups for each
+// of the 256 CUs, else four or two, so that a small grid is not a few long
+// chains of planes.  C3D_RHS_KC (2, 4, 8) overrides it (tuning knob).
+int rhs_planes(const DevGrid& g) {
+  static const int forced = [] {
     const char* e = getenv("C3D_RHS_KC");
     const int v = e ? atoi(e) : 0;
-    return (v == 2 || v == 4 || v == 8 || v == 16) ? v : 8;
+    return (v == 2 || v == 4 || v == 8) ? v : 0;
   }();
+  if (forced) return forced;
+  const long long cols = (long long)((g.nxg - 2 + 63) / 64) * ((g.nyg - 2 + 3) / 4);
+  int kc = 8;
+  while (kc > 2 && cols * ((g.nzg - 2 + kc - 1) / kc) < 1024) kc /= 2;
   return kc;
 }
 
 hipError_t launch_rhs(const DevGrid& g, const double* U, const double* V, const double* W,
                       const double* Hu, const double* Hv, const double* Hw, double nu, double dPdx,
                       double dPdy, double dPdz, double* Fu, double* Fv, double* Fw, hipStream_t s) {
-  const int kc = rhs_kc();
+  const int kc = rhs_planes(g);
   const dim3 grid = gpts(g.nxg - 2, g.nyg - 2, (g.nzg - 2 + kc - 1) / kc);
   switch (kc) {
     case 2: hipLaunchKernelGGL(k_rhs<2>, grid, dim3(kB), 0, s, g, U, V, W, Hu, Hv, Hw, nu, dPdx, dPdy, dPdz, Fu, Fv, Fw); break;
     case 4: hipLaunchKernelGGL(k_rhs<4>, grid, dim3(kB), 0, s, g, U, V, W, Hu, Hv, Hw, nu, dPdx, dPdy, dPdz, Fu, Fv, Fw); break;
-    case 16: hipLaunchKernelGGL(k_rhs<16>, grid, dim3(kB), 0, s, g, U, V, W, Hu, Hv, Hw, nu, dPdx, dPdy, dPdz, Fu, Fv, Fw); break;
     default: hipLaunchKernelGGL(k_rhs<8>, grid, dim3(kB), 0, s, g, U, V, W, Hu, Hv, Hw, nu, dPdx, dPdy, dPdz, Fu, Fv, Fw); break;
   }
   return hipGetLastError();
@@ -416,10 +497,26 @@ hipError_t launch_hold_flow(const DevGrid& g, double* U, const double* sums, dou
   return hipGetLastError();
 }
 
+// Runs of planes per workgroup: about 2048 workgroups (8 per CU), at least
+// kDtPlanes planes each.
+static int dt_run(const DevGrid& g) {
+  const int cols = ((g.nxg - 2 + 63) / 64) * ((g.nyg - 2 + 3) / 4), nk = g.nzg - 2;
+  const int runs = std::max(1, std::min((2048 + cols - 1) / cols, nk / kDtPlanes));
+  return (nk + runs - 1) / runs;
+}
+static dim3 dt_grid(const DevGrid& g) {
+  const int run = dt_run(g);
+  return gpts(g.nxg - 2, g.nyg - 2, (g.nzg - 2 + run - 1) / run);
+}
+int dt_parts(const DevGrid& g) {
+  const dim3 n = dt_grid(g);
+  return (int)(n.x * n.y * n.z);
+}
+
 hipError_t launch_dt_max(const DevGrid& g, const double* U, const double* V, const double* W,
-                         unsigned long long* red3, hipStream_t s) {
-  hipLaunchKernelGGL(k_dt_max, gpts(g.nxg - 2, g.nyg - 2, g.nzg - 2 < 16 ? g.nzg - 2 : 16), dim3(kB),
-                     0, s, g, U, V, W, red3);
+                         double* part, double* host3, hipStream_t s) {
+  hipLaunchKernelGGL(k_dt_max, dt_grid(g), dim3(kB), 0, s, g, U, V, W, dt_run(g), part);
+  hipLaunchKernelGGL(k_dt_final, dim3(1), dim3(kDtFinal), 0, s, (const double*)part, dt_parts(g), host3);
   return hipGetLastError();
 }
 
@@ -455,15 +552,26 @@ hipError_t launch_monitor_finish(const double* r7, double vol, double* out, hipS
 
 hipError_t launch_monitor(const DevGrid& g, const double* U, const double* V, const double* W,
                           double* part, double* out7, hipStream_t s) {
-  static_assert(kMonBlocks == kB, "the final reduction holds one partial per thread");
+  static_assert(kMonBlocks % kB == 0, "the final reduction takes whole rounds of partials");
   hipLaunchKernelGGL(k_monitor_part, dim3(kMonBlocks), dim3(kB), 0, s, g, U, V, W, part);
   hipLaunchKernelGGL(k_monitor_final, dim3(1), dim3(kB), 0, s, (const double*)part, out7);
   return hipGetLastError();
 }
 
+// Planes per chunk of the plane sums: about 1024 workgroups.
+static int stat_run(const DevGrid& g) {
+  const int nk = g.nzg - 3, chunks = std::max(1, std::min(1024 / g.nyg, (nk + 3) / 4));
+  return (nk + chunks - 1) / chunks;
+}
+static int stat_chunks(const DevGrid& g) { return (g.nzg - 3 + stat_run(g) - 1) / stat_run(g); }
+size_t plane_sums_part_size(const DevGrid& g) { return (size_t)stat_chunks(g) * kStats * g.nyg; }
+
 hipError_t launch_plane_sums(const DevGrid& g, const double* U, const double* V, const double* W,
-                             double* sums, hipStream_t s) {
-  hipLaunchKernelGGL(k_plane_sums, dim3(g.nyg), dim3(kB), 0, s, g, U, V, W, sums);
+                             double* part, double* sums, hipStream_t s) {
+  const int n = kStats * g.nyg, c = stat_chunks(g);
+  hipLaunchKernelGGL(k_plane_sums, dim3(g.nyg, c), dim3(kB), 0, s, g, U, V, W, stat_run(g), part);
+  hipLaunchKernelGGL(k_plane_final, dim3((n + kB - 1) / kB), dim3(kB), 0, s, (const double*)part, n, c,
+                     sums);
   return hipGetLastError();
 }
 

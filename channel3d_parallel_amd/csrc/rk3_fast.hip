@@ -52,17 +52,21 @@ __device__ __forceinline__ void rhs_stage_body(const DevGrid& g, const RkStage& 
   TileAccX A{{tile, i0, j0, kb}, xt};
   // planes kb-1 and kb in LDS, kb+1 in registers; with PIPE, at plane k the
   // loads of plane k+2 are in flight while k is evaluated
+  // the first three planes' loads are all in flight before the first is stored
   PlaneRegs nxt;
-  load_plane(g, a.U, a.V, a.W, A, kb - 1, nxt);
-  store_plane(tile, A, kb - 1, nxt);
-  load_plane(g, a.U, a.V, a.W, A, kb, nxt);
-  store_plane(tile, A, kb, nxt);
-  if (PIPE) load_plane(g, a.U, a.V, a.W, A, kb + 1, nxt);
+  {
+    PlaneRegs p0, p1;
+    load_plane(g, a.U, a.V, a.W, A, kb - 1, p0);
+    load_plane(g, a.U, a.V, a.W, A, kb, p1);
+    load_plane(g, a.U, a.V, a.W, A, kb + 1, nxt);
+    store_plane(tile, A, kb - 1, p0);
+    store_plane(tile, A, kb, p1);
+  }
   const double dt = a.dt;
   for (int kk = 0; kk < KC; kk++) {
     const int k = kb + kk;
     if (k > nzg - 1) break;  // uniform across the workgroup
-    if (!PIPE) load_plane(g, a.U, a.V, a.W, A, k + 1, nxt);
+    if (!PIPE && kk > 0) load_plane(g, a.U, a.V, a.W, A, k + 1, nxt);
     store_plane(tile, A, k + 1, nxt);  // its slot held plane k-2, done with last iteration
     __syncthreads();
     if (PIPE && kk + 1 < KC && k + 1 <= nzg - 1) load_plane(g, a.U, a.V, a.W, A, k + 2, nxt);
@@ -134,9 +138,9 @@ int rhs_pipe() {
   return v;
 }
 
-template <int STAGE>
-void launch_stage_kernel(const DevGrid& g, const RkStage& a, dim3 grid, hipStream_t s) {
-  constexpr int KC = 8;
+template <int STAGE, int KC>
+void launch_stage_kernel(const DevGrid& g, const RkStage& a, hipStream_t s) {
+  const dim3 grid = gpts_f(g.nxg - 2, g.nyg - 2, (g.nzg - 2 + KC - 1) / KC);
   switch (rhs_pipe()) {
     case 1: hipLaunchKernelGGL((k_rhs_stage<KC, STAGE, true>), grid, dim3(kBf), 0, s, g, a); break;
     case 2: hipLaunchKernelGGL((k_rhs_stage_w4<KC, STAGE>), grid, dim3(kBf), 0, s, g, a); break;
@@ -144,17 +148,27 @@ void launch_stage_kernel(const DevGrid& g, const RkStage& a, dim3 grid, hipStrea
   }
 }
 
+template <int KC>
+hipError_t launch_stage(const DevGrid& g, int stage, const RkStage& a, hipStream_t s) {
+  switch (stage) {
+    case 1: launch_stage_kernel<1, KC>(g, a, s); break;
+    case 2: launch_stage_kernel<2, KC>(g, a, s); break;
+    case 3: launch_stage_kernel<3, KC>(g, a, s); break;
+    default: return hipErrorInvalidValue;
+  }
+  return hipSuccess;
+}
+
 }  // namespace
 
 hipError_t launch_rhs_stage(const DevGrid& g, int stage, const RkStage& a, hipStream_t s) {
-  constexpr int KC = 8;
-  const dim3 grid = gpts_f(g.nxg - 2, g.nyg - 2, (g.nzg - 2 + KC - 1) / KC);
-  switch (stage) {
-    case 1: launch_stage_kernel<1>(g, a, grid, s); break;
-    case 2: launch_stage_kernel<2>(g, a, grid, s); break;
-    case 3: launch_stage_kernel<3>(g, a, grid, s); break;
-    default: return hipErrorInvalidValue;
+  hipError_t e;
+  switch (rhs_planes(g)) {
+    case 2: e = launch_stage<2>(g, stage, a, s); break;
+    case 4: e = launch_stage<4>(g, stage, a, s); break;
+    default: e = launch_stage<8>(g, stage, a, s); break;
   }
+  if (e != hipSuccess) return e;
   return hipGetLastError();
 }
 
