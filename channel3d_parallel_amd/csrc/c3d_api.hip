@@ -81,10 +81,15 @@ struct IBState {
   };
   std::vector<IterGraph> graphs;
   bool use_graphs = true;
-  double* herr = nullptr;  // pinned host word: squared residual norm of the last iteration
+  // partials of the squared residual norm of the last two iterations, in
+  // (coherent) host memory that the device writes, and the events after them
+  double* herr = nullptr;
+  hipEvent_t iter_done[2] = {nullptr, nullptr};
   ~IBState() {
     for (auto& gr : graphs) (void)hipGraphExecDestroy(gr.exec);
     if (herr) (void)hipHostFree(herr);
+    for (hipEvent_t e : iter_done)
+      if (e) (void)hipEventDestroy(e);
   }
   // marker arrays (device) and the grid the stencil set-up reads
   double *xb = nullptr, *yb = nullptr, *zb = nullptr, *normals = nullptr, *sb = nullptr,
@@ -1392,9 +1397,19 @@ static int ib_poisson_reg(c3d_ctx* c, double dt, int rk_step, bool rows = false)
 // the Schur rows and the correction at interior cells) read no boundary cell.
 static int ib_spread_force(c3d_ctx* c, const double* f, double dt) {
   IBState* ib = c->ib;
-  const int nb = ib->m.nb;
   HIPCHK(c, c3d::ib::launch_aux(ib->m, f, dt, c->desc.nu, ib->aux, c->stream));
   HIPCHK(c, c3d::ib::launch_spread3(ib->m, ib->sp, ib->aux, ib->Ureg, ib->Vreg, ib->Wreg, c->stream));
+  return 0;
+}
+
+// schur (src/projection.f90:98-144) from the spread forces, up to the mean of
+// the pressure rows.
+static int ib_schur_rows(c3d_ctx* c, const double* f, double* Sf, double dt, int rk_step) {
+  IBState* ib = c->ib;
+  int rc = ib_poisson_reg(c, dt, rk_step, true);
+  if (rc) return rc;
+  HIPCHK(c, c3d::ib::launch_schur_rows(c->g, ib->m, ib->sp, ib->phi, dt, ib->Ureg, ib->Vreg, ib->Wreg,
+                                       ib->E1nH, f, Sf, c->stream));
   return 0;
 }
 
@@ -1403,34 +1418,39 @@ static int ib_schur_launch(c3d_ctx* c, const double* f, double* Sf, double dt, i
   IBState* ib = c->ib;
   const size_t nb = ib->m.nb;
   int rc = ib_spread_force(c, f, dt);
-  if (!rc) rc = ib_poisson_reg(c, dt, rk_step, true);
+  if (!rc) rc = ib_schur_rows(c, f, Sf, dt, rk_step);
   if (rc) return rc;
-  HIPCHK(c, c3d::ib::launch_schur_rows(c->g, ib->m, ib->sp, ib->phi, dt, ib->Ureg, ib->Vreg, ib->Wreg,
-                                       ib->E1nH, f, Sf, c->stream));
   HIPCHK(c, c3d::ib::launch_remove_mean(ib->m, Sf + 3 * nb, ib->E1nHc, f + 3 * nb, ib->mpart, c->stream));
   return 0;
 }
 
 // One BiCGSTAB iteration (src/projection.f90:160-182) on the stream, ending
-// with the squared residual norm stored to the pinned host word ib->herr.
+// with the partials of the squared residual norm stored to ib->herr.
 static int ib_bicg_iteration(c3d_ctx* c, double* x, double dt, int rk_step) {
   IBState* ib = c->ib;
   namespace B = c3d::ib;
   const size_t n = 4 * (size_t)ib->m.nb;
   double *r = ib->vec[1], *rhat = ib->vec[2], *p = ib->vec[3], *v = ib->vec[4], *h = ib->vec[5],
          *sv = ib->vec[6], *t = ib->vec[7];
+  const double nu = c->desc.nu;
+  // S f from the aux that the vector update before it left, and its dots
+  auto product = [&](const double* f, double* Sf, const double* a, bool two, int slot) -> int {
+    HIPCHK(c, B::launch_spread3(ib->m, ib->sp, ib->aux, ib->Ureg, ib->Vreg, ib->Wreg, c->stream));
+    int rc = ib_schur_rows(c, f, Sf, dt, rk_step);
+    if (rc) return rc;
+    HIPCHK(c, B::launch_mean_dot(ib->m, Sf, ib->E1nHc, f + 3 * (size_t)ib->m.nb, a, two, ib->mpart,
+                                 ib->part, slot, c->stream));
+    return 0;
+  };
   int rc = 0;
   // partial slot 0 holds rhat.r on entry (the initial dot, then k_bicg_xr)
-  HIPCHK(c, B::launch_bicg_p(r, v, ib->sc, ib->part, p, n, c->stream));
-  if ((rc = ib_schur_launch(c, p, v, dt, rk_step))) return rc;
-  HIPCHK(c, B::launch_dot(rhat, v, nullptr, nullptr, n, ib->part, 1, c->stream));
-  HIPCHK(c, B::launch_bicg_hs(x, p, r, v, ib->sc, ib->part, h, sv, n, c->stream));
-  if ((rc = ib_schur_launch(c, sv, t, dt, rk_step))) return rc;
-  HIPCHK(c, B::launch_dot(t, sv, t, t, n, ib->part, 2, c->stream));
-  HIPCHK(c, B::launch_bicg_xr(h, sv, t, rhat, ib->sc, ib->part, x, r, n, c->stream));
-  // the scalar kernel stores ||r||^2 straight into the pinned host word, so a
-  // captured iteration holds kernel nodes only (no device-to-host copy node)
-  HIPCHK(c, B::launch_bicg_scalar(4, ib->sc, ib->part, ib->herr, c->stream));
+  HIPCHK(c, B::launch_bicg_p(ib->m, r, v, ib->sc, ib->part, dt, nu, p, ib->aux, c->stream));
+  if ((rc = product(p, v, rhat, false, 1))) return rc;
+  HIPCHK(c, B::launch_bicg_hs(ib->m, x, p, r, v, ib->sc, ib->part, dt, nu, h, sv, ib->aux, c->stream));
+  if ((rc = product(sv, t, sv, true, 2))) return rc;
+  // the residual's partials go straight to host memory, so a captured
+  // iteration holds kernel nodes only (no device-to-host copy node)
+  HIPCHK(c, B::launch_bicg_xr(h, sv, t, rhat, ib->sc, ib->part, x, r, ib->herr, n, c->stream));
   return 0;
 }
 
@@ -1476,30 +1496,38 @@ static int ib_bicgstab_launch(c3d_ctx* c, double* x, const double* b, double tol
   double *r = ib->vec[1], *rhat = ib->vec[2], *p = ib->vec[3], *v = ib->vec[4];
   int rc = 0;
   // coherent (fine-grained) host memory: the kernel's store is visible to the
-  // host once the stream is synchronised
-  if (!ib->herr &&
-      hipHostMalloc((void**)&ib->herr, sizeof(double), hipHostMallocCoherent) != hipSuccess) {
+  // host once the iteration's event is done
+  if (!ib->herr && hipHostMalloc((void**)&ib->herr, 2 * B::kDotBlocks * sizeof(double),
+                                 hipHostMallocCoherent) != hipSuccess) {
     ib->herr = nullptr;
     (void)hipGetLastError();
-    return fail(c, C3D_ENOMEM, "pinned residual word");
+    return fail(c, C3D_ENOMEM, "residual words in host memory");
   }
+  for (hipEvent_t& e : ib->iter_done)
+    if (!e) HIPCHK(c, hipEventCreateWithFlags(&e, hipEventDisableTiming));
+  const double eps = tol * tol;
   if (!r_ready && (rc = ib_schur_launch(c, x, r, dt, rk_step))) return rc;
   HIPCHK(c, B::launch_bicg_init(r_ready ? nullptr : b, r, rhat, p, v, n, c->stream));
-  HIPCHK(c, B::launch_bicg_scalar(0, ib->sc, ib->part, nullptr, c->stream));
+  HIPCHK(c, B::launch_bicg_scalar(0, ib->sc, ib->part, eps, c->stream));
   HIPCHK(c, B::launch_dot(rhat, r, nullptr, nullptr, n, ib->part, 0, c->stream));
   hipGraphExec_t exec = nullptr;
   if (ib->use_graphs && maxit > 0 && (rc = ib_iteration_graph(c, x, dt, rk_step, &exec))) return rc;
+  // One iteration is queued ahead of the residual that decides on it, so that
+  // the device does not wait for the host between two (about 20 us each); once
+  // converged it leaves x as it is (k_bicg_p).
   double error = 1.0;
-  const double eps = tol * tol;
-  int iter = 0;
+  int iter = 0, queued = 0;
   while (iter < maxit && error >= eps) {
-    if (exec)
-      HIPCHK(c, hipGraphLaunch(exec, c->stream));
-    else if ((rc = ib_bicg_iteration(c, x, dt, rk_step)))
-      return rc;
-    HIPCHK(c, hipStreamSynchronize(c->stream));
-    error = *ib->herr;
+    for (; queued < maxit && queued < iter + 2; queued++) {
+      if (exec)
+        HIPCHK(c, hipGraphLaunch(exec, c->stream));
+      else if ((rc = ib_bicg_iteration(c, x, dt, rk_step)))
+        return rc;
+      HIPCHK(c, hipEventRecord(ib->iter_done[queued % 2], c->stream));
+    }
+    HIPCHK(c, hipEventSynchronize(ib->iter_done[iter % 2]));
     iter++;
+    error = B::residual_of_partials(ib->herr + (iter % 2) * B::kDotBlocks);
   }
   ib->last_iters = iter;
   ib->accum_iters += iter;
@@ -1728,7 +1756,7 @@ int ib_create(c3d_ctx* c, int nb, int nzb, int nxb, int nxb1) {
       (rc = dalloc(c, &ib->rhs_ib, n4)) || (rc = dalloc(c, &ib->fb, n4)) ||
       (rc = dalloc(c, &ib->fin, n4)) || (rc = dalloc(c, &ib->fout, n4)) ||
       (rc = dalloc(c, &ib->fprev, n4)) ||
-      (rc = dalloc(c, &ib->sc, 8)) || (rc = dalloc(c, &ib->part, 5 * (size_t)B::kDotBlocks)) ||
+      (rc = dalloc(c, &ib->sc, B::kBicgScalars)) || (rc = dalloc(c, &ib->part, 5 * (size_t)B::kDotBlocks)) ||
       (rc = dalloc(c, &ib->mpart, 128)) || (rc = dalloc(c, &ib->live, 3 * (size_t)c->nym)))
     return rc;
   for (int v = 0; v < 8; v++)
@@ -2455,7 +2483,7 @@ static int mlp_guess(c3d_ctx* c, double dt, int rk_step) {
   HIPCHK(c, N::apply(nb, m->act[N::kLayers - 1], m->oscale, nullptr, d, c->stream));
   if ((rc = ib_schur_launch(c, d, Sd, dt, rk_step))) return rc;      // S d
   HIPCHK(c, B::launch_dot(r, Sd, Sd, Sd, n4, ib->part, 2, c->stream));
-  HIPCHK(c, B::launch_bicg_scalar(5, ib->sc, ib->part, nullptr, c->stream));
+  HIPCHK(c, B::launch_bicg_scalar(5, ib->sc, ib->part, 0.0, c->stream));
   HIPCHK(c, B::launch_line_step(ib->fb, d, r, Sd, ib->sc, n4, c->stream));
   return 0;
 }

@@ -492,11 +492,22 @@ __global__ __launch_bounds__(kBlock) void k_spread3(Spread s0, Spread s1, Spread
 // (src/immersed_boundary_geometry.f90:400-442), then f -= coef*pj.  Block
 // partial sums of the two bodies, then every block re-reduces the partials
 // in the same fixed order and applies.
-constexpr int kMeanBlocks = 64;
+constexpr int kMeanBlocks = 64;  // one partial per lane of a wavefront
+
+__device__ __forceinline__ double block_sum(double v, double* sh) {
+  v = wave_sum(v);
+  const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  if (lane == 0) sh[w] = v;
+  __syncthreads();
+  double r = 0.0;
+  if (threadIdx.x == 0)
+    for (int q = 0; q < kBlock / 64; q++) r += sh[q];
+  return r;
+}
 
 __global__ __launch_bounds__(kBlock) void k_body_sums(Markers m, const double* __restrict__ f,
                                                       double* __restrict__ part) {
-  __shared__ double s1[kBlock], s2[kBlock];
+  __shared__ double s1[kBlock / 64], s2[kBlock / 64];
   const int nb = m.nb, nxb = m.nxb, nxb1 = m.nxb1;
   double a = 0.0, b = 0.0;
   for (int l = blockIdx.x * kBlock + threadIdx.x; l < nb; l += kMeanBlocks * kBlock) {
@@ -505,37 +516,33 @@ __global__ __launch_bounds__(kBlock) void k_body_sums(Markers m, const double* _
     else
       b += f[l];
   }
-  s1[threadIdx.x] = a;
-  s2[threadIdx.x] = b;
-  __syncthreads();
-  for (int o = kBlock / 2; o > 0; o >>= 1) {
-    if ((int)threadIdx.x < o) {
-      s1[threadIdx.x] += s1[threadIdx.x + o];
-      s2[threadIdx.x] += s2[threadIdx.x + o];
-    }
-    __syncthreads();
-  }
+  a = block_sum(a, s1);
+  b = block_sum(b, s2);
   if (threadIdx.x == 0) {
-    part[blockIdx.x] = s1[0];
-    part[kMeanBlocks + blockIdx.x] = s2[0];
+    part[blockIdx.x] = a;
+    part[kMeanBlocks + blockIdx.x] = b;
   }
+}
+
+// The two bodies' means from the partials: every wavefront sums them in the
+// same order.
+struct Means {
+  double a, b;
+};
+__device__ __forceinline__ Means body_means(const Markers& m, const double* __restrict__ part) {
+  const int lane = threadIdx.x & 63;
+  return {wave_sum(part[lane]) / (double)(m.nxb1 * m.nzb),
+          wave_sum(part[kMeanBlocks + lane]) / (double)((m.nxb - m.nxb1) * m.nzb)};
 }
 
 __global__ __launch_bounds__(kBlock) void k_remove_mean(Markers m, double* __restrict__ f,
                                                         const double* __restrict__ part,
                                                         const double* __restrict__ coef,
                                                         const double* __restrict__ pj) {
-  const int nb = m.nb, nxb = m.nxb, nxb1 = m.nxb1;
-  double a = 0.0, b = 0.0;
-  for (int q = 0; q < kMeanBlocks; q++) {
-    a += part[q];
-    b += part[kMeanBlocks + q];
-  }
-  const double avg1 = a / (double)(nxb1 * m.nzb);
-  const double avg2 = b / (double)((nxb - nxb1) * m.nzb);
+  const Means avg = body_means(m, part);
   const int l = blockIdx.x * kBlock + threadIdx.x;
-  if (l >= nb) return;
-  double v = f[l] - ((l % nxb < nxb1) ? avg1 : avg2);
+  if (l >= m.nb) return;
+  double v = f[l] - ((l % m.nxb < m.nxb1) ? avg.a : avg.b);
   if (coef) v = v - coef[l] * pj[l];
   f[l] = v;
 }
@@ -607,17 +614,6 @@ __global__ void k_h_interp(DevGrid g, const double* __restrict__ Hc, double* __r
 }
 
 // ---- BiCGSTAB ----
-__device__ __forceinline__ double block_sum(double v, double* sh) {
-  v = wave_sum(v);
-  const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  if (lane == 0) sh[w] = v;
-  __syncthreads();
-  double r = 0.0;
-  if (threadIdx.x == 0)
-    for (int q = 0; q < kBlock / 64; q++) r += sh[q];
-  return r;
-}
-
 __global__ __launch_bounds__(kBlock) void k_dot(const double* __restrict__ a, const double* __restrict__ b,
                                                 const double* __restrict__ a2,
                                                 const double* __restrict__ b2, size_t n,
@@ -636,10 +632,44 @@ __global__ __launch_bounds__(kBlock) void k_dot(const double* __restrict__ a, co
   }
 }
 
+// The partials of one slot, summed by a whole wavefront in a fixed order (the
+// host repeats it for the residual: residual_of_partials).
+static_assert(kDotBlocks == 128, "two partials per lane");
 __device__ __forceinline__ double sum_part(const double* part, int slot) {
-  double r = 0.0;
-  for (int b = 0; b < kDotBlocks; b++) r += part[slot * kDotBlocks + b];
-  return r;
+  const double* p = part + slot * kDotBlocks + (threadIdx.x & 63);
+  return wave_sum(p[0] + p[64]);
+}
+
+// The pressure rows' mean removal (k_remove_mean) and the dot products of the
+// finished Schur product with BiCGSTAB's vector a: <a, Sf> into partial slot
+// `slot` and, when two is set, <Sf, Sf> into the next.
+__global__ __launch_bounds__(kBlock) void k_mean_dot(Markers m, double* __restrict__ Sf,
+                                                     const double* __restrict__ mpart,
+                                                     const double* __restrict__ coef,
+                                                     const double* __restrict__ pj,
+                                                     const double* __restrict__ a, int two,
+                                                     double* __restrict__ part, int slot) {
+  __shared__ double sh[2][kBlock / 64];
+  const Means avg = body_means(m, mpart);
+  const int nb = m.nb, n3 = 3 * nb, n = 4 * nb;
+  double s1 = 0.0, s2 = 0.0;
+  for (int t = blockIdx.x * kBlock + threadIdx.x; t < n; t += kDotBlocks * kBlock) {
+    double v = Sf[t];
+    if (t >= n3) {
+      const int l = t - n3;
+      v = v - ((l % m.nxb < m.nxb1) ? avg.a : avg.b);
+      v = v - coef[l] * pj[l];
+      Sf[t] = v;
+    }
+    s1 += a[t] * v;
+    s2 += v * v;
+  }
+  const double r1 = block_sum(s1, sh[0]);
+  if (threadIdx.x == 0) part[slot * kDotBlocks + blockIdx.x] = r1;
+  if (two) {
+    const double r2 = block_sum(s2, sh[1]);
+    if (threadIdx.x == 0) part[(slot + 1) * kDotBlocks + blockIdx.x] = r2;
+  }
 }
 
 // Per-solve input normalisation of the learned guess: out[0] = 1/rms of the
@@ -647,114 +677,133 @@ __device__ __forceinline__ double sum_part(const double* part, int slot) {
 // same for slot sf (0 for a zero vector).
 __global__ void k_norm_scales(const double* __restrict__ part, int sr, double n_r, int sf, double n_f,
                               double* __restrict__ out) {
-  if (threadIdx.x != 0 || blockIdx.x != 0) return;
-  const double qr = sum_part(part, sr), qf = sum_part(part, sf);
+  const double qr = sum_part(part, sr), qf = sum_part(part, sf);  // launched as one wavefront
+  if (threadIdx.x != 0) return;
   out[0] = qr > 0.0 ? 1.0 / sqrt(qr / n_r) : 0.0;
   out[1] = qf > 0.0 ? 1.0 / sqrt(qf / n_f) : 0.0;
 }
 
 // Scalar slots: 0 rho_o, 1 alpha, 2 om, 3 rho_n, 4 bta, 5 err, 6 line-search
-// step.  The vector kernels below compute their scalar from the dot partials
-// themselves (thread 0 of every block, the same fixed-order sum) and block 0
-// stores it; no block of a kernel reads a slot that the same kernel writes.
-__global__ void k_bicg_scalar(int step, double* sc, const double* __restrict__ part,
-                              double* host_err) {
-  if (threadIdx.x != 0 || blockIdx.x != 0) return;
-  switch (step) {
-    case 0:
-      sc[0] = 1.0;
-      sc[1] = 1.0;
-      sc[2] = 1.0;
-      break;
-    case 4: {
-      const double e = sum_part(part, 4);
-      sc[5] = e;
-      if (host_err) {  // pinned host word read after the stream synchronises
-        *host_err = e;
-        __threadfence_system();
-      }
-      break;
-    }
-    case 5: {  // minimal-residual step along d: a = <r, S d> / <S d, S d>
-      const double den = sum_part(part, 3);
-      sc[6] = den > 0.0 ? sum_part(part, 2) / den : 0.0;
-      break;
-    }
+// step, 7 iterations begun, 8 the squared tolerance, 9 set once the solve has
+// converged.  The vector kernels compute their scalars from the dot partials
+// themselves (every wavefront, the same fixed-order sum) and block 0 stores
+// them; no block of a kernel reads a slot that the same kernel writes.
+__global__ void k_bicg_scalar(int step, double* sc, const double* __restrict__ part, double eps) {
+  const double den = sum_part(part, 3), num = sum_part(part, 2);  // launched as one wavefront
+  if (threadIdx.x != 0) return;
+  if (step == 0) {
+    sc[0] = 1.0;
+    sc[1] = 1.0;
+    sc[2] = 1.0;
+    sc[7] = 0.0;
+    sc[8] = eps;
+    sc[9] = 0.0;
+  } else {  // minimal-residual step along d: a = <r, S d> / <S d, S d>
+    sc[6] = den > 0.0 ? num / den : 0.0;
   }
 }
 
+// aux of the spreading (k_aux) for the entry (l, c = 0..2) of f, fp its
+// pressure entry.
+__device__ __forceinline__ double aux_entry(const Markers& m, double dt, double nu, double f, double fp,
+                                            int t) {
+  return dt * nu * f - dt * fp * m.normals[t];
+}
+
 // rho_n = rhat.r (partial slot 0); bta = (rho_n/rho_o)*(alpha/om);
-// p = r + bta*(p - om*v).  Writes sc[3] = rho_n, sc[4] = bta.
+// p = r + bta*(p - om*v), and the next spreading's aux of p; one lane per
+// marker.  Writes sc[3] = rho_n, sc[4] = bta and counts the iteration.
+// The host queues an iteration before it knows the last one's residual: when
+// that one (partial slot 4) met the tolerance, p, k_bicg_hs and k_bicg_xr
+// leave every vector as it is.
 // Breakdown guards here and in k_bicg_hs / k_bicg_xr: an exactly zero
 // denominator gives a zero step instead of the reference's 0/0
 // (src/projection.f90:165-172); a zero right-hand side then converges to
 // x = 0 in one iteration.  Nonzero denominators are untouched.
-__global__ void k_bicg_p(const double* __restrict__ r, const double* __restrict__ v,
-                         double* __restrict__ sc, const double* __restrict__ part,
-                         double* __restrict__ p, size_t n) {
-  __shared__ double bsh;
-  if (threadIdx.x == 0) {
-    const double rho_n = sum_part(part, 0);
-    const double bta = (sc[0] != 0.0 && sc[2] != 0.0) ? (rho_n / sc[0]) * (sc[1] / sc[2]) : 0.0;
-    bsh = bta;
-    if (blockIdx.x == 0) {
-      sc[3] = rho_n;
-      sc[4] = bta;
-    }
+__global__ __launch_bounds__(kBlock) void k_bicg_p(Markers m, const double* __restrict__ r,
+                                                   const double* __restrict__ v, const double* sc,
+                                                   double* scw, const double* __restrict__ part,
+                                                   double dt, double nu, double* __restrict__ p,
+                                                   double* __restrict__ aux) {
+  const double begun = sc[7];
+  const bool go = begun == 0.0 || sum_part(part, 4) >= sc[8];
+  const bool first = blockIdx.x == 0 && threadIdx.x == 0;
+  if (!go) {
+    if (first) scw[9] = 1.0;
+    return;
   }
-  __syncthreads();
-  const double bta = bsh, om = sc[2];
-  const size_t t = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= n) return;
-  p[t] = r[t] + bta * (p[t] - om * v[t]);
+  const double rho_n = sum_part(part, 0);
+  const double bta = (sc[0] != 0.0 && sc[2] != 0.0) ? (rho_n / sc[0]) * (sc[1] / sc[2]) : 0.0;
+  const double om = sc[2];
+  if (first) {
+    scw[3] = rho_n;
+    scw[4] = bta;
+    scw[5] = begun + 1.0;  // k_bicg_hs moves it to sc[7], which this kernel reads
+  }
+  const int l = blockIdx.x * kBlock + threadIdx.x, nb = m.nb;
+  if (l >= nb) return;
+  double q[4];
+#pragma unroll
+  for (int c = 0; c < 4; c++) {
+    const int t = c * nb + l;
+    q[c] = r[t] + bta * (p[t] - om * v[t]);
+    p[t] = q[c];
+  }
+#pragma unroll
+  for (int c = 0; c < 3; c++) aux[c * nb + l] = aux_entry(m, dt, nu, q[c], q[3], c * nb + l);
 }
 
-// alpha = rho_n / rhat.v (partial slot 1); h = x + alpha*p; s = r - alpha*v.
+// alpha = rho_n / rhat.v (partial slot 1); h = x + alpha*p; s = r - alpha*v,
+// and the next spreading's aux of s.
 // Writes sc[1] = alpha and sc[0] = rho_n (rho_o of the next iteration).
-__global__ void k_bicg_hs(const double* __restrict__ x, const double* __restrict__ p,
-                          const double* __restrict__ r, const double* __restrict__ v,
-                          double* __restrict__ sc, const double* __restrict__ part,
-                          double* __restrict__ h, double* __restrict__ sv, size_t n) {
-  __shared__ double ash;
-  if (threadIdx.x == 0) {
-    const double rho_n = sc[3];
-    const double den = sum_part(part, 1);
-    const double alpha = den != 0.0 ? rho_n / den : 0.0;
-    ash = alpha;
-    if (blockIdx.x == 0) {
-      sc[1] = alpha;
-      sc[0] = rho_n;
-    }
+__global__ __launch_bounds__(kBlock) void k_bicg_hs(Markers m, const double* __restrict__ x,
+                                                    const double* __restrict__ p,
+                                                    const double* __restrict__ r,
+                                                    const double* __restrict__ v, const double* sc,
+                                                    double* scw, const double* __restrict__ part,
+                                                    double dt, double nu, double* __restrict__ h,
+                                                    double* __restrict__ sv,
+                                                    double* __restrict__ aux) {
+  if (sc[9] != 0.0) return;
+  const double rho_n = sc[3];
+  const double den = sum_part(part, 1);
+  const double alpha = den != 0.0 ? rho_n / den : 0.0;
+  if (blockIdx.x == 0 && threadIdx.x == 0) {
+    scw[1] = alpha;
+    scw[0] = rho_n;
+    scw[7] = sc[5];
   }
-  __syncthreads();
-  const double alpha = ash;
-  const size_t t = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= n) return;
-  h[t] = x[t] + alpha * p[t];
-  sv[t] = r[t] - alpha * v[t];
+  const int l = blockIdx.x * kBlock + threadIdx.x, nb = m.nb;
+  if (l >= nb) return;
+  double q[4];
+#pragma unroll
+  for (int c = 0; c < 4; c++) {
+    const int t = c * nb + l;
+    h[t] = x[t] + alpha * p[t];
+    q[c] = r[t] - alpha * v[t];
+    sv[t] = q[c];
+  }
+#pragma unroll
+  for (int c = 0; c < 3; c++) aux[c * nb + l] = aux_entry(m, dt, nu, q[c], q[3], c * nb + l);
 }
 
 // om = t.s / t.t (partial slots 2, 3); x = h + om*s; r = s - om*t; partials
-// of r.r into slot 4 and of rhat.r into slot 0 (the next iteration's rho_n).
+// of r.r into slot 4 and of rhat.r into slot 0 (the next iteration's rho_n),
+// those of r.r also to host memory, one half of `host` for odd iterations and
+// one for even ones (the host reads one while the next iteration may run).
 // Writes sc[2] = om.
 __global__ __launch_bounds__(kBlock) void k_bicg_xr(const double* __restrict__ h,
                                                     const double* __restrict__ sv,
                                                     const double* __restrict__ tv,
                                                     const double* __restrict__ rhat,
-                                                    double* __restrict__ sc,
-                                                    double* __restrict__ part,
+                                                    const double* sc, double* scw, double* part,
                                                     double* __restrict__ x, double* __restrict__ r,
-                                                    size_t n) {
+                                                    double* host, size_t n) {
   __shared__ double sh[2][kBlock / 64];
-  __shared__ double osh;
-  if (threadIdx.x == 0) {
-    const double tt = sum_part(part, 3);
-    const double om = tt != 0.0 ? sum_part(part, 2) / tt : 0.0;
-    osh = om;
-    if (blockIdx.x == 0) sc[2] = om;
-  }
-  __syncthreads();
-  const double om = osh;
+  if (sc[9] != 0.0) return;
+  const double tt = sum_part(part, 3);
+  const double om = tt != 0.0 ? sum_part(part, 2) / tt : 0.0;
+  if (blockIdx.x == 0 && threadIdx.x == 0) scw[2] = om;
   double s4 = 0.0, s0 = 0.0;
   for (size_t t = (size_t)blockIdx.x * kBlock + threadIdx.x; t < n; t += (size_t)kDotBlocks * kBlock) {
     x[t] = h[t] + om * sv[t];
@@ -768,6 +817,7 @@ __global__ __launch_bounds__(kBlock) void k_bicg_xr(const double* __restrict__ h
   if (threadIdx.x == 0) {
     part[4 * kDotBlocks + blockIdx.x] = t4;
     part[0 * kDotBlocks + blockIdx.x] = t0;
+    host[((int)sc[7] & 1) * kDotBlocks + blockIdx.x] = t4;
   }
 }
 
@@ -820,9 +870,10 @@ __global__ __launch_bounds__(kBlock) void k_mdot(VecSet A, const double* __restr
   }
 }
 
-__global__ void k_mreduce(const double* __restrict__ part, int k, double* __restrict__ coef) {
-  const int j = threadIdx.x;
-  if (j < k) coef[j] = sum_part(part, j);
+// one wavefront per slot
+__global__ void k_mreduce(const double* __restrict__ part, double* __restrict__ coef) {
+  const double v = sum_part(part, blockIdx.x);
+  if (threadIdx.x == 0) coef[blockIdx.x] = v;
 }
 
 // qa = (set ? 0 : qa) + sgn * sum_j coef[j] A_j ; xb likewise with B_j
@@ -975,6 +1026,16 @@ hipError_t launch_remove_mean(const Markers& m, double* f, const double* coef, c
   return hipGetLastError();
 }
 
+hipError_t launch_mean_dot(const Markers& m, double* Sf, const double* coef, const double* pj,
+                           const double* a, bool two, double* mpart, double* part, int slot,
+                           hipStream_t s) {
+  hipLaunchKernelGGL(k_body_sums, dim3(kMeanBlocks), dim3(kBlock), 0, s, m,
+                     (const double*)(Sf + 3 * (size_t)m.nb), mpart);
+  hipLaunchKernelGGL(k_mean_dot, dim3(kDotBlocks), dim3(kBlock), 0, s, m, Sf, (const double*)mpart, coef,
+                     pj, a, two ? 1 : 0, part, slot);
+  return hipGetLastError();
+}
+
 hipError_t launch_ib_correct(const DevGrid& g, const double* Uint, const double* Vint,
                              const double* Wint, const double* Ureg, const double* Vreg,
                              const double* Wreg, const double* Pint, const double* phi, double dt,
@@ -1009,30 +1070,43 @@ hipError_t launch_norm_scales(const double* part, int sr, size_t n_r, int sf, si
   return hipGetLastError();
 }
 
-hipError_t launch_bicg_scalar(int step, double* sc, const double* part, double* host_err,
-                              hipStream_t s) {
-  hipLaunchKernelGGL(k_bicg_scalar, dim3(1), dim3(64), 0, s, step, sc, part, host_err);
+hipError_t launch_bicg_scalar(int step, double* sc, const double* part, double eps, hipStream_t s) {
+  hipLaunchKernelGGL(k_bicg_scalar, dim3(1), dim3(64), 0, s, step, sc, part, eps);
   return hipGetLastError();
 }
 
-hipError_t launch_bicg_p(const double* r, const double* v, double* sc, const double* part, double* p,
-                         size_t n, hipStream_t s) {
-  hipLaunchKernelGGL(k_bicg_p, blocks_for(n), dim3(kBlock), 0, s, r, v, sc, part, p, n);
+hipError_t launch_bicg_p(const Markers& m, const double* r, const double* v, double* sc,
+                         const double* part, double dt, double nu, double* p, double* aux,
+                         hipStream_t s) {
+  hipLaunchKernelGGL(k_bicg_p, blocks_for(m.nb), dim3(kBlock), 0, s, m, r, v, (const double*)sc, sc, part,
+                     dt, nu, p, aux);
   return hipGetLastError();
 }
 
-hipError_t launch_bicg_hs(const double* x, const double* p, const double* r, const double* v,
-                          double* sc, const double* part, double* h, double* sv, size_t n,
-                          hipStream_t s) {
-  hipLaunchKernelGGL(k_bicg_hs, blocks_for(n), dim3(kBlock), 0, s, x, p, r, v, sc, part, h, sv, n);
+hipError_t launch_bicg_hs(const Markers& m, const double* x, const double* p, const double* r,
+                          const double* v, double* sc, const double* part, double dt, double nu,
+                          double* h, double* sv, double* aux, hipStream_t s) {
+  hipLaunchKernelGGL(k_bicg_hs, blocks_for(m.nb), dim3(kBlock), 0, s, m, x, p, r, v, (const double*)sc, sc,
+                     part, dt, nu, h, sv, aux);
   return hipGetLastError();
 }
 
 hipError_t launch_bicg_xr(const double* h, const double* sv, const double* t, const double* rhat,
-                          double* sc, double* part, double* x, double* r, size_t n, hipStream_t s) {
-  hipLaunchKernelGGL(k_bicg_xr, dim3(kDotBlocks), dim3(kBlock), 0, s, h, sv, t, rhat, sc, part, x, r,
-                     n);
+                          double* sc, double* part, double* x, double* r, double* host, size_t n,
+                          hipStream_t s) {
+  hipLaunchKernelGGL(k_bicg_xr, dim3(kDotBlocks), dim3(kBlock), 0, s, h, sv, t, rhat, (const double*)sc,
+                     sc, part, x, r, host, n);
   return hipGetLastError();
+}
+
+double residual_of_partials(const double* host) {
+  double a[64], b[64];
+  for (int l = 0; l < 64; l++) a[l] = host[l] + host[l + 64];
+  for (int off = 32; off > 0; off >>= 1) {  // wave_sum
+    for (int l = 0; l < 64; l++) b[l] = a[l] + a[l ^ off];
+    for (int l = 0; l < 64; l++) a[l] = b[l];
+  }
+  return a[0];
 }
 
 hipError_t launch_bicg_init(const double* b, double* r, double* rhat, double* p, double* v,
@@ -1055,7 +1129,7 @@ hipError_t launch_mdot(const VecSet& A, const double* q, size_t n, double* part,
 
 hipError_t launch_mreduce(const double* part, int k, double* coef, hipStream_t s) {
   if (k < 1 || k > kHist + 1) return hipErrorInvalidValue;
-  hipLaunchKernelGGL(k_mreduce, dim3(1), dim3(64), 0, s, part, k, coef);
+  hipLaunchKernelGGL(k_mreduce, dim3(k), dim3(64), 0, s, part, coef);
   return hipGetLastError();
 }
 

@@ -155,33 +155,45 @@ hipError_t launch_h_interp(const DevGrid& g, const double* Hc, double* Hu, doubl
                            hipStream_t s);
 
 // BiCGSTAB (src/projection.f90:146-186) device scalars and vector kernels.
-// Scalar slots: 0 rho_o, 1 alpha, 2 om, 3 rho_n, 4 bta, 5 err.
 constexpr int kDotBlocks = 128;
 // part[slot*kDotBlocks + b] = block b's partial of sum a*b (slot selects one of
 // the partial arrays); two dots at once when a2 != nullptr (slot + 1).
 hipError_t launch_dot(const double* a, const double* b, const double* a2, const double* b2,
                       size_t n, double* part, int slot, hipStream_t s);
-// Scalar steps: 0 initialise, 4 err (also to *host_err when not null), 5
 // out[0] = 1/rms over n_r entries of the squares summed in slot sr, out[1]
 // likewise for slot sf (0 where the sum is 0).
 hipError_t launch_norm_scales(const double* part, int sr, size_t n_r, int sf, size_t n_f,
                               double* out, hipStream_t s);
-// minimal-residual step sc[6] = <r,Sd>/<Sd,Sd> from partial slots 2 and 3.
-hipError_t launch_bicg_scalar(int step, double* sc, const double* part, double* host_err,
-                              hipStream_t s);
+// Scalar steps: 0 initialise (eps: the squared tolerance), 5 minimal-residual
+// step sc[6] = <r,Sd>/<Sd,Sd> from partial slots 2 and 3.  sc: kBicgScalars.
+constexpr int kBicgScalars = 16;
+hipError_t launch_bicg_scalar(int step, double* sc, const double* part, double eps, hipStream_t s);
 // rho_n = rhat.r (slot 0), bta = (rho_n/rho_o)*(alpha/om) -> sc[3], sc[4];
-// p = r + bta*(p - om*v)
-hipError_t launch_bicg_p(const double* r, const double* v, double* sc, const double* part, double* p,
-                         size_t n, hipStream_t s);
+// p = r + bta*(p - om*v), and aux of p (launch_aux).  Once the residual of
+// the iteration before is below the tolerance, this kernel and the two below
+// change nothing any more.
+hipError_t launch_bicg_p(const Markers& m, const double* r, const double* v, double* sc,
+                         const double* part, double dt, double nu, double* p, double* aux,
+                         hipStream_t s);
 // alpha = rho_n / rhat.v (slot 1) -> sc[1], rho_o = rho_n -> sc[0];
-// h = x + alpha*p;  s = r - alpha*v
-hipError_t launch_bicg_hs(const double* x, const double* p, const double* r, const double* v,
-                          double* sc, const double* part, double* h, double* sv, size_t n,
-                          hipStream_t s);
+// h = x + alpha*p;  s = r - alpha*v, and aux of s
+hipError_t launch_bicg_hs(const Markers& m, const double* x, const double* p, const double* r,
+                          const double* v, double* sc, const double* part, double dt, double nu,
+                          double* h, double* sv, double* aux, hipStream_t s);
 // om = t.s / t.t (slots 2, 3) -> sc[2]; x = h + om*s;  r = s - om*t;
-// partials of r.r into slot 4 and of rhat.r into slot 0
+// partials of r.r into slot 4 and of rhat.r into slot 0; those of r.r also to
+// host[(iteration % 2)*kDotBlocks ...] (host memory), the iterations counted
+// from 1
 hipError_t launch_bicg_xr(const double* h, const double* sv, const double* t, const double* rhat,
-                          double* sc, double* part, double* x, double* r, size_t n, hipStream_t s);
+                          double* sc, double* part, double* x, double* r, double* host, size_t n,
+                          hipStream_t s);
+// r.r from one half of `host`, as launch_bicg_p sums it (host code)
+double residual_of_partials(const double* host);
+// launch_remove_mean of Sf's pressure rows (Sf + 3nb) and the dots of the
+// result: <a, Sf> into slot and, if two, <Sf, Sf> into slot + 1
+hipError_t launch_mean_dot(const Markers& m, double* Sf, const double* coef, const double* pj,
+                           const double* a, bool two, double* mpart, double* part, int slot,
+                           hipStream_t s);
 // r = b - r (b == null: r unchanged); rhat = r; p = v = 0
 hipError_t launch_bicg_init(const double* b, double* r, double* rhat, double* p, double* v,
                             size_t n, hipStream_t s);
