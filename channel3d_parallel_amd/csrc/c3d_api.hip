@@ -2612,50 +2612,49 @@ int c3d_mlp_train(c3d_ctx* c, const float* X, const float* T, int n, int epochs,
   const int nbatch = n / batch;
   if (nbatch == 0) return fail(c, C3D_EINVAL, "fewer samples than one batch");
   if ((rc = mlp_reserve(c, n > batch ? n : batch))) return rc;
-  // shuffled copies of the data set, uploaded per epoch into the staging rows
-  float *DX = nullptr, *DT = nullptr;
-  if (hipMalloc(&DX, (size_t)n * N::kIn * 4) != hipSuccess ||
-      hipMalloc(&DT, (size_t)n * N::kOut * 4) != hipSuccess) {
+  // the data set as given, its rows in an epoch's order, and that order: the
+  // set is uploaded once and reordered on the device
+  float* dev = nullptr;
+  const size_t nx = (size_t)n * N::kIn, nt = (size_t)n * N::kOut;
+  if (hipMalloc(&dev, (2 * (nx + nt) + (size_t)n) * 4) != hipSuccess) {
     (void)hipGetLastError();  // the launchers report hipGetLastError()
-    if (DX) (void)hipFree(DX);
     return fail(c, C3D_ENOMEM, "training set buffers");
   }
+  // the epoch's rows first: 16-byte aligned batches of targets and inputs
+  float *DT = dev, *DX = DT + nt, *RX = DX + nx, *RT = RX + nx;
+  int* didx = reinterpret_cast<int*>(RT + nt);
   std::vector<int> perm(n);
   for (int i = 0; i < n; i++) perm[i] = i;
-  std::vector<float> hx((size_t)n * N::kIn), ht((size_t)n * N::kOut);
+  if (hipMemcpyAsync(RX, X, nx * 4, hipMemcpyHostToDevice, c->stream) != hipSuccess ||
+      hipMemcpyAsync(RT, T, nt * 4, hipMemcpyHostToDevice, c->stream) != hipSuccess)
+    rc = fail(c, C3D_EHIP, "training upload");
   uint64_t st = seed;
   const float b1 = 0.9f, b2 = 0.999f, eps = 1e-8f;
   for (int e = 0; e < epochs && !rc; e++) {
+    // without the loss read-back of the epoch before: its order may still be
+    // on the way to the device
+    if (e > 0 && !loss_hist && (rc = sync(c))) break;
     for (int i = n - 1; i > 0; i--) std::swap(perm[i], perm[(int)(splitmix(st) % (uint64_t)(i + 1))]);
-    for (int i = 0; i < n; i++) {
-      std::memcpy(&hx[(size_t)i * N::kIn], &X[(size_t)perm[i] * N::kIn], N::kIn * 4);
-      std::memcpy(&ht[(size_t)i * N::kOut], &T[(size_t)perm[i] * N::kOut], N::kOut * 4);
-    }
-    if (hipMemcpyAsync(DX, hx.data(), hx.size() * 4, hipMemcpyHostToDevice, c->stream) != hipSuccess ||
-        hipMemcpyAsync(DT, ht.data(), ht.size() * 4, hipMemcpyHostToDevice, c->stream) != hipSuccess) {
-      rc = fail(c, C3D_EHIP, "training upload");
+    if (hipMemcpyAsync(didx, perm.data(), (size_t)n * 4, hipMemcpyHostToDevice, c->stream) != hipSuccess ||
+        N::shuffle(n, didx, RX, RT, DX, DT, c->stream) != hipSuccess) {
+      rc = fail(c, C3D_EHIP, "training set order");
       break;
     }
     for (int b = 0; b < nbatch && !rc; b++) {
-      if (hipMemcpyAsync(m->X, DX + (size_t)b * batch * N::kIn, (size_t)batch * N::kIn * 4,
-                         hipMemcpyDeviceToDevice, c->stream) != hipSuccess ||
-          hipMemcpyAsync(m->T, DT + (size_t)b * batch * N::kOut, (size_t)batch * N::kOut * 4,
-                         hipMemcpyDeviceToDevice, c->stream) != hipSuccess) {
-        rc = fail(c, C3D_EHIP, "batch copy");
+      const float *bX = DX + (size_t)b * batch * N::kIn, *bT = DT + (size_t)b * batch * N::kOut;
+      if (N::forward_grad(m->L, m->P, bX, bT, batch, m->act, m->dY, c->stream) != hipSuccess ||
+          N::backward(m->L, m->P, bX, batch, m->act, m->dY, m->dH, m->G, c->stream) != hipSuccess) {
+        rc = fail(c, C3D_EHIP, "training step");
         break;
       }
-      rc = mlp_loss_grad_launch(c, batch, nullptr);
-      if (rc) break;
       m->t++;
       const float lr_t = lr * std::sqrt(1.f - std::pow(b2, (float)m->t)) / (1.f - std::pow(b1, (float)m->t));
       if (N::adam(m->P, m->G, m->M, m->V, m->L.total, lr_t, b1, b2, eps, c->stream) != hipSuccess)
         rc = fail(c, C3D_EHIP, "adam");
     }
     if (!rc && loss_hist) {  // full-set loss after the epoch
-      if (hipMemcpyAsync(m->X, DX, (size_t)n * N::kIn * 4, hipMemcpyDeviceToDevice, c->stream) != hipSuccess ||
-          hipMemcpyAsync(m->T, DT, (size_t)n * N::kOut * 4, hipMemcpyDeviceToDevice, c->stream) != hipSuccess ||
-          N::forward(m->L, m->P, m->X, n, m->act, c->stream) != hipSuccess ||
-          N::loss_grad(m->act[N::kLayers - 1], m->T, n, m->dY, m->part, c->stream) != hipSuccess) {
+      if (N::forward(m->L, m->P, DX, n, m->act, c->stream) != hipSuccess ||
+          N::loss_grad(m->act[N::kLayers - 1], DT, n, m->dY, m->part, c->stream) != hipSuccess) {
         rc = fail(c, C3D_EHIP, "epoch loss");
         break;
       }
@@ -2671,8 +2670,7 @@ int c3d_mlp_train(c3d_ctx* c, const float* X, const float* T, int n, int epochs,
     }
   }
   (void)hipStreamSynchronize(c->stream);
-  (void)hipFree(DX);
-  (void)hipFree(DT);
+  (void)hipFree(dev);
   if (!rc) m->ready = true;
   return rc;
 }

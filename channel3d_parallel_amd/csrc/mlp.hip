@@ -35,7 +35,9 @@ __device__ __forceinline__ short bf16_bits(float x) {
 //   op(A)(m,k) = TA ? A[k*lda + m] : A[m*lda + k]
 //   op(B)(k,n) = TB ? B[n*ldb + k] : B[k*ldb + n]
 // Epilogues: kEpiNone, kEpiBias (+bias[n]), kEpiBiasRelu, kEpiMask
-// (C *= (H(m,n) > 0), the ReLU derivative of the forward activation H).
+// (C *= (H(m,n) > 0), the ReLU derivative of the forward activation H),
+// kEpiMse (+bias[n], then the mean-squared error's gradient against the
+// targets H: C = 2 (C - H) scale).
 //
 // A workgroup computes a T x T tile of C (T = 64, or 32 for products too
 // small to give every CU a 64 x 64 tile); its 4 wavefronts each own a
@@ -111,17 +113,38 @@ struct Slice {
   }
 };
 
+struct Gemm {
+  int M, N, K;
+  const float* A;
+  int lda;
+  const float* B;
+  int ldb;
+  float* C;
+  int ldc;
+  const float* bias;
+  const float* H;
+  int ldh;
+  float scale;
+};
+
+// LDS of a workgroup's two slices.
+template <int T>
+struct Slices {
+  __align__(16) short a[T * kTKP], b[T * kTKP];
+};
+
 template <bool TA, bool TB, int EPI, int T, bool VA, bool VB>
-__global__ __launch_bounds__(kBlock) void k_gemm(int M, int N, int K, const float* __restrict__ A,
-                                                 int lda, const float* __restrict__ B, int ldb,
-                                                 float* __restrict__ C, int ldc,
-                                                 const float* __restrict__ bias,
-                                                 const float* __restrict__ H, int ldh) {
+__device__ __forceinline__ void gemm_block(const Gemm& q_, Slices<T>& lds, int bx, int by) {
+  const int M = q_.M, N = q_.N, K = q_.K, lda = q_.lda, ldb = q_.ldb, ldc = q_.ldc, ldh = q_.ldh;
+  const float* __restrict__ A = q_.A;
+  const float* __restrict__ B = q_.B;
+  float* __restrict__ C = q_.C;
+  const float* __restrict__ bias = q_.bias;
+  const float* __restrict__ H = q_.H;
   constexpr int F = T / 32;  // MFMA tiles per wavefront along m and along n
-  __shared__ __align__(16) short As[T * kTKP];
-  __shared__ __align__(16) short Bs[T * kTKP];
+  short *As = lds.a, *Bs = lds.b;
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
-  const int m0 = blockIdx.x * T, n0 = blockIdx.y * T;
+  const int m0 = bx * T, n0 = by * T;
   const int wm = (wave >> 1) * (T / 2), wn = (wave & 1) * (T / 2);
   const int r = lane & 15, q = lane >> 4;
   float4_t acc[F][F];
@@ -167,12 +190,22 @@ __global__ __launch_bounds__(kBlock) void k_gemm(int M, int N, int K, const floa
         const int m = m0 + wm + 16 * i + 4 * q + e, n = n0 + wn + 16 * j + r;
         if (m < M && n < N) {
           float v = acc[i][j][e];
-          if (EPI == kEpiBias || EPI == kEpiBiasRelu) v += bias[n];
+          if (EPI == kEpiBias || EPI == kEpiBiasRelu || EPI == kEpiMse) v += bias[n];
           if (EPI == kEpiBiasRelu) v = fmaxf(v, 0.f);
           if (EPI == kEpiMask) v = (H[(size_t)m * ldh + n] > 0.f) ? v : 0.f;
+          if (EPI == kEpiMse) {
+            const float d = v - H[(size_t)m * ldh + n];
+            v = 2.f * d * q_.scale;
+          }
           C[(size_t)m * ldc + n] = v;
         }
       }
+}
+
+template <bool TA, bool TB, int EPI, int T, bool VA, bool VB>
+__global__ __launch_bounds__(kBlock) void k_gemm(Gemm q) {
+  __shared__ Slices<T> lds;
+  gemm_block<TA, TB, EPI, T, VA, VB>(q, lds, blockIdx.x, blockIdx.y);
 }
 
 // Mean-squared error over n x 4 outputs: dY = 2 (Y - T) / (4n); per-block
@@ -202,14 +235,15 @@ __global__ __launch_bounds__(kBlock) void k_mse(const float* __restrict__ Y, con
 // ... (consecutive lanes read consecutive columns), then the slices are
 // added pairwise in LDS.
 constexpr int kColN = 16, kColR = kBlock / kColN;
-__global__ __launch_bounds__(kBlock) void k_colsum(const float* __restrict__ dY, int M, int N,
-                                                   float* __restrict__ db) {
-  __shared__ float sh[kColR][kColN];
+__device__ __forceinline__ void colsum_block(const float* __restrict__ dY, int M, int N,
+                                             float* __restrict__ db, float (*sh)[kColN], int bx) {
   const int c = threadIdx.x % kColN, r = threadIdx.x / kColN;
-  const int n = blockIdx.x * kColN + c;
+  const int n = bx * kColN + c;
   float s = 0.f;
-  if (n < N)
+  if (n < N) {
+#pragma unroll 4
     for (int m = r; m < M; m += kColR) s += dY[(size_t)m * N + n];
+  }
   sh[r][c] = s;
   __syncthreads();
   for (int h = kColR / 2; h > 0; h >>= 1) {
@@ -217,6 +251,46 @@ __global__ __launch_bounds__(kBlock) void k_colsum(const float* __restrict__ dY,
     __syncthreads();
   }
   if (r == 0 && n < N) db[n] = sh[0][c];
+}
+
+// Everything that one layer's backward step derives from its dL/d(output) d:
+// the input's gradient (dgrad, TD x TD tiles, none for the first layer), the
+// weights' gradient (wgrad, 32 x 32 tiles) and the bias' (colsum), side by side
+// in one launch: each is a few dozen workgroups (a batch of 256 through a
+// 256 x 256 layer: 64, 64 and 16 for 256 CUs) and took a launch of 4 to 6 us.
+// WV: the layer's input is read as float4.
+template <bool WV, int TD, bool DGRAD>
+__global__ __launch_bounds__(kBlock) void k_backward(Gemm dg, Gemm wg, float* __restrict__ db, int nd,
+                                                     int nw) {
+  __shared__ union {
+    Slices<TD> d;
+    Slices<32> w;
+    float c[kColR][kColN];
+  } lds;
+  int b = blockIdx.x;
+  if (DGRAD && b < nd) {
+    const int gx = (dg.M + TD - 1) / TD;
+    gemm_block<false, false, kEpiMask, TD, true, true>(dg, lds.d, b % gx, b / gx);
+    return;
+  }
+  b -= nd;
+  if (b < nw) {
+    const int gx = (wg.M + 31) / 32;
+    gemm_block<true, false, kEpiNone, 32, true, WV>(wg, lds.w, b % gx, b / gx);
+    return;
+  }
+  colsum_block(wg.A, wg.K, wg.M, db, lds.c, b - nw);
+}
+
+// Rows idx[r] of the data set (X n x 54, T n x 4) in the order of an epoch.
+__global__ void k_shuffle(int n, const int* __restrict__ idx, const float* __restrict__ X,
+                          const float* __restrict__ T, float* __restrict__ Xs, float* __restrict__ Ts) {
+  constexpr int kRow = kIn + kOut;
+  const size_t e = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (e >= (size_t)n * kRow) return;
+  const int r = (int)(e / kRow), c = (int)(e - (size_t)r * kRow), o = idx[r];
+  if (c < kIn) Xs[(size_t)r * kIn + c] = X[(size_t)o * kIn + c];
+  else Ts[(size_t)r * kOut + c - kIn] = T[(size_t)o * kOut + c - kIn];
 }
 
 // Adam (FP32), bias-corrected step size lr_t passed in.
@@ -262,37 +336,39 @@ __global__ void k_apply(int nb, const float* __restrict__ Y, const float* __rest
 }
 
 template <bool TA, bool TB, int EPI, int T>
-hipError_t gemm_tile(int M, int N, int K, const float* A, int lda, const float* B, int ldb,
-                     float* C, int ldc, const float* bias, const float* H, int ldh, hipStream_t s) {
+hipError_t gemm_tile(const Gemm& q, hipStream_t s) {
   // float4 operand loads: the contiguous extent and the leading dimension
   // multiples of 4, the base 16-byte aligned
   auto al = [](const float* p) { return ((uintptr_t)p & 15) == 0; };
-  const bool va = al(A) && lda % 4 == 0 && (TA ? M : K) % 4 == 0;
-  const bool vb = al(B) && ldb % 4 == 0 && (TB ? K : N) % 4 == 0;
-  const dim3 grid((M + T - 1) / T, (N + T - 1) / T);
-  if (va && vb)
-    hipLaunchKernelGGL((k_gemm<TA, TB, EPI, T, true, true>), grid, dim3(kBlock), 0, s, M, N, K, A,
-                       lda, B, ldb, C, ldc, bias, H, ldh);
-  else if (vb)
-    hipLaunchKernelGGL((k_gemm<TA, TB, EPI, T, false, true>), grid, dim3(kBlock), 0, s, M, N, K, A,
-                       lda, B, ldb, C, ldc, bias, H, ldh);
-  else if (va)
-    hipLaunchKernelGGL((k_gemm<TA, TB, EPI, T, true, false>), grid, dim3(kBlock), 0, s, M, N, K, A,
-                       lda, B, ldb, C, ldc, bias, H, ldh);
-  else
-    hipLaunchKernelGGL((k_gemm<TA, TB, EPI, T, false, false>), grid, dim3(kBlock), 0, s, M, N, K, A,
-                       lda, B, ldb, C, ldc, bias, H, ldh);
+  const bool va = al(q.A) && q.lda % 4 == 0 && (TA ? q.M : q.K) % 4 == 0;
+  const bool vb = al(q.B) && q.ldb % 4 == 0 && (TB ? q.K : q.N) % 4 == 0;
+  const dim3 grid((q.M + T - 1) / T, (q.N + T - 1) / T);
+  if (va && vb) hipLaunchKernelGGL((k_gemm<TA, TB, EPI, T, true, true>), grid, dim3(kBlock), 0, s, q);
+  else if (vb) hipLaunchKernelGGL((k_gemm<TA, TB, EPI, T, false, true>), grid, dim3(kBlock), 0, s, q);
+  else if (va) hipLaunchKernelGGL((k_gemm<TA, TB, EPI, T, true, false>), grid, dim3(kBlock), 0, s, q);
+  else hipLaunchKernelGGL((k_gemm<TA, TB, EPI, T, false, false>), grid, dim3(kBlock), 0, s, q);
   return hipGetLastError();
 }
 
+// 64 x 64 tiles when they give at least one workgroup per CU (256), else
+// 32 x 32 (the training batches: 256 x 256 products)
+bool big_tiles(int M, int N) { return (long long)((M + 63) / 64) * ((N + 63) / 64) >= 256; }
+
 template <bool TA, bool TB, int EPI>
 hipError_t gemm(int M, int N, int K, const float* A, int lda, const float* B, int ldb, float* C,
-                int ldc, const float* bias, const float* H, int ldh, hipStream_t s) {
-  // 64 x 64 tiles when they give at least one workgroup per CU (256), else
-  // 32 x 32 (the training batches: 256 x 256 products)
-  const long long big = (long long)((M + 63) / 64) * ((N + 63) / 64);
-  if (big >= 256) return gemm_tile<TA, TB, EPI, 64>(M, N, K, A, lda, B, ldb, C, ldc, bias, H, ldh, s);
-  return gemm_tile<TA, TB, EPI, 32>(M, N, K, A, lda, B, ldb, C, ldc, bias, H, ldh, s);
+                int ldc, const float* bias, const float* H, int ldh, hipStream_t s, float scale = 0.f) {
+  const Gemm q{M, N, K, A, lda, B, ldb, C, ldc, bias, H, ldh, scale};
+  return big_tiles(M, N) ? gemm_tile<TA, TB, EPI, 64>(q, s) : gemm_tile<TA, TB, EPI, 32>(q, s);
+}
+
+template <bool WV, int TD>
+void backward_layer(const Gemm& dg, const Gemm& wg, float* db, bool dgrad, hipStream_t s) {
+  const int nd = dgrad ? ((dg.M + TD - 1) / TD) * ((dg.N + TD - 1) / TD) : 0;
+  const int nw = ((wg.M + 31) / 32) * ((wg.N + 31) / 32), nc = (wg.M + kColN - 1) / kColN;
+  if (dgrad)
+    hipLaunchKernelGGL((k_backward<WV, TD, true>), dim3(nd + nw + nc), dim3(kBlock), 0, s, dg, wg, db, nd, nw);
+  else
+    hipLaunchKernelGGL((k_backward<WV, TD, false>), dim3(nd + nw + nc), dim3(kBlock), 0, s, dg, wg, db, nd, nw);
 }
 
 }  // namespace
@@ -313,21 +389,39 @@ Layout layout() {
   return L;
 }
 
+namespace {
+hipError_t layer_forward(const Layout& L, const float* P, const float* in, int n, int i, float* out,
+                         hipStream_t s) {
+  if (i < kLayers - 1)
+    return gemm<false, true, kEpiBiasRelu>(n, L.out[i], L.in[i], in, L.in[i], P + L.w[i], L.in[i], out,
+                                           L.out[i], P + L.b[i], nullptr, 0, s);
+  return gemm<false, true, kEpiBias>(n, L.out[i], L.in[i], in, L.in[i], P + L.w[i], L.in[i], out,
+                                     L.out[i], P + L.b[i], nullptr, 0, s);
+}
+}  // namespace
+
 hipError_t forward(const Layout& L, const float* P, const float* X, int n, float* const act[kLayers],
                    hipStream_t s) {
   const float* in = X;
   for (int i = 0; i < kLayers; i++) {
-    hipError_t e;
-    if (i < kLayers - 1)
-      e = gemm<false, true, kEpiBiasRelu>(n, L.out[i], L.in[i], in, L.in[i], P + L.w[i], L.in[i],
-                                          act[i], L.out[i], P + L.b[i], nullptr, 0, s);
-    else
-      e = gemm<false, true, kEpiBias>(n, L.out[i], L.in[i], in, L.in[i], P + L.w[i], L.in[i],
-                                      act[i], L.out[i], P + L.b[i], nullptr, 0, s);
+    const hipError_t e = layer_forward(L, P, in, n, i, act[i], s);
     if (e != hipSuccess) return e;
     in = act[i];
   }
   return hipSuccess;
+}
+
+hipError_t forward_grad(const Layout& L, const float* P, const float* X, const float* T, int n,
+                        float* const act[kLayers], float* dY, hipStream_t s) {
+  const float* in = X;
+  for (int i = 0; i < kLayers - 1; i++) {
+    const hipError_t e = layer_forward(L, P, in, n, i, act[i], s);
+    if (e != hipSuccess) return e;
+    in = act[i];
+  }
+  constexpr int i = kLayers - 1;
+  return gemm<false, true, kEpiMse>(n, L.out[i], L.in[i], in, L.in[i], P + L.w[i], L.in[i], dY, L.out[i],
+                                    P + L.b[i], T, kOut, s, 1.f / (float)(n * kOut));
 }
 
 hipError_t loss_grad(const float* Y, const float* T, int n, float* dY, float* part, hipStream_t s) {
@@ -338,22 +432,31 @@ hipError_t loss_grad(const float* Y, const float* T, int n, float* dY, float* pa
 hipError_t backward(const Layout& L, const float* P, const float* X, int n,
                     float* const act[kLayers], float* dY, float* const dH[kLayers - 1], float* G,
                     hipStream_t s) {
-  // layer i maps act[i-1] (X for i = 0) to act[i]; d holds dL/d(pre-activation)
+  // layer i maps act[i-1] (X for i = 0) to act[i]; d holds dL/d(pre-activation).
+  // d, the weights and the hidden activations have widths of 4 or 256 and
+  // 16-byte aligned bases: float4 loads; the first layer's input (54) has not.
   const float* d = dY;
   for (int i = kLayers - 1; i >= 0; i--) {
-    const float* in = (i == 0) ? X : act[i - 1];
-    hipError_t e = gemm<true, false, kEpiNone>(L.out[i], L.in[i], n, d, L.out[i], in, L.in[i],
-                                               G + L.w[i], L.in[i], nullptr, nullptr, 0, s);
+    const bool dgrad = i > 0;
+    const float* in = dgrad ? act[i - 1] : X;
+    const Gemm wg{L.out[i], L.in[i], n, d, L.out[i], in, L.in[i], G + L.w[i], L.in[i], nullptr, nullptr, 0, 0.f};
+    const Gemm dg{n, L.in[i], L.out[i], d, L.out[i], P + L.w[i], L.in[i], dgrad ? dH[i - 1] : nullptr,
+                  L.in[i], nullptr, dgrad ? act[i - 1] : nullptr, L.in[i], 0.f};
+    if (!dgrad) backward_layer<false, 32>(dg, wg, G + L.b[i], false, s);
+    else if (big_tiles(n, L.in[i])) backward_layer<true, 64>(dg, wg, G + L.b[i], true, s);
+    else backward_layer<true, 32>(dg, wg, G + L.b[i], true, s);
+    const hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
-    hipLaunchKernelGGL(k_colsum, dim3((L.out[i] + kColN - 1) / kColN), dim3(kBlock), 0, s, d, n,
-                       L.out[i], G + L.b[i]);
-    if (i > 0) {
-      e = gemm<false, false, kEpiMask>(n, L.in[i], L.out[i], d, L.out[i], P + L.w[i], L.in[i],
-                                       dH[i - 1], L.in[i], nullptr, act[i - 1], L.in[i], s);
-      if (e != hipSuccess) return e;
-      d = dH[i - 1];
-    }
+    if (dgrad) d = dH[i - 1];
   }
+  return hipSuccess;
+}
+
+hipError_t shuffle(int n, const int* idx, const float* X, const float* T, float* Xs, float* Ts,
+                   hipStream_t s) {
+  const size_t e = (size_t)n * (kIn + kOut);
+  hipLaunchKernelGGL(k_shuffle, dim3((unsigned)((e + kBlock - 1) / kBlock)), dim3(kBlock), 0, s, n, idx, X,
+                     T, Xs, Ts);
   return hipGetLastError();
 }
 

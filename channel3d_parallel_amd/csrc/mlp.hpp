@@ -15,7 +15,7 @@ constexpr int kOut = 4;          // dudn_x, dudn_y, dudn_z, p_jump
 constexpr int kLayers = 4;
 constexpr int kLossBlocks = 64;
 
-constexpr int kEpiNone = 0, kEpiBias = 1, kEpiBiasRelu = 2, kEpiMask = 3;
+constexpr int kEpiNone = 0, kEpiBias = 1, kEpiBiasRelu = 2, kEpiMask = 3, kEpiMse = 4;
 
 struct Layout {
   int w[kLayers], b[kLayers], in[kLayers], out[kLayers];
@@ -25,6 +25,13 @@ Layout layout();
 
 // act[i] (n x out_i) = relu(act[i-1] W_i^T + b_i), the last layer linear.
 hipError_t forward(const Layout& L, const float* P, const float* X, int n, float* const act[kLayers],
+                   hipStream_t s);
+// forward with the last layer's output replaced by dY = dMSE/dY against T (as
+// loss_grad gives it; act[kLayers - 1] is not written).
+hipError_t forward_grad(const Layout& L, const float* P, const float* X, const float* T, int n,
+                        float* const act[kLayers], float* dY, hipStream_t s);
+// Xs, Ts = rows idx[0 .. n) of X (n x 54) and T (n x 4).
+hipError_t shuffle(int n, const int* idx, const float* X, const float* T, float* Xs, float* Ts,
                    hipStream_t s);
 // dY = dMSE/dY over n x 4, per-block loss partials (kLossBlocks).
 hipError_t loss_grad(const float* Y, const float* T, int n, float* dY, float* part, hipStream_t s);
