@@ -13,7 +13,7 @@
 #include "kernels.hpp"
 
 #pragma clang fp contract(off)
-#include "rk3_point.hpp"
+#include "rk3_march.hpp"
 
 namespace c3d {
 
@@ -27,12 +27,7 @@ constexpr int kB = 256;
 
 // compute_rhs_u/v/w evaluated together.  Ranges: F_u (2:nx-1, 2:nyg-1,
 // 2:nzg-1), F_v (2:nxg-1, 2:ny-1, 2:nzg-1), F_w (2:nxg-1, 2:nyg-1, 2:nz-1);
-// the grid covers their union.  Each workgroup owns a 64 x 4 column of
-// points and marches KC z planes; U, V, W around it are staged in LDS as a
-// ring of three planes with a one-cell x/y halo, so every neighbour read of
-// the point functions is an LDS read and each field value is fetched from
-// HBM about once.  Out-of-array halo cells are zero and only feed outputs
-// outside the ranges above.
+// the grid covers their union, walked plane by plane (rk3_march.hpp).
 template <int KC>
 __global__ __launch_bounds__(kB) void k_rhs(DevGrid g, const double* __restrict__ U,
                                             const double* __restrict__ V,
@@ -42,44 +37,15 @@ __global__ __launch_bounds__(kB) void k_rhs(DevGrid g, const double* __restrict_
                                             const double* __restrict__ Hw, double nu, double dPdx,
                                             double dPdy, double dPdz, double* __restrict__ Fu,
                                             double* __restrict__ Fv, double* __restrict__ Fw) {
-  __shared__ double tile[3 * 3 * kTP];
-  __shared__ double xt[kXT * kTX];
-  unsigned bx, by, bz;
-  xcd_tile(bx, by, bz);  // neighbouring tiles on one XCD (shared halo rows)
-  const int i0 = bx * 64 + 2, j0 = by * 4 + 2, kb = bz * KC + 2;
-  // j is the same on all lanes of a wavefront (one row of 64 x positions)
-  const int i = i0 + (threadIdx.x & 63);
-  const int j = __builtin_amdgcn_readfirstlane(j0 + (int)(threadIdx.x >> 6));
-  const int nx = g.nx, ny = g.ny, nz = g.nz, nxg = g.nxg, nyg = g.nyg, nzg = g.nzg;
-  // LDS copy of the tile's x spacing factors (the same table values, so the
-  // result stays bitwise); the first plane's barrier makes it visible
-  for (int e = threadIdx.x; e < kXT * kTX; e += kB) {
-    const int t = e / kTX, ii = min(i0 - 1 + e % kTX, nx + 1);
-    const double* src = t == kXrdxg ? g.rdxg : t == kXrdxf ? g.rdxf : t == kXnudxf ? g.nudxf : g.nudxg;
-    xt[e] = src[ii];
-  }
-  TileAccX A{{tile, i0, j0, kb}, xt};
-  auto stage = [&](int k) { stage_tile_plane(g, U, V, W, tile, A, k, kB); };
-  stage(kb - 1);
-  stage(kb);
-  for (int kk = 0; kk < KC; kk++) {
-    const int k = kb + kk;
-    if (k > nzg - 1) break;  // uniform across the workgroup
-    stage(k + 1);
-    __syncthreads();
-    if (i <= nxg - 1 && j <= nyg - 1) {
-      if (i <= nx - 1)
-        Fu[(size_t)(i - 2) + (size_t)(nx - 2) * ((size_t)(j - 2) + (size_t)(nyg - 2) * (size_t)(k - 2))] =
-            rhs_u_at<false>(g, A, Hu, nu, dPdx, i, j, k);
-      if (j <= ny - 1)
-        Fv[(size_t)(i - 2) + (size_t)(nxg - 2) * ((size_t)(j - 2) + (size_t)(ny - 2) * (size_t)(k - 2))] =
-            rhs_v_at<false>(g, A, Hv, nu, dPdy, i, j, k);
-      if (k <= nz - 1)
-        Fw[(size_t)(i - 2) + (size_t)(nxg - 2) * ((size_t)(j - 2) + (size_t)(nyg - 2) * (size_t)(k - 2))] =
-            rhs_w_at<false>(g, A, Hw, nu, dPdz, i, j, k);
-    }
-    __syncthreads();  // plane k-1's slot is refilled next
-  }
+  auto put = [](double* F, double v, int k, const Spot& s) { cell(F + (size_t)(k - 2) * s.pf, s.f) = v; };
+  march<KC>(
+      g, U, V, W, [](int, const Spot&, const Spot&, const Spot&) {},
+      [&](const MarchAcc& A, const MarchGrid& G, int k, const Spot& su, const Spot& sv, const Spot& sw) {
+        const int i = A.i, j = A.j;
+        if (su.in) put(Fu, rhs_u_at<false>(G, A, Hu, nu, dPdx, i, j, k), k, su);
+        if (sv.in) put(Fv, rhs_v_at<false>(G, A, Hv, nu, dPdy, i, j, k), k, sv);
+        if (sw.in && k <= g.nz - 1) put(Fw, rhs_w_at<false>(G, A, Hw, nu, dPdz, i, j, k), k, sw);
+      });
 }
 
 // RK3 stage update on the interior of one component
