@@ -280,10 +280,11 @@ __device__ __forceinline__ double gather_pair(const DevGrid& g, const Markers& m
   const bool hi = lane >= 32;
   const int p = lane & 31;
   const bool on = p < 25 && (CB >= 0 || !hi);
-  const int i = on ? p % 5 : 0, j = on ? p / 5 : 0;
-  const size_t b = (size_t)l * kStencils;           // wave-uniform
-  const int ba = CA * kStencil;
-  const int bl = ba + (hi ? DS * kStencil : 0);     // this half's stencil
+  const int j = on ? p * 13 >> 6 : 0, i = on ? p - 5 * j : 0;  // p / 5, p % 5 (p < 25)
+  // the marker's tables (wave-uniform pointers) and this half's stencil in them
+  const int* im = idx + (size_t)l * kStencils + CA * kStencil;
+  const double* pm = phi + (size_t)l * kStencils + CA * kStencil;
+  const unsigned h = hi ? DS * kStencil : 0;
   // strides of the field (the centre field is rhs_p-shaped, first index 2)
   auto n1 = [&](int c) { return c == 0 ? g.nx : (c == 3 ? g.nxg - 2 : g.nxg); };
   auto n2 = [&](int c) { return c == 1 ? g.ny : (c == 3 ? g.nyg - 2 : g.nyg); };
@@ -291,14 +292,14 @@ __device__ __forceinline__ double gather_pair(const DevGrid& g, const Markers& m
   const int s2 = hi ? n1(C1) * n2(C1) : n1(CA) * n2(CA);
   const int first = (hi ? C1 : CA) == 3 ? 2 : 1;
   const double* F = hi && CB >= 0 ? FB : FA;
-  const int X = idx[b + bl + i], Y = idx[b + bl + 5 + j];
-  const double px = phi[b + bl + i], py = phi[b + bl + 5 + j];
+  const int X = im[h + (unsigned)i], Y = im[h + 5 + (unsigned)j];
+  const double px = pm[h + (unsigned)i], py = pm[h + 5 + (unsigned)j];
   int Z[5];
   double pz[5];
 #pragma unroll
   for (int k = 0; k < 5; k++) {
-    const int za = idx[b + ba + 10 + k], zb = idx[b + ba + DS * kStencil + 10 + k];
-    const double pa = phi[b + ba + 10 + k], pb = phi[b + ba + DS * kStencil + 10 + k];
+    const int za = im[10 + k], zb = im[DS * kStencil + 10 + k];
+    const double pa = pm[10 + k], pb = pm[DS * kStencil + 10 + k];
     Z[k] = hi ? zb : za;
     pz[k] = hi ? pb : pa;
   }
@@ -309,12 +310,13 @@ __device__ __forceinline__ double gather_pair(const DevGrid& g, const Markers& m
   const double wxy = (m.A * px) * py;
   double acc = 0.0;
   if (DA || DB) {
-    const double dx = dd[b + bl + i], dy = dd[b + bl + 5 + j];
+    const double* dm = dd + (size_t)l * kStencils + CA * kStencil;
+    const double dx = dm[h + (unsigned)i], dy = dm[h + 5 + (unsigned)j];
     const double nx = normals[l], ny = normals[m.nb + l], nz = normals[2 * (size_t)m.nb + l];
     const double dxy = nx * dx + ny * dy;
 #pragma unroll
     for (int k = 0; k < 5; k++) {
-      const double da = dd[b + ba + 10 + k], db = dd[b + ba + DS * kStencil + 10 + k];
+      const double da = dm[10 + k], db = dm[DS * kStencil + 10 + k];
       const double v = (wxy * pz[k]) * f[k];
       const double vd = v * (dxy + nz * (hi ? db : da));
       acc += (hi ? DB : DA) ? vd : v;
@@ -452,18 +454,45 @@ __global__ void k_spread_coeffs(int nb, double A, double factor, const double* _
   sp.wfs[e] = w * factor * sb[l];
 }
 
+// entries per batch (16: 29.4 against 26.7 us per spreading of two cylinders'
+// 24,576 markers; 8 with each batch's loads waited for: 30.7 us)
+constexpr int kSpreadB = 8;
+
 // R, src/immersed_boundary_operators.f90:544-603: one thread per support node,
 // contributions in ascending marker order.
 __device__ __forceinline__ void spread_node(const Spread& sp, int t, const double* __restrict__ f,
                                             double* __restrict__ F) {
   double acc = 0.0;
   const int n = sp.cnt[t];
-  // loads of several entries in flight (8 measured 1% faster than 4 per
-  // BiCGSTAB iteration); the sum stays in entry order
-#pragma unroll 8
-  for (int i = 0; i < n; i++) {
-    const int e = sp.slot[i] + t;
-    acc = acc + sp.wfs[e] * f[sp.ml[e]];
+  // The lanes of a wavefront walk the entries together, up to the largest
+  // count (the first lane's: ranks descend in it); a lane past its own count
+  // reads its first entry and does not add it.  The next batch's coefficients
+  // and markers load while this batch's forces are gathered: a node has up to
+  // about 100 entries, and the few wavefronts of the longest lists, which run
+  // alone in the end, waited for both in turn.  The sum stays in entry order.
+  const int nmax = __builtin_amdgcn_readfirstlane(n);
+  int ml[kSpreadB];
+  double wf[kSpreadB];
+  auto load = [&](int i0) {
+#pragma unroll
+    for (int r = 0; r < kSpreadB; r++) {
+      const int i = i0 + r;
+      const int e = i < n ? sp.slot[min(i, nmax - 1)] + t : t;
+      ml[r] = sp.ml[e];
+      wf[r] = sp.wfs[e];
+    }
+  };
+  load(0);
+  for (int i0 = 0; i0 < nmax; i0 += kSpreadB) {
+    double fv[kSpreadB], wc[kSpreadB];
+#pragma unroll
+    for (int r = 0; r < kSpreadB; r++) {
+      fv[r] = f[ml[r]];
+      wc[r] = wf[r];
+    }
+    if (i0 + kSpreadB < nmax) load(i0 + kSpreadB);
+#pragma unroll
+    for (int r = 0; r < kSpreadB; r++) acc = i0 + r < n ? acc + wc[r] * fv[r] : acc;
   }
   F[sp.node[t]] = acc;
 }
