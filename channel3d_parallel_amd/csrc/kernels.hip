@@ -623,13 +623,30 @@ __global__ __launch_bounds__(kBlock) void k_grad_correct(DevGrid g, double* __re
     if constexpr (SPLIT) return (a - b) + (ac - bc);
     else return a - b;
   };
-  double pc;
-  double p = pot(ridx(i, j, kb, nxg, nyg), pc);
+  // All planes' loads are in flight before the first value is stored (planes
+  // past the end and the row past the wall read clamped cells, not used):
+  // with each plane's loads after the stores of the plane before it, and
+  // behind its branches, a lane waited for memory once per plane and field.
+  const int kend = BC ? nz - 1 : nzg - 1;
+  const int jv = min(j, ny - 1), jp = min(j + 1, nyg - 1);
+  double pz[KC + 1], pzc[KC + 1], pxe[KC], pxce[KC], py[KC], pyc[KC], uo[KC], vo[KC], wo[KC];
+  pz[0] = pot(ridx(i, j, kb, nxg, nyg), pzc[0]);
+#pragma unroll
+  for (int kk = 0; kk < KC; kk++) {
+    const int k = min(kb + kk, kend);
+    pz[kk + 1] = pot(ridx(i, j, k + 1, nxg, nyg), pzc[kk + 1]);
+    pxe[kk] = pot(ridx(ie + 1, j, k, nxg, nyg), pxce[kk]);
+    py[kk] = pot(ridx(i, jp, k, nxg, nyg), pyc[kk]);
+    uo[kk] = U[fidx(i, j, k, nx, nyg)];
+    vo[kk] = V[fidx(i, jv, k, nxg, ny)];
+    wo[kk] = W[fidx(i, j, min(k, nz), nxg, nyg)];
+  }
   bool bad = false;
 #pragma unroll
   for (int kk = 0; kk < KC; kk++) {
     const int k = kb + kk;
-    if (k > (BC ? nz - 1 : nzg - 1)) break;
+    if (k > kend) break;
+    const double p = pz[kk], pc = pzc[kk];
     if constexpr (SPLIT) {
       const double o = (p + pc) / dt;
       pout[ridx(i, j, k, nxg, nyg)] = o;
@@ -647,34 +664,23 @@ __global__ __launch_bounds__(kBlock) void k_grad_correct(DevGrid g, double* __re
     }
     const double pxn = wave_shl1(p);
     const double pxcn = SPLIT ? wave_shl1(pc) : 0.0;
-    double pxce;
-    const double pxe = pot(ridx(ie + 1, j, k, nxg, nyg), pxce);
-    const double px = (i == ie) ? pxe : pxn;
-    const double pxc = (i == ie) ? pxce : pxcn;
-    const size_t iu = fidx(i, j, k, nx, nyg);
-    const double u = U[iu] - dif(px, pxc, p, pc) / hx;
+    const double px = (i == ie) ? pxe[kk] : pxn;
+    const double pxc = (i == ie) ? pxce[kk] : pxcn;
+    const double u = uo[kk] - dif(px, pxc, p, pc) / hx;
     if constexpr (BC) put_u(g, U, i, j, k, u);
-    else U[iu] = u;
+    else U[fidx(i, j, k, nx, nyg)] = u;
     bad |= !isfinite(u);
     if (j <= ny - 1) {
-      double pyc;
-      const double py = pot(ridx(i, j + 1, k, nxg, nyg), pyc);
-      const size_t iv = fidx(i, j, k, nxg, ny);
-      const double v = V[iv] - dif(py, pyc, p, pc) / hy;
+      const double v = vo[kk] - dif(py[kk], pyc[kk], p, pc) / hy;
       if constexpr (BC) put_v(g, V, i, j, k, v);
-      else V[iv] = v;
+      else V[fidx(i, j, k, nxg, ny)] = v;
       bad |= !isfinite(v);
     }
     if (k <= nz - 1) {
-      double pzc;
-      const double pz = pot(ridx(i, j, k + 1, nxg, nyg), pzc);
-      const size_t iw = fidx(i, j, k, nxg, nyg);
-      const double w = W[iw] - dif(pz, pzc, p, pc) / g.dzg[k];
+      const double w = wo[kk] - dif(pz[kk + 1], pzc[kk + 1], p, pc) / g.dzg[k];
       if constexpr (BC) put_w(g, W, i, j, k, w);
-      else W[iw] = w;
+      else W[fidx(i, j, k, nxg, nyg)] = w;
       bad |= !isfinite(w);
-      p = pz;
-      pc = pzc;
     }
   }
   if (bad && g.nonfinite) *g.nonfinite = 1u;  // every writer writes the same
@@ -1055,12 +1061,12 @@ hipError_t launch_inv_x32(const DevGrid& g, int mode, const cpx<float>* S, const
 // z planes per lane of the gradient correction (at 384x193x384, 2 measured
 // fastest for the single potential: 0.303 against 0.305 ms for 1, more
 // workgroups in flight; 4 for the two-part potential: 0.457 against
-// 0.468 ms for 2); C3D_GRAD_KC (1, 2, 4, 8, 16) overrides both (tuning knob).
+// 0.468 ms for 2); C3D_GRAD_KC (1, 2, 4) overrides both (tuning knob).
 static int grad_kc(bool split) {
   static const int forced = [] {
     const char* e = getenv("C3D_GRAD_KC");
     const int v = e ? atoi(e) : 0;
-    return (v == 1 || v == 2 || v == 4 || v == 8 || v == 16) ? v : 0;
+    return (v == 1 || v == 2 || v == 4) ? v : 0;
   }();
   return forced ? forced : (split ? kGradKCSplitDefault : kGradKCDefault);
 }
@@ -1080,8 +1086,6 @@ hipError_t grad_correct_any(const DevGrid& g, double* U, double* V, double* W, c
     C3D_GC_CASE(1)
     C3D_GC_CASE(2)
     C3D_GC_CASE(4)
-    C3D_GC_CASE(8)
-    C3D_GC_CASE(16)
 #undef C3D_GC_CASE
     default:
       return hipErrorInvalidValue;
