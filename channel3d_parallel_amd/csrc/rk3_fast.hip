@@ -26,7 +26,11 @@ constexpr double kC11 = 8.0 / 15.0, kC21 = 1.0 / 4.0, kC22 = 5.0 / 12.0, kC31 = 
 
 // Stages 2 and 3 also read the point's own words, the step-start velocity and
 // F1: loaded before the plane's barrier, used after its evaluation.
-template <int KC, int STAGE>
+// MASK: H masks (none otherwise: six pointers less to keep in scalar registers,
+// which stage 2 overflowed into 118 lane reads per plane).  96 to 104 VGPRs;
+// held to 96 (5 waves per SIMD), stages 2 and 3 reload from scratch and take
+// 903 and 731 instead of 817 and 667 us on 384x192x384 cells.
+template <int KC, int STAGE, bool MASK>
 __global__ __launch_bounds__(kBf) void k_rhs_stage(DevGrid g, RkStage a) {
   double xo[3] = {0.0, 0.0, 0.0}, f1[3] = {0.0, 0.0, 0.0};
   auto own = [&](int c, const double* Xo, const double* F1, int k, const Spot& s) {
@@ -54,13 +58,13 @@ __global__ __launch_bounds__(kBf) void k_rhs_stage(DevGrid g, RkStage a) {
         const int i = A.i, j = A.j;
         // U(2:nx-1, 2:nyg-1, 2:nzg-1)
         if (su.in)
-          put(0, a.Fu, a.Un, A.U(i, j, k), rhs_u_at<true>(G, A, a.Hu, a.nu, a.dPdx, i, j, k), k, su);
+          put(0, a.Fu, a.Un, A.U(i, j, k), rhs_u_at<true>(G, A, MASK ? a.Hu : nullptr, a.nu, a.dPdx, i, j, k), k, su);
         // V(2:nxg-1, 2:ny-1, 2:nzg-1)
         if (sv.in)
-          put(1, a.Fv, a.Vn, A.V(i, j, k), rhs_v_at<true>(G, A, a.Hv, a.nu, a.dPdy, i, j, k), k, sv);
+          put(1, a.Fv, a.Vn, A.V(i, j, k), rhs_v_at<true>(G, A, MASK ? a.Hv : nullptr, a.nu, a.dPdy, i, j, k), k, sv);
         // W(2:nxg-1, 2:nyg-1, 2:nz-1)
         if (sw.in && k <= g.nz - 1)
-          put(2, a.Fw, a.Wn, A.W(i, j, k), rhs_w_at<true>(G, A, a.Hw, a.nu, a.dPdz, i, j, k), k, sw);
+          put(2, a.Fw, a.Wn, A.W(i, j, k), rhs_w_at<true>(G, A, MASK ? a.Hw : nullptr, a.nu, a.dPdz, i, j, k), k, sw);
       });
 }
 
@@ -69,7 +73,10 @@ inline dim3 gpts_f(int ni, int nj, int nk) { return dim3((ni + 63) / 64, (nj + 3
 template <int STAGE, int KC>
 void launch_stage_kernel(const DevGrid& g, const RkStage& a, hipStream_t s) {
   const dim3 grid = gpts_f(g.nxg - 2, g.nyg - 2, (g.nzg - 2 + KC - 1) / KC);
-  hipLaunchKernelGGL((k_rhs_stage<KC, STAGE>), grid, dim3(kBf), 0, s, g, a);
+  if (a.Hu && a.Hv && a.Hw)
+    hipLaunchKernelGGL((k_rhs_stage<KC, STAGE, true>), grid, dim3(kBf), 0, s, g, a);
+  else
+    hipLaunchKernelGGL((k_rhs_stage<KC, STAGE, false>), grid, dim3(kBf), 0, s, g, a);
 }
 
 template <int KC>
