@@ -440,11 +440,27 @@ int sync(c3d_ctx* c) {
   return 0;
 }
 
-// The Poisson pipeline between the forward and the inverse x transforms.
-int spectral_core(c3d_ctx* c, const c3d::Planes* pl = nullptr) {
+// The halves of the Poisson pipeline: div(U, V, W) or rhs to its spectrum, and
+// the spectrum's solution to out (launch_fwd_x, launch_inv_x).
+int spectral_forward(c3d_ctx* c, bool from_uvw, const double* U, const double* V, const double* W,
+                     const double* rhs, bool per, const c3d::Planes* pl = nullptr) {
+  if (c3d::plane_fft(c->g)) {
+    HIPCHK(c, c3d::launch_fwd_plane(c->g, from_uvw, U, V, W, rhs, c->S, per, c->stream, pl));
+    return 0;
+  }
+  HIPCHK(c, c3d::launch_fwd_x(c->g, from_uvw, U, V, W, rhs, c->S, per, c->stream, pl));
   HIPCHK(c, c3d::launch_fft_z(c->g, -1, c->S, c->stream, pl));
+  return 0;
+}
+int spectral_inverse(c3d_ctx* c, int mode, double* out, double dt, bool rk1,
+                     const c3d::Planes* pl = nullptr) {
   HIPCHK(c, c3d::launch_tri(c->g, c->S, c->CP, c->stream, pl));
+  if (c3d::plane_fft(c->g)) {
+    HIPCHK(c, c3d::launch_inv_plane(c->g, mode, c->S, out, c->P, dt, rk1, c->stream, pl));
+    return 0;
+  }
   HIPCHK(c, c3d::launch_fft_z(c->g, +1, c->S, c->stream, pl));
+  HIPCHK(c, c3d::launch_inv_x(c->g, mode, c->S, out, c->P, dt, rk1, c->stream, pl));
   return 0;
 }
 
@@ -721,11 +737,9 @@ int c3d_solve_poisson_equation(c3d_ctx* c, double* rhs, int rk_step, double dt) 
   if (!c || !rhs) return C3D_EINVAL;
   if (rk_step == 1 && !(dt != 0.0)) return fail(c, C3D_EINVAL, "dt must be nonzero at rk_step 1");
   HIPCHK(c, hipMemcpyAsync(c->rhs, rhs, c->nr * 8, hipMemcpyHostToDevice, c->stream));
-  HIPCHK(c, c3d::launch_fwd_x(c->g, false, nullptr, nullptr, nullptr, c->rhs, c->S, false,
-                              c->stream));
-  int rc = spectral_core(c);
+  int rc = spectral_forward(c, false, nullptr, nullptr, nullptr, c->rhs, false);
+  if (!rc) rc = spectral_inverse(c, 0, c->rhs, dt, rk_step == 1);
   if (rc) return rc;
-  HIPCHK(c, c3d::launch_inv_x(c->g, 0, c->S, c->rhs, c->P, dt, rk_step == 1, c->stream));
   HIPCHK(c, hipMemcpyAsync(rhs, c->rhs, c->nr * 8, hipMemcpyDeviceToHost, c->stream));
   return sync(c);
 }
@@ -749,7 +763,14 @@ static int projection_launch(c3d_ctx* c, double dt, int rk_step, hipEvent_t* ev,
   const DevGrid& g = c->g;
   hipStream_t st = c->stream;
   if (ev) HIPCHK(c, hipEventRecord(ev[0], st));
-  if (!mixed && nref == 0) {
+  if (!mixed && nref == 0 && !ev) {
+    int rc = spectral_forward(c, true, c->U, c->V, c->W, nullptr, bc);
+    if (!rc) rc = spectral_inverse(c, 1, c->Pint, dt, rk1);
+    if (rc) return rc;
+    HIPCHK(c, c3d::launch_grad_correct(g, c->U, c->V, c->W, c->Pint, dt, bc, st));
+    return 0;
+  }
+  if (!mixed && nref == 0) {  // kernel by kernel, with an event after each
     HIPCHK(c, c3d::launch_fwd_x(g, true, c->U, c->V, c->W, nullptr, c->S, bc, st));
     if (ev) HIPCHK(c, hipEventRecord(ev[1], st));
     HIPCHK(c, c3d::launch_fft_z(g, -1, c->S, st));
@@ -1383,12 +1404,8 @@ static int ib_poisson_reg(c3d_ctx* c, double dt, int rk_step, bool rows = false)
   IBState* ib = c->ib;
   const bool rk1 = rk_step == 1;
   const c3d::Planes* pl = rows && !rk1 && ib->planes.n ? &ib->planes : nullptr;
-  HIPCHK(c, c3d::launch_fwd_x(c->g, true, ib->Ureg, ib->Vreg, ib->Wreg, nullptr, c->S, true,
-                              c->stream, pl));
-  int rc = spectral_core(c, pl);
-  if (rc) return rc;
-  HIPCHK(c, c3d::launch_inv_x(c->g, 1, c->S, ib->phi, c->P, dt, rk1, c->stream, pl));
-  return 0;
+  int rc = spectral_forward(c, true, ib->Ureg, ib->Vreg, ib->Wreg, nullptr, true, pl);
+  return rc ? rc : spectral_inverse(c, 1, ib->phi, dt, rk1, pl);
 }
 
 // U_reg = R f (src/projection.f90:66-73): aux, three spreads.  The boundary
@@ -1944,11 +1961,11 @@ int ib_heaviside(c3d_ctx* c) {
   ok = ok && c3d::launch_apply_bc(c->g, ib->Ureg, ib->Vreg, ib->Wreg, c->stream) == hipSuccess;
   ok = ok && c3d::launch_divergence(c->g, ib->Ureg, ib->Vreg, ib->Wreg, ib->Hc_ext, c->stream) == hipSuccess;
   ok = ok && B::launch_affine(ib->Hc_ext, -0.0, -1.0, ib->Hc_ext, c->nr, c->stream) == hipSuccess;
-  ok = ok && c3d::launch_fwd_x(c->g, false, nullptr, nullptr, nullptr, ib->Hc_ext, c->S, false, c->stream) == hipSuccess;
   if (!ok) return fail(c, C3D_EHIP, "Heaviside set-up failed");
-  if ((rc = spectral_core(c))) return rc;
-  ok = c3d::launch_inv_x(c->g, 0, c->S, ib->Hc_ext, c->P, 1.0, false, c->stream) == hipSuccess;
-  ok = ok && B::launch_affine(ib->Hc_ext, 1.0, -1.0, ib->Hc_ext, c->nr, c->stream) == hipSuccess;
+  if ((rc = spectral_forward(c, false, nullptr, nullptr, nullptr, ib->Hc_ext, false)) ||
+      (rc = spectral_inverse(c, 0, ib->Hc_ext, 1.0, false)))
+    return rc;
+  ok = B::launch_affine(ib->Hc_ext, 1.0, -1.0, ib->Hc_ext, c->nr, c->stream) == hipSuccess;
   ok = ok && hipMemsetAsync(Hu, 0, c->nu * 8, c->stream) == hipSuccess &&
        hipMemsetAsync(Hv, 0, c->nv * 8, c->stream) == hipSuccess &&
        hipMemsetAsync(Hw, 0, c->nw * 8, c->stream) == hipSuccess;

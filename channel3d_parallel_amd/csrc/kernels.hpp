@@ -72,6 +72,15 @@ hipError_t launch_fwd_x(const DevGrid& g, bool from_uvw, const double* U, const 
                         const Planes* pl = nullptr);
 hipError_t launch_fft_z(const DevGrid& g, int sign, cpx<double>* S, hipStream_t s,
                         const Planes* pl = nullptr);
+// Whether a plane's two transforms run in one kernel each way (plane_fft.hip):
+// launch_fwd_plane in place of launch_fwd_x and launch_fft_z(-1),
+// launch_inv_plane in place of launch_fft_z(+1) and launch_inv_x.
+bool plane_fft(const DevGrid& g);
+hipError_t launch_fwd_plane(const DevGrid& g, bool from_uvw, const double* U, const double* V,
+                            const double* W, const double* rhs, cpx<double>* S, bool per,
+                            hipStream_t s, const Planes* pl = nullptr);
+hipError_t launch_inv_plane(const DevGrid& g, int mode, const cpx<double>* S, double* out, double* P,
+                            double dt, bool rk1, hipStream_t s, const Planes* pl = nullptr);
 // Tridiagonal solve along y for every (kx,kz): the partitioned register
 // solver from 33 to 768 rows, else the plain Thomas sweep with CP, nym*nxh*nzp
 // doubles of scratch (may be null unless tri_needs_scratch).
