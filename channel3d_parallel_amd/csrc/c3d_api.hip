@@ -1481,6 +1481,8 @@ static int ib_iteration_graph(c3d_ctx* c, double* x, double dt, int rk_step, hip
       return 0;
     }
   if (ib->graphs.size() >= 8) {  // bounded cache: start over
+    // (the last solve's iteration queued ahead may still be running)
+    HIPCHK(c, hipStreamSynchronize(c->stream));
     for (auto& gr : ib->graphs) (void)hipGraphExecDestroy(gr.exec);
     ib->graphs.clear();
   }
