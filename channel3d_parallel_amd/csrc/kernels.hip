@@ -55,7 +55,14 @@ constexpr int kSrcUVWB = 2;   // same, and the FP64 divergence also stored to bo
 constexpr int kSrcUVWc = 4;   // as kSrcUVW with cached U and W loads (fields that fit in cache)
 constexpr int kSrcResid = 5;  // FP64 residual b - M phi of the refinement, on the fly
 
-template <typename real, int N, int TK, int SRC>
+// IMG: the divergence takes the boundary values from the interior (U(1) =
+// U(nx-1), W(1) = W(nz-1), V = 0 on the walls), so the fields need no boundary
+// conditions applied, and `planes` (may be null) lists the y planes; else the
+// fields as they are, on every plane.  The loads are the same either way and
+// the boundary values replaced after them: chosen before the loads, at run
+// time, they split the 16-byte load of U(i-1), U(i) in two and put branches
+// around V's (384x192x384 cells: 207 against 191 us without the choice).
+template <typename real, int N, int TK, int SRC, bool IMG = false>
 __global__ __launch_bounds__(kBlock) void k_fwd_x(DevGrid g, const double* __restrict__ U,
                                                   const double* __restrict__ V,
                                                   const double* __restrict__ W,
@@ -64,7 +71,7 @@ __global__ __launch_bounds__(kBlock) void k_fwd_x(DevGrid g, const double* __res
                                                   cpx<real>* __restrict__ S,
                                                   double* __restrict__ bout,
                                                   const double* __restrict__ gauge,
-                                                  unsigned long long* __restrict__ rmax, int per,
+                                                  unsigned long long* __restrict__ rmax,
                                                   const int* __restrict__ planes) {
   constexpr bool FROM_UVW = (SRC == kSrcUVW || SRC == kSrcUVWB || SRC == kSrcUVWc);
   constexpr bool RESID = (SRC == kSrcResid);
@@ -81,7 +88,7 @@ __global__ __launch_bounds__(kBlock) void k_fwd_x(DevGrid g, const double* __res
   const int tid = threadIdx.x;
   const int k0 = blockIdx.x * TK;
   const int js = blockIdx.y;  // the plane's place in the spectrum
-  const int j = (planes ? planes[js] : js) + 2;
+  const int j = (IMG && planes ? planes[js] : js) + 2;
   const int nx = g.nx, ny = g.ny, nxg = g.nxg, nyg = g.nyg;
 
   // 1) rows -> LDS.  Rows are walked with uniform (scalar) row bases; each
@@ -93,17 +100,14 @@ __global__ __launch_bounds__(kBlock) void k_fwd_x(DevGrid g, const double* __res
   const double ry = g.rdyf[j];
   double wprev[NPL];  // W(k-1) of the next row: the W row of the row before
   if constexpr (FROM_UVW) {
-    const double* W0 = W + fidx(1, j, (per && k0 == 0) ? g.nz - 1 : k0 + 1, nxg, nyg);
+    const double* W0 = W + fidx(1, j, (IMG && k0 == 0) ? g.nz - 1 : k0 + 1, nxg, nyg);
 #pragma unroll
     for (int p = 0; p < NPL; p++) {
       const int n = tid + p * kBlock;
       wprev[p] = (N % kBlock == 0 || n < N) ? W0[n + 1] : 0.0;
     }
   }
-  // per: the boundary values are taken from the interior (U(1) = U(nx-1),
-  // W(1) = W(nz-1), V = 0 on the walls), so the fields need no boundary
-  // conditions applied; else from the fields as they are
-  const bool vlo = per && j == 2, vhi = per && j == ny;
+  const bool vlo = IMG && j == 2, vhi = IMG && j == ny;
   // Residual r = b - M phi (D G on the unique cells, periodic in x and z, no
   // gradient on the wall faces, plus the (0,0)-mode gauge row at j = 2), with
   // U = phi and rhs_in = b; each lane walks its x positions down the tile's
@@ -152,6 +156,7 @@ __global__ __launch_bounds__(kBlock) void k_fwd_x(DevGrid g, const double* __res
 #pragma unroll
   for (int t0 = 0; t0 < TK; t0 += RB) {
     double v[RB][NPL][NV];
+    double ul[RB];  // IMG: U(nx-1) of each row
 #pragma unroll
     for (int r = 0; r < RB; r++) {
       const int k = k0 + t0 + r + 2;
@@ -160,11 +165,11 @@ __global__ __launch_bounds__(kBlock) void k_fwd_x(DevGrid g, const double* __res
         const double* Vr = V + fidx(1, j, k, nxg, ny);
         const double* Wr = W + fidx(1, j, k, nxg, nyg);
         const double* Vm = Vr - nxg;
+        if constexpr (IMG) ul[r] = Ur[N];
 #pragma unroll
         for (int p = 0; p < NPL; p++) {
           const int n = tid + p * kBlock;
           if (N % kBlock == 0 || n < N) {
-            const int nm = (per && n == 0) ? N : n;
             // x index i = n + 2 -> offset n + 1 in the row.  U and W rows
             // are read by this workgroup only: non-temporal when the fields
             // are too large to stay in cache between kernels.  V rows are
@@ -172,15 +177,15 @@ __global__ __launch_bounds__(kBlock) void k_fwd_x(DevGrid g, const double* __res
             // workgroup): cached.
             if constexpr (NTL) {
               v[r][p][0] = __builtin_nontemporal_load(&Ur[n + 1]);
-              v[r][p][1] = __builtin_nontemporal_load(&Ur[nm]);
+              v[r][p][1] = __builtin_nontemporal_load(&Ur[n]);
               v[r][p][4] = __builtin_nontemporal_load(&Wr[n + 1]);
             } else {
               v[r][p][0] = Ur[n + 1];
-              v[r][p][1] = Ur[nm];
+              v[r][p][1] = Ur[n];
               v[r][p][4] = Wr[n + 1];
             }
-            v[r][p][2] = vhi ? 0.0 : Vr[n + 1];
-            v[r][p][3] = vlo ? 0.0 : Vm[n + 1];
+            v[r][p][2] = Vr[n + 1];
+            v[r][p][3] = Vm[n + 1];
           }
         }
       } else if constexpr (RESID) {
@@ -222,8 +227,16 @@ __global__ __launch_bounds__(kBlock) void k_fwd_x(DevGrid g, const double* __res
               // face-spacing reciprocals tabulated
               const double rz = g.rdzf[k0 + t0 + r + h + 2];
               const double wm = (r + h == 0) ? wprev[p] : v[r + h - 1][p][4];
-              d[h] = (v[r + h][p][0] - v[r + h][p][1]) * rx +
-                     (v[r + h][p][2] - v[r + h][p][3]) * ry + (v[r + h][p][4] - wm) * rz;
+              double um = v[r + h][p][1], vp = v[r + h][p][2], vm = v[r + h][p][3];
+              if constexpr (IMG) {
+                if (p == 0) um = (n == 0) ? ul[r + h] : um;
+                vp = vhi ? 0.0 : vp;
+                vm = vlo ? 0.0 : vm;
+              }
+              // fused in one order for every source: which product is rounded by
+              // itself would else be the compiler's choice in each of them, and
+              // a body's iteration count in few rows follows the last bits
+              d[h] = fma(v[r + h][p][4] - wm, rz, fma(v[r + h][p][0] - um, rx, (vp - vm) * ry));
             } else if constexpr (RESID) {
               // r = b - D G phi on the unique cells (i = 2..nxp+1,
               // j = 2..nyg-1, k = 2..nzp+1): periodic in x and z (the face
@@ -892,6 +905,7 @@ inline dim3 grid_pts(const DevGrid& g, int ni, int nj, int nk) {
 hipError_t launch_fwd_x(const DevGrid& g, bool from_uvw, const double* U, const double* V,
                         const double* W, const double* rhs, cpx<double>* S, bool per, hipStream_t s,
                         const Planes* pl) {
+  if (pl && !(from_uvw && per)) return hipErrorInvalidValue;
   const int tk = tile_rows(g.nxp, g.nzp);
   dim3 grid(g.nzp / tk, pl ? pl->n : g.nym);
   const int* list = pl ? pl->list : nullptr;
@@ -899,16 +913,16 @@ hipError_t launch_fwd_x(const DevGrid& g, bool from_uvw, const double* U, const 
   // between the kernel that wrote them and this one: cached loads there
   // (measured 13.2 against 15.6 us at 128^3), non-temporal loads above.
   const bool small = 3.0 * g.nx * g.nyg * g.nzg * 8.0 < 128.0 * (1 << 20);
+  auto run = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, grid, dim3(kBlock), 0, s, g, U, V, W, (const void*)rhs, g.twx64, S, nullptr,
+                       nullptr, nullptr, list);
+  };
   C3D_DISPATCH_N(g.nxp, C3D_DISPATCH_TK(tk, {
-    if (from_uvw && small)
-      hipLaunchKernelGGL((k_fwd_x<double, NN, TK, kSrcUVWc>), grid, dim3(kBlock), 0, s, g, U, V, W,
-                         (const void*)rhs, g.twx64, S, nullptr, nullptr, nullptr, per ? 1 : 0, list);
-    else if (from_uvw)
-      hipLaunchKernelGGL((k_fwd_x<double, NN, TK, kSrcUVW>), grid, dim3(kBlock), 0, s, g, U, V, W,
-                         (const void*)rhs, g.twx64, S, nullptr, nullptr, nullptr, per ? 1 : 0, list);
-    else
-      hipLaunchKernelGGL((k_fwd_x<double, NN, TK, kSrcRhs>), grid, dim3(kBlock), 0, s, g, U, V, W,
-                         (const void*)rhs, g.twx64, S, nullptr, nullptr, nullptr, per ? 1 : 0, list);
+    if (!from_uvw) run(k_fwd_x<double, NN, TK, kSrcRhs>);
+    else if (small && per) run(k_fwd_x<double, NN, TK, kSrcUVWc, true>);
+    else if (small) run(k_fwd_x<double, NN, TK, kSrcUVWc>);
+    else if (per) run(k_fwd_x<double, NN, TK, kSrcUVW, true>);
+    else run(k_fwd_x<double, NN, TK, kSrcUVW>);
   }));
   return hipGetLastError();
 }
@@ -918,15 +932,15 @@ hipError_t launch_fwd_x32(const DevGrid& g, const double* U, const double* V, co
   if (!U || !V || !W) return hipErrorInvalidValue;
   const int tk = tile_rows(g.nxp, g.nzp);
   dim3 grid(g.nzp / tk, g.nym);
+  auto run = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, grid, dim3(kBlock), 0, s, g, U, V, W, (const void*)nullptr, g.twx32, S, b,
+                       nullptr, nullptr, nullptr);
+  };
   C3D_DISPATCH_N(g.nxp, C3D_DISPATCH_TK(tk, {
-    if (b)
-      hipLaunchKernelGGL((k_fwd_x<float, NN, TK, kSrcUVWB>), grid, dim3(kBlock), 0, s, g, U, V, W,
-                         (const void*)nullptr, g.twx32, S, b, nullptr, nullptr, per ? 1 : 0,
-                         nullptr);
-    else
-      hipLaunchKernelGGL((k_fwd_x<float, NN, TK, kSrcUVW>), grid, dim3(kBlock), 0, s, g, U, V, W,
-                         (const void*)nullptr, g.twx32, S, nullptr, nullptr, nullptr, per ? 1 : 0,
-                         nullptr);
+    if (b && per) run(k_fwd_x<float, NN, TK, kSrcUVWB, true>);
+    else if (b) run(k_fwd_x<float, NN, TK, kSrcUVWB>);
+    else if (per) run(k_fwd_x<float, NN, TK, kSrcUVW, true>);
+    else run(k_fwd_x<float, NN, TK, kSrcUVW>);
   }));
   return hipGetLastError();
 }
@@ -943,8 +957,7 @@ hipError_t fwd_x_resid(const DevGrid& g, const double* b, const double* phi, dou
   hipLaunchKernelGGL(k_gauge_final, dim3(1), dim3(kBlock), 0, s, g, (const double*)(gauge + 1), gauge);
   C3D_DISPATCH_N(g.nxp, C3D_DISPATCH_TK(tk, {
     hipLaunchKernelGGL((k_fwd_x<real, NN, TK, kSrcResid>), grid, dim3(kBlock), 0, s, g, phi,
-                       nullptr, nullptr, (const void*)b, tw, S, rout, (const double*)gauge, rmax, 0,
-                       nullptr);
+                       nullptr, nullptr, (const void*)b, tw, S, rout, (const double*)gauge, rmax, nullptr);
   }));
   return hipGetLastError();
 }
@@ -965,10 +978,13 @@ hipError_t launch_fwd_x_b64(const DevGrid& g, const double* U, const double* V, 
                             double* b, cpx<double>* S, bool per, hipStream_t s) {
   const int tk = tile_rows(g.nxp, g.nzp);
   dim3 grid(g.nzp / tk, g.nym);
+  auto run = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, grid, dim3(kBlock), 0, s, g, U, V, W, (const void*)nullptr, g.twx64, S, b,
+                       nullptr, nullptr, nullptr);
+  };
   C3D_DISPATCH_N(g.nxp, C3D_DISPATCH_TK(tk, {
-    hipLaunchKernelGGL((k_fwd_x<double, NN, TK, kSrcUVWB>), grid, dim3(kBlock), 0, s, g, U, V, W,
-                       (const void*)nullptr, g.twx64, S, b, nullptr, nullptr, per ? 1 : 0,
-                       nullptr);
+    if (per) run(k_fwd_x<double, NN, TK, kSrcUVWB, true>);
+    else run(k_fwd_x<double, NN, TK, kSrcUVWB>);
   }));
   return hipGetLastError();
 }

@@ -66,7 +66,8 @@ bool planes_supported(const DevGrid& g);
 // Forward x transform.  from_uvw: input is div(U,V,W) computed on the fly,
 // else the rhs_p array.  Writes the half spectrum S[j][kx][kz].  per: the
 // divergence takes the boundary values from the interior (the periodic
-// images and V = 0 on the walls) instead of the fields' boundary cells.
+// images and V = 0 on the walls) instead of the fields' boundary cells.  pl: with
+// from_uvw and per only.
 hipError_t launch_fwd_x(const DevGrid& g, bool from_uvw, const double* U, const double* V,
                         const double* W, const double* rhs, cpx<double>* S, bool per, hipStream_t s,
                         const Planes* pl = nullptr);
