@@ -62,6 +62,9 @@ constexpr int kSrcResid = 5;  // FP64 residual b - M phi of the refinement, on t
 // the boundary values replaced after them: chosen before the loads, at run
 // time, they split the 16-byte load of U(i-1), U(i) in two and put branches
 // around V's (384x192x384 cells: 207 against 191 us without the choice).
+// Cached fields take U(nx-1) by lane 0's own address instead: there a scalar
+// load per row costs more than the split one (iterations of a body's solve on
+// 128x128x128 cells 245.4 against 243.4 us).
 template <typename real, int N, int TK, int SRC, bool IMG = false>
 __global__ __launch_bounds__(kBlock) void k_fwd_x(DevGrid g, const double* __restrict__ U,
                                                   const double* __restrict__ V,
@@ -156,7 +159,7 @@ __global__ __launch_bounds__(kBlock) void k_fwd_x(DevGrid g, const double* __res
 #pragma unroll
   for (int t0 = 0; t0 < TK; t0 += RB) {
     double v[RB][NPL][NV];
-    double ul[RB];  // IMG: U(nx-1) of each row
+    double ul[RB];  // IMG, NTL: U(nx-1) of each row
 #pragma unroll
     for (int r = 0; r < RB; r++) {
       const int k = k0 + t0 + r + 2;
@@ -165,7 +168,7 @@ __global__ __launch_bounds__(kBlock) void k_fwd_x(DevGrid g, const double* __res
         const double* Vr = V + fidx(1, j, k, nxg, ny);
         const double* Wr = W + fidx(1, j, k, nxg, nyg);
         const double* Vm = Vr - nxg;
-        if constexpr (IMG) ul[r] = Ur[N];
+        if constexpr (IMG && NTL) ul[r] = Ur[N];
 #pragma unroll
         for (int p = 0; p < NPL; p++) {
           const int n = tid + p * kBlock;
@@ -181,7 +184,7 @@ __global__ __launch_bounds__(kBlock) void k_fwd_x(DevGrid g, const double* __res
               v[r][p][4] = __builtin_nontemporal_load(&Wr[n + 1]);
             } else {
               v[r][p][0] = Ur[n + 1];
-              v[r][p][1] = Ur[n];
+              v[r][p][1] = Ur[IMG && n == 0 ? N : n];
               v[r][p][4] = Wr[n + 1];
             }
             v[r][p][2] = Vr[n + 1];
@@ -229,7 +232,7 @@ __global__ __launch_bounds__(kBlock) void k_fwd_x(DevGrid g, const double* __res
               const double wm = (r + h == 0) ? wprev[p] : v[r + h - 1][p][4];
               double um = v[r + h][p][1], vp = v[r + h][p][2], vm = v[r + h][p][3];
               if constexpr (IMG) {
-                if (p == 0) um = (n == 0) ? ul[r + h] : um;
+                if (NTL && p == 0) um = (n == 0) ? ul[r + h] : um;
                 vp = vhi ? 0.0 : vp;
                 vm = vlo ? 0.0 : vm;
               }
