@@ -227,9 +227,11 @@ int c3d_set_rhs_exact(c3d_ctx *ctx, int on);
 /* Timing of resident projections with HIP events on the context stream:
  * a pass of `iters` back-to-back projections with an event between kernel
  * stages gives kernel_ms[0..nk), the average ms per stage (order from
- * c3d_stage_name, nk <= c3d_stage_count()); a second pass of `iters`
- * projections between two events only gives total_ms, the average ms per
- * projection.  No reference counterpart: measurement hook for the hot path. */
+ * c3d_stage_name, nk <= c3d_stage_count(); where one kernel does both
+ * transforms of a plane, the x stages hold it and the z stages are 0); a
+ * second pass of `iters` projections between two events only gives total_ms,
+ * the average ms per projection.  No reference counterpart: measurement hook
+ * for the hot path. */
 int c3d_time_projection(c3d_ctx *ctx, int iters, double dt, double *total_ms, double *kernel_ms,
                         int nk);
 int c3d_stage_count(void);
