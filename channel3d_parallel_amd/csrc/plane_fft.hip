@@ -233,16 +233,26 @@ __global__ __launch_bounds__(kPB) void k_inv_plane(DevGrid g, const cpx<double>*
 // separate ones 26.8 us.
 constexpr int kPlaneMax = 4608;
 
-// BODY with N and NZ, the transform lengths.
-#define C3D_PLANE_Z(NN, nz, ...)                                                                    \
-  switch (nz) {                                                                                     \
-    case 16: { constexpr int NZ = 16; __VA_ARGS__; } break;                                         \
-    case 32: { constexpr int NZ = 32; __VA_ARGS__; } break;                                         \
-    case 48: { constexpr int NZ = 48; __VA_ARGS__; } break;                                         \
-    case 64: { constexpr int NZ = 64; __VA_ARGS__; } break;                                         \
-    case 96: if constexpr (NN * 96 <= kPlaneMax) { constexpr int NZ = 96; __VA_ARGS__; } else return hipErrorInvalidValue; break;\
-    case 128: if constexpr (NN * 128 <= kPlaneMax) { constexpr int NZ = 128; __VA_ARGS__; } else return hipErrorInvalidValue; break;\
-    default: return hipErrorInvalidValue;                                                           \
+// BODY with N and NZ, the transform lengths; planes above kPlaneMax are not
+// built, since plane_fft() never takes them.
+#define C3D_PLANE_CASE(NN, M, ...)                      \
+  case M:                                               \
+    if constexpr (NN * M <= kPlaneMax) {                \
+      constexpr int NZ = M;                             \
+      __VA_ARGS__;                                      \
+    } else {                                            \
+      return hipErrorInvalidValue;                      \
+    }                                                   \
+    break;
+#define C3D_PLANE_Z(NN, nz, ...)                        \
+  switch (nz) {                                         \
+    C3D_PLANE_CASE(NN, 16, __VA_ARGS__)                 \
+    C3D_PLANE_CASE(NN, 32, __VA_ARGS__)                 \
+    C3D_PLANE_CASE(NN, 48, __VA_ARGS__)                 \
+    C3D_PLANE_CASE(NN, 64, __VA_ARGS__)                 \
+    C3D_PLANE_CASE(NN, 96, __VA_ARGS__)                 \
+    C3D_PLANE_CASE(NN, 128, __VA_ARGS__)                \
+    default: return hipErrorInvalidValue;               \
   }
 #define C3D_PLANE(nx, nz, ...)                                                                      \
   switch (nx) {                                                                                     \

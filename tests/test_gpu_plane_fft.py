@@ -44,3 +44,31 @@ def test_planes(nx, ny, nz):
             assert rel(out["P"][c], P[c]) <= 1e-12
             # P_interim = solution/dt off the plane that the divergence leaves zero
             assert rel(phi[:, :, :-1], 1e-3 * ref["P_interim"][:, :, :-1]) <= 1e-12
+
+
+# every pair of lengths that has such a kernel: planes of up to 4608 points
+LENGTHS = (16, 32, 48, 64, 96, 128)
+PAIRS = [(n, m) for n in LENGTHS for m in LENGTHS if n * m <= 4608]
+
+
+@pytest.mark.parametrize("nxp,nzp", PAIRS)
+def test_every_plane_kernel(nxp, nzp):
+    nx, ny, nz = nxp + 2, 34 + (nxp + 3 * nzp) // 16 % 13, nzp + 2
+    print(f"\n[case] plane kernels {nx}x{ny}x{nz}", flush=True)
+    g = orc.Grid(nx, ny, nz)
+    U, V, W = fields.white_faces(nx, ny, nz, seed=nx + nz)
+    g.apply_bc(U, V, W)
+    with Channel(nx, ny, nz) as ch:
+        ch.set_fields(U, V, W)
+        ch.compute_non_IB_projection(1e-3, rk_step=1)
+        out = ch.get_fields()
+        phi = ch.solve_poisson_equation(np.asfortranarray(ch.divergence(U, V, W)))
+        stages = ch.time_projection(1, 1e-3)[1]
+    assert stages["fft_z_fwd"] == stages["fft_z_inv"] == 0  # the plane's own kernels ran
+    P = g.zeros("p")
+    ref = g.projection(U, V, W, rk_step=1, dt=1e-3, P=P)
+    for name, b in (("U", U), ("V", V), ("W", W), ("P_interim", ref["P_interim"])):
+        assert rel(out[name], b) <= 1e-12, name
+    c = np.s_[1:-1, 1:-1, 1:-1]
+    assert rel(out["P"][c], P[c]) <= 1e-12
+    assert rel(phi[:, :, :-1], 1e-3 * ref["P_interim"][:, :, :-1]) <= 1e-12
