@@ -27,3 +27,27 @@ def test_planes_near_the_body(nx, ny, nz, kind):
             assert np.abs(full).max() > 0
             assert np.array_equal(ch.schur(f, 0.01, rk_step=2), full)
             f = full / np.abs(full).max()
+
+
+# planes of more than 4608 points, which the separate x and z transforms take
+BIG = [(98, 65, 66, "body"), (130, 50, 66, "body"), (50, 101, 130, "body"), (98, 101, 66, "walls"),
+       (258, 129, 34, "walls")]
+
+
+@pytest.mark.parametrize("nx,ny,nz,kind", BIG)
+def test_planes_near_the_body_with_separate_transforms(nx, ny, nz, kind):
+    print(f"\n[case] planes near the body {nx}x{ny}x{nz} {kind}", flush=True)
+    args = dict(grid_type=2, alpha=2.6, min_buffer_width=0.1) if kind == "walls" else dict(grid_type=0)
+    with Channel(nx, ny, nz, nu=1e-3, **args) as ch:
+        if kind == "walls":
+            ch.setup_IB_wave("standing_wave", 32, 16, 0.03, 2.0, 1.0, 0.0, 0.0)
+        else:
+            ch.setup_IB(ib_geometry.two_cylinders(ch.grid(11)[9], nzb=16, nth=24))
+        stages = ch.time_projection(1, 1e-3)[1]
+        assert stages["fft_z_fwd"] > 0 and stages["fft_z_inv"] > 0
+        f = np.random.default_rng(ny).standard_normal(4 * ch.nb)
+        for _ in range(2):  # the second product finds the first one's spectrum and potential
+            full = ch.schur(f, 0.01, rk_step=1)
+            assert np.abs(full).max() > 0
+            assert np.array_equal(ch.schur(f, 0.01, rk_step=2), full)
+            f = full / np.abs(full).max()
