@@ -230,7 +230,9 @@ __global__ __launch_bounds__(kPB) void k_inv_plane(DevGrid g, const cpx<double>*
 // few microseconds of one CU's work: 20 steps of 32x64x32 cells 2.92 against
 // 3.54 ms with separate transforms, of 96x100x48 cells 4.76 against 5.19 ms; at
 // 128 x 64 points the two kernels of a plane take 17.0 + 13.7 us, the four
-// separate ones 26.8 us.
+// separate ones 26.8 us.  Between the two, planes of 6144 points are mixed:
+// projections of 96x64x64 cells 41.0 against 43.2 us, of 64x64x96 41.0 against
+// 41.7, of 128x96x48 44.5 against 46.2, but of 48x64x128 46.7 against 38.2 us.
 constexpr int kPlaneMax = 4608;
 
 // BODY with N and NZ, the transform lengths; planes above kPlaneMax are not
@@ -265,6 +267,20 @@ constexpr int kPlaneMax = 4608;
     default: return hipErrorInvalidValue;                                                           \
   }
 
+// Rows from which a plane's kernels pay: their time is that of a plane's chain
+// of passes up to 256 planes, that of the separate transforms grows with the
+// rows, and the chain is long where eight threads walk long z columns.
+// Projections, us, separate | plane's kernels (a time step in brackets): 32 x 128
+// points 33 rows 30.8 | 35.3, 96 rows 40.4 | 42.4 [185 | 188], 128 rows 46.2 |
+// 42.5; 16 x 128 points 96 rows 35.2 | 36.0, 128 rows 39.8 | 39.5; 48 x 96 points
+// 48 rows 36.3 | 37.8 [156 | 158], 80 rows 41.4 | 41.6 [175 | 171].  All other
+// shapes gain from 33 rows on (96 x 48 points, the least: 33 rows 33.0 | 33.3,
+// 40 rows [144 | 143], 48 rows 35.6 | 35.4).
+int plane_rows(int nxp, int nzp) {
+  if (nzp >= 128) return 128;
+  return nzp > 64 && nxp * nzp > 4096 ? 64 : 0;
+}
+
 }  // namespace
 
 // C3D_PLANE_MAX lowers the largest plane (tuning knob; 0: none).
@@ -277,7 +293,8 @@ bool plane_fft(const DevGrid& g) {
   // With up to 32 rows the iteration count of an immersed body's solve follows
   // the last bits of the transforms and the elimination (two cylinders in 32
   // rows: 97 iterations with this path, the reference's 114 +- 2 without).
-  return g.nxp <= 128 && g.nzp <= 128 && g.nxp * g.nzp <= most && planes_supported(g);
+  return g.nxp <= 128 && g.nzp <= 128 && g.nxp * g.nzp <= most &&
+         g.nym >= plane_rows(g.nxp, g.nzp) && planes_supported(g);
 }
 
 hipError_t launch_fwd_plane(const DevGrid& g, bool from_uvw, const double* U, const double* V,

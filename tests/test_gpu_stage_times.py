@@ -1,7 +1,8 @@
 """Stage times of c3d_time_projection are those of the kernels that a
 projection runs: where one kernel does both transforms of a plane (up to 4608
-points, FP64 without refinement, 33 rows or more), the x stages hold them and
-the z stages are 0; elsewhere every transform has its stage."""
+points, FP64 without refinement, 33 rows or more, for long z columns only from
+the row count on where it is the faster), the x stages hold them and the z
+stages are 0; elsewhere every transform has its stage."""
 import pytest
 
 from channel3d_parallel_amd import Channel, fields
@@ -11,7 +12,9 @@ pytestmark = pytest.mark.gpu
 
 CASES = [(34, 65, 34, PREC_FP64, None, True), (98, 40, 50, PREC_FP64, None, True), (34, 65, 34, PREC_FP64, 1, False),
          (34, 65, 34, PREC_MIXED, 0, False), (34, 33, 34, PREC_FP64, None, False),
-         (98, 65, 66, PREC_FP64, None, False)]
+         (98, 65, 66, PREC_FP64, None, False), (34, 45, 130, PREC_FP64, None, False),
+         (34, 129, 130, PREC_FP64, None, True), (18, 128, 130, PREC_FP64, None, False),
+         (50, 64, 98, PREC_FP64, None, False), (50, 65, 98, PREC_FP64, None, True)]
 
 
 @pytest.mark.parametrize("nx,ny,nz,precision,sweeps,one", CASES)
