@@ -268,7 +268,10 @@ constexpr int kStats = 7;
 
 // The planes are split into chunks so that 1024 workgroups share them (one
 // workgroup per row was 193 of them, 597 us on 384x192x384 cells); the chunks
-// are added in order by k_plane_final.
+// are added in order by k_plane_final, a single chunk holds the sums already.
+// L: lanes per x row, so that short rows share a wavefront (16 and 32 cells in
+// x: 800 rows 9.1 -> 6.9 us, 300 rows 9.5 -> 5.8 us).
+template <int L>
 __global__ __launch_bounds__(kB) void k_plane_sums(DevGrid g, const double* __restrict__ U,
                                                    const double* __restrict__ V,
                                                    const double* __restrict__ W, int run,
@@ -284,12 +287,12 @@ __global__ __launch_bounds__(kB) void k_plane_sums(DevGrid g, const double* __re
   double a[kStats] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
   // U, V: k = 2..nzg-2; W: k = 2..nz-1, the same range (nzg = nz + 1)
   const int ka = blockIdx.y * run + 2, ke = min(ka + run - 1, g.nzg - 2);
-  for (int k = ka + wv; k <= ke; k += kB / 64) {
+  for (int k = ka + (L == 64 ? wv : (int)threadIdx.x / L); k <= ke; k += kB / L) {
     const double* u = U + fidx(1, j, k, nx, nyg);
     const double* v = V + fidx(1, jv, k, nxg, ny);
     const double* w = W + fidx(1, j, k, nxg, nyg);
 #pragma unroll 2
-    for (int i = 1 + lane; i <= nxg - 3; i += 64) {  // offset of x index i + 1
+    for (int i = 1 + lane % L; i <= nxg - 3; i += L) {  // offset of x index i + 1
       const double t1 = 0.5 * (u[i - 1] + u[i]);
       const double t2 = sg * (0.5 * (v[i - nxg] + v[i]));
       const double t3 = w[i];
@@ -328,30 +331,45 @@ __global__ __launch_bounds__(kB) void k_plane_final(const double* __restrict__ p
 // the sums and maxima of U(2:nx-1,2:nyg-1,2:nzg-1), V(2:nxg-1,2:ny-1,2:nzg-1)
 // and W(2:nxg-1,2:nyg-1,2:nz-1), and the count of non-finite entries of the
 // three (a NaN guard), into part[b*kMon + q]; k_monitor_final reduces the
-// kMonBlocks partials in a fixed order.
+// partials, up to kMonBlocks, in a fixed order.
 constexpr int kMon = 7;  // sum U, V, W; max U, V, W; non-finite count
 constexpr int kMonBlocks = 1024;
 
+// Lanes per x row of the field summaries: rows of up to 64 share a unit.
+inline int mon_lanes(long long ni) { return ni <= 16 ? 16 : (ni <= 32 ? 32 : (ni <= 64 ? 64 : 256)); }
+
+// Interior (2..i1, 2..j1, 2..k1) of an (n1, n2, *) array: a wavefront takes
+// units of four loads per lane, 256 x positions of a row (L = 256) or, of rows
+// of up to L positions, 256 / L rows of a plane, so the index arithmetic is
+// scalar (a division per element made this 838 us on 384x192x384 cells; a row
+// per unit whatever its length 15.9 us on 16x799x16 cells, now 8.0).
+template <int L>
 __device__ __forceinline__ void mon_field(const double* __restrict__ F, int n1, int n2, int i1, int j1,
                                           int k1, double& sum, double& mx, double& bad) {
-  // interior (2..i1, 2..j1, 2..k1) of an (n1, n2, *) array: a wavefront takes
-  // 256 x positions of a row at a time, so the index arithmetic is scalar (a
-  // division per element made this 838 us on 384x192x384 cells)
+  constexpr int R = 256 / L;  // rows of a unit
   const int lane = threadIdx.x & 63;
-  const long long ni = i1 - 1, nj = j1 - 1, nseg = (ni + 255) / 256;
-  const long long n = nseg * nj * (k1 - 1);
+  const long long ni = i1 - 1, nj = j1 - 1, nseg = (ni + L - 1) / L, nu = (nj + R - 1) / R;
+  const long long n = nseg * nu * (k1 - 1);
   const int wv = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
-  for (long long t = (long long)blockIdx.x * (kB / 64) + wv; t < n; t += kMonBlocks * (kB / 64)) {
-    const long long r = t / nseg, i0 = (t - r * nseg) * 256;
-    const long long k = r / nj, j = r - k * nj;
-    const double* row = F + 1 + (size_t)n1 * ((size_t)(j + 1) + (size_t)n2 * (size_t)(k + 1)) + i0;
+  for (long long t = (long long)blockIdx.x * (kB / 64) + wv; t < n; t += gridDim.x * (kB / 64)) {
+    const long long r = R == 1 ? t / nseg : t, i0 = R == 1 ? (t - r * nseg) * L : 0;
+    const long long k = r / nu, j0 = (r - k * nu) * R;
+    const double* row = F + 1 + (size_t)n1 * ((size_t)(j0 + 1) + (size_t)n2 * (size_t)(k + 1)) + i0;
+    auto at = [&](int q, bool& in) {  // the lane's q-th element of the unit
+      const int e = q * 64 + lane, i = e % L, j = e / L;
+      in = i0 + i < ni && (R == 1 || j0 + j < nj);
+      return (size_t)j * n1 + i;
+    };
     double v[4];
+    bool in[4];
+#pragma unroll
+    for (int q = 0; q < 4; q++) {
+      const size_t o = at(q, in[q]);
+      if (in[q]) v[q] = row[o];
+    }
 #pragma unroll
     for (int q = 0; q < 4; q++)
-      if (i0 + q * 64 + lane < ni) v[q] = row[q * 64 + lane];
-#pragma unroll
-    for (int q = 0; q < 4; q++)
-      if (i0 + q * 64 + lane < ni) {
+      if (in[q]) {
         sum += v[q];
         mx = fmax(mx, v[q]);
         bad += isfinite(v[q]) ? 0.0 : 1.0;
@@ -359,15 +377,16 @@ __device__ __forceinline__ void mon_field(const double* __restrict__ F, int n1, 
   }
 }
 
+template <int L>
 __global__ __launch_bounds__(kB) void k_monitor_part(DevGrid g, const double* __restrict__ U,
                                                      const double* __restrict__ V,
                                                      const double* __restrict__ W,
                                                      double* __restrict__ part) {
   __shared__ double sh[kMon][kB];
   double a[kMon] = {0.0, 0.0, 0.0, -INFINITY, -INFINITY, -INFINITY, 0.0};
-  mon_field(U, g.nx, g.nyg, g.nx - 1, g.nyg - 1, g.nzg - 1, a[0], a[3], a[6]);
-  mon_field(V, g.nxg, g.ny, g.nxg - 1, g.ny - 1, g.nzg - 1, a[1], a[4], a[6]);
-  mon_field(W, g.nxg, g.nyg, g.nxg - 1, g.nyg - 1, g.nz - 1, a[2], a[5], a[6]);
+  mon_field<L>(U, g.nx, g.nyg, g.nx - 1, g.nyg - 1, g.nzg - 1, a[0], a[3], a[6]);
+  mon_field<L>(V, g.nxg, g.ny, g.nxg - 1, g.ny - 1, g.nzg - 1, a[1], a[4], a[6]);
+  mon_field<L>(W, g.nxg, g.nyg, g.nxg - 1, g.nyg - 1, g.nz - 1, a[2], a[5], a[6]);
 #pragma unroll
   for (int q = 0; q < kMon; q++) sh[q][threadIdx.x] = a[q];
   __syncthreads();
@@ -383,14 +402,17 @@ __global__ __launch_bounds__(kB) void k_monitor_part(DevGrid g, const double* __
   if (threadIdx.x < kMon) part[(size_t)blockIdx.x * kMon + threadIdx.x] = sh[threadIdx.x][0];
 }
 
-__global__ __launch_bounds__(kB) void k_monitor_final(const double* __restrict__ part,
+__global__ __launch_bounds__(kB) void k_monitor_final(const double* __restrict__ part, int n,
                                                       double* __restrict__ out) {
   __shared__ double sh[kMon][kB];
 #pragma unroll
   for (int q = 0; q < kMon; q++) {
-    double a = part[(size_t)threadIdx.x * kMon + q];
-    for (int b = threadIdx.x + kB; b < kMonBlocks; b += kB) {
-      const double v = part[(size_t)b * kMon + q];
+    const double none = (q >= 3 && q < 6) ? -INFINITY : 0.0;
+    double a = none;
+#pragma unroll
+    for (int r = 0; r < kMonBlocks / kB; r++) {
+      const int b = threadIdx.x + r * kB;
+      const double v = b < n ? part[(size_t)b * kMon + q] : none;
       a = (q >= 3 && q < 6) ? fmax(a, v) : a + v;
     }
     sh[q][threadIdx.x] = a;
@@ -518,15 +540,30 @@ hipError_t launch_monitor_finish(const double* r7, double vol, double* out, hipS
 
 hipError_t launch_monitor(const DevGrid& g, const double* U, const double* V, const double* W,
                           double* part, double* out7, hipStream_t s) {
-  static_assert(kMonBlocks % kB == 0, "the final reduction takes whole rounds of partials");
-  hipLaunchKernelGGL(k_monitor_part, dim3(kMonBlocks), dim3(kB), 0, s, g, U, V, W, part);
-  hipLaunchKernelGGL(k_monitor_final, dim3(1), dim3(kB), 0, s, (const double*)part, out7);
+  // a unit per wavefront, up to kMonBlocks workgroups: fewer partials of a
+  // small grid (18x4x18: final 5.6 -> 2.3 us)
+  const long long ni = g.nxg - 2;
+  const int lanes = mon_lanes(ni), rows = 256 / lanes;
+  const long long units = (ni + lanes - 1) / lanes * ((g.nyg - 2 + rows - 1) / rows) * (g.nzg - 2);
+  const int n = (int)std::min<long long>((units + kB / 64 - 1) / (kB / 64), kMonBlocks);
+  switch (lanes) {
+    case 16: hipLaunchKernelGGL(k_monitor_part<16>, dim3(n), dim3(kB), 0, s, g, U, V, W, part); break;
+    case 32: hipLaunchKernelGGL(k_monitor_part<32>, dim3(n), dim3(kB), 0, s, g, U, V, W, part); break;
+    case 64: hipLaunchKernelGGL(k_monitor_part<64>, dim3(n), dim3(kB), 0, s, g, U, V, W, part); break;
+    default: hipLaunchKernelGGL(k_monitor_part<256>, dim3(n), dim3(kB), 0, s, g, U, V, W, part); break;
+  }
+  hipLaunchKernelGGL(k_monitor_final, dim3(1), dim3(kB), 0, s, (const double*)part, n, out7);
   return hipGetLastError();
 }
 
-// Planes per chunk of the plane sums: about 1024 workgroups.
+// Lanes per x row of the plane sums, and planes per chunk: about 1024
+// workgroups, but chunks of at least eight rounds of a workgroup's loads, so
+// that small grids need no second launch (32x299x32 cells: the call 34.4 -> 31.1 us).
+static int stat_lanes(const DevGrid& g) { return g.nxg - 3 <= 16 ? 16 : (g.nxg - 3 <= 32 ? 32 : 64); }
 static int stat_run(const DevGrid& g) {
-  const int nk = g.nzg - 3, chunks = std::max(1, std::min(1024 / g.nyg, (nk + 3) / 4));
+  const int lanes = stat_lanes(g), once = kB / lanes, nk = g.nzg - 3;
+  const int rounds = (nk + once - 1) / once * ((g.nxg - 3 + lanes - 1) / lanes);
+  const int chunks = std::max(1, std::min(1024 / g.nyg, rounds / 8));
   return (nk + chunks - 1) / chunks;
 }
 static int stat_chunks(const DevGrid& g) { return (g.nzg - 3 + stat_run(g) - 1) / stat_run(g); }
@@ -535,9 +572,15 @@ size_t plane_sums_part_size(const DevGrid& g) { return (size_t)stat_chunks(g) * 
 hipError_t launch_plane_sums(const DevGrid& g, const double* U, const double* V, const double* W,
                              double* part, double* sums, hipStream_t s) {
   const int n = kStats * g.nyg, c = stat_chunks(g);
-  hipLaunchKernelGGL(k_plane_sums, dim3(g.nyg, c), dim3(kB), 0, s, g, U, V, W, stat_run(g), part);
-  hipLaunchKernelGGL(k_plane_final, dim3((n + kB - 1) / kB), dim3(kB), 0, s, (const double*)part, n, c,
-                     sums);
+  double* out = c == 1 ? sums : part;
+  switch (stat_lanes(g)) {
+    case 16: hipLaunchKernelGGL(k_plane_sums<16>, dim3(g.nyg, c), dim3(kB), 0, s, g, U, V, W, stat_run(g), out); break;
+    case 32: hipLaunchKernelGGL(k_plane_sums<32>, dim3(g.nyg, c), dim3(kB), 0, s, g, U, V, W, stat_run(g), out); break;
+    default: hipLaunchKernelGGL(k_plane_sums<64>, dim3(g.nyg, c), dim3(kB), 0, s, g, U, V, W, stat_run(g), out); break;
+  }
+  if (c > 1)
+    hipLaunchKernelGGL(k_plane_final, dim3((n + kB - 1) / kB), dim3(kB), 0, s, (const double*)part, n, c,
+                       sums);
   return hipGetLastError();
 }
 
