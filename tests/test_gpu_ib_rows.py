@@ -2,7 +2,7 @@
 solve is the partitioned one, Schur products transform only the planes near the
 body, and planes of up to 4608 points have a kernel for both transforms
 (34x34x34 to 34x65x34; 98x50x66 is above): Schur products, the first BiCGSTAB
-iterates, and a projection.
+iterates, and a projection; the stencils at odd marker counts.
 
 Bars: Schur products 1e-12 of the largest entry (one Poisson solve); iterates
 after 1 to 3 iterations relative 1e-11, up to 7 products each 1e-12 off (the
@@ -81,3 +81,17 @@ def test_projection(nx, ny, nz, nth, nzb):
     assert rel(fbg, fbo) < 1e-6
     for a, b in ((r["U"], Uo), (r["V"], Vo), (r["W"], Wo)):
         assert rel(a, b) < 1e-8
+
+
+@pytest.mark.parametrize("nth,nzb", [(8, 4), (9, 7), (23, 13)])
+def test_stencils_of_any_marker_count(nth, nzb):
+    """Bit for bit but the weights (1e-14, device asin and sqrt), for marker
+    counts that leave a part of the last workgroup's 64 and one below 64."""
+    g, m, ib, ch = body(34, 34, 18, nth, nzb)
+    with ch:
+        for s in range(4):
+            got, ref = ch.ib_stencil(s), ib.stencil(s)
+            for a, b in zip(got[:3], ref[:3]):
+                assert np.array_equal(a, b), s
+            assert np.max(np.abs(got[3] - ref[3])) <= 1e-14 * np.max(np.abs(ref[3])), s
+            assert np.array_equal(got[4], ref[4]), s
