@@ -440,14 +440,16 @@ int sync(c3d_ctx* c) {
   return 0;
 }
 
-// The halves of the Poisson pipeline: div(U, V, W) or rhs to its spectrum, and
-// the spectrum's solution to out (launch_fwd_x, launch_inv_x).  ev: events after
-// the stages, two and three of them; a plane's kernels hold both transforms,
-// which makes them the x stage and leaves nothing between the z stage's events.
+// The event after a stage of a timed projection (ev null: none).
 int stage_done(c3d_ctx* c, hipEvent_t* ev, int stage) {
   if (ev) HIPCHK(c, hipEventRecord(ev[stage], c->stream));
   return 0;
 }
+
+// The halves of the Poisson pipeline: div(U, V, W) or rhs to its spectrum, and
+// the spectrum's solution to out (launch_fwd_x, launch_inv_x).  ev: events after
+// their two and three stages; a plane's kernels hold both transforms, which
+// makes them the x stage and leaves nothing between the z stage's events.
 int spectral_forward(c3d_ctx* c, bool from_uvw, const double* U, const double* V, const double* W,
                      const double* rhs, bool per, const c3d::Planes* pl = nullptr,
                      hipEvent_t* ev = nullptr) {

@@ -396,7 +396,7 @@ __global__ __launch_bounds__(kBlock) void k_interp_c(DevGrid g, Markers m, C3D_S
 // G(dt*phi) - Reg_c of the Schur velocity rows (src/projection.f90:131-142) in
 // place of Reg_c, at the support nodes of each component (block row c): each
 // node once, where the markers' stencils would evaluate it for every one of
-// the (36 on average, two cylinders) entries that share it.  Every node lies
+// the (37 on average, two cylinders) entries that share it.  Every node lies
 // in the gradient's index ranges (checked at set-up), where
 // apply_boundary_conditions does not write.
 __global__ __launch_bounds__(kBlock) void k_node_grad(DevGrid g, Spread s0, Spread s1, Spread s2,

@@ -141,9 +141,9 @@ int c3d_monitor(c3d_ctx *ctx, double *out);
  * V(nxg,ny,nzg), W(nxg,nyg,nz) that the caller owns, into the device array
  * out[7], enqueued on `stream` (a hipStream_t; NULL: the null stream) and
  * not waited for.  No context and no allocation: the kernels' scratch (the
- * 256 x 7 partials and the reduced sums, 14 KB whatever the grid) is a
- * static device array of the library, one per GPU, held until the process
- * ends.  Face counts 3 .. 1000000 each; C3D_EINVAL otherwise or for NULL
+ * up to 1024 x 7 partials and the reduced sums, in 64 KB whatever the grid)
+ * is a static device array of the library, one per GPU, held until the
+ * process ends.  Face counts 3 .. 1000000 each; C3D_EINVAL otherwise or for NULL
  * arrays.  Calls that overlap on one GPU share that scratch and race: serialise
  * them (one stream, or events).  No counterpart in the reference: for callers
  * that cannot allocate device memory (code under HIP graph capture, serving
